@@ -4,7 +4,7 @@
 
 #include <vector>
 
-#include "awk_fft.h"
+#include "awk_dense.h"
 
 namespace awk {
 
@@ -20,6 +20,8 @@ struct AxisPlan {
   int m = 0;
   std::vector<int> mrad;
   const float2 *chirp = nullptr, *bhat = nullptr, *mtw = nullptr;
+  // Dense transform on the matrix cores (0 tiles: not used)
+  DenseAxis dense{nullptr, 0, 0, 0, 0};
   // the line length the LDS stages hold (the work area of m when used)
   int stage_len() const { return m > n ? m : n; }
 };

@@ -175,10 +175,17 @@ __device__ __forceinline__ float load_mul(const XFwdArgs &a, size_t i) {
   return __builtin_nontemporal_load(a.i1 + i);
 }
 
+// Which transform an x pass runs: the LDS stages, or the dense product (awk_dense.h),
+// whose lines are the rows' components as real lines [x][kDenseLS].
+enum XEngine { XENG_STAGES = 0, XENG_DENSE = 1 };
+constexpr int kDenseLS = 33;   // floats per staged x (an odd stride: no bank conflicts along x)
+constexpr int kDenseRows = 10; // rows per dense x block: 30 of the product's 32 lines
+constexpr int kDenseXThreads = 512;  // at most: a wave per tile, and at least 4 waves
+
 // NC, RTC, BDC: compile-time length, rows per block and block size (0 = runtime).
-template <int NC, int RTC, int BDC>
-__global__ void __launch_bounds__(BDC ? BDC : 1024)
-k_xfwd(XFwdArgs a, Axis ax, int nx_rt, int ny, int nz, int nxh_rt, int nxh_pad, int RT_rt,
+template <int NC, int RTC, int BDC, int ENG = XENG_STAGES>
+__global__ void __launch_bounds__(ENG == XENG_DENSE ? kDenseXThreads : BDC ? BDC : 1024)
+k_xfwd(XFwdArgs a, Axis ax, DenseAxis da, int nx_rt, int ny, int nz, int nxh_rt, int nxh_pad, int RT_rt,
        float2 *__restrict__ spec, size_t plane, Batch bt) {
   extern __shared__ float2 sm[];
   __shared__ double red[16];
@@ -199,6 +206,13 @@ k_xfwd(XFwdArgs a, Axis ax, int nx_rt, int ny, int nz, int nxh_rt, int nxh_pad, 
   double ssd = 0.0;
   float *smf = reinterpret_cast<float *>(sm);
   auto put = [&](int q, int x, float f0, float f1, float f2) {
+    if constexpr (ENG == XENG_DENSE) {
+      float *o = smf + x * kDenseLS + 3 * q;
+      o[0] = f0;
+      o[1] = f1;
+      o[2] = f2;
+      return;
+    }
     const int p = q >> 1;
     if ((q & 1) == 0) {
       sm[x * LS + 3 * p] = make_float2(f0, f1);
@@ -313,6 +327,26 @@ k_xfwd(XFwdArgs a, Axis ax, int nx_rt, int ny, int nz, int nxh_rt, int nxh_pad, 
     put(q, x, f0, f1, f2);
   }
   }
+  if constexpr (ENG == XENG_DENSE) {
+    for (int w = threadIdx.x; w < kDenseLS; w += bdim) smf[nx * kDenseLS + w] = 0.f;
+    __syncthreads();
+    const int lane = threadIdx.x & 63, hi = lane >> 5, col = lane & 31;
+    const int tile = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    if (tile < da.tiles) {
+      v16f E, O;
+      dense_tile<true, true>(smf + hi * kDenseLS + col, smf + (nx - hi) * kDenseLS + col, 2 * kDenseLS,
+                             -2 * kDenseLS, da.tab + (size_t)tile * da.ks * 64 + lane, da.ks, E, O);
+      const int k = 32 * tile + col;
+      if (k < nxh) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int line = dense_row(i, lane), q = line / 3, c = line - 3 * q;
+          if (line < 3 * kDenseRows && r0 + q < NR)
+            spec[c * plane + (size_t)(r0 + q) * nxh_pad + k] = make_float2(E[i], -O[i]);
+        }
+      }
+    }
+  } else {
   __syncthreads();
   if constexpr (NC != 0) ct_fft<NC, 3 * RTC / 2, 3 * RTC / 2 + 1, BDC>(sm, ax.tw, false);
   else lds_fft(sm, ax, NL, LS, false, sm + (size_t)nx * LS);
@@ -328,6 +362,7 @@ k_xfwd(XFwdArgs a, Axis ax, int nx_rt, int ny, int nz, int nxh_rt, int nxh_pad, 
     line_targets(line, r0, rowA, cA, rowB, cB);
     if (rowA < NR) spec[cA * plane + (size_t)rowA * nxh_pad + k] = A;
     if (rowB < NR) spec[cB * plane + (size_t)rowB * nxh_pad + k] = B;
+  }
   }
   if (a.mode == XLOAD_FORCE && a.partials) {
     // deterministic block reduction of the FP64 SSD partial
@@ -350,9 +385,10 @@ k_xfwd(XFwdArgs a, Axis ax, int nx_rt, int ny, int nz, int nxh_rt, int nxh_pad, 
 // iteration's deformed image.  STG (COMPOSE only; NC, RTC, BDC set, ny % RTC == 0):
 // the composition reads the current field from the block's rows and their
 // neighbours staged in LDS.
-template <int NC, int RTC, int BDC, int XU, bool PAIRS = false, bool APPLY = false, bool STG = false>
-__global__ void __launch_bounds__(BDC ? BDC : 1024)
-k_xinv(XInvArgs a, Axis ax, int nx_rt, int ny, int nz, int nxh_rt, int nxh_pad, int RT_rt,
+template <int NC, int RTC, int BDC, int XU, bool PAIRS = false, bool APPLY = false, bool STG = false,
+          int ENG = XENG_STAGES>
+__global__ void __launch_bounds__(ENG == XENG_DENSE ? kDenseXThreads : BDC ? BDC : 1024)
+k_xinv(XInvArgs a, Axis ax, DenseAxis da, int nx_rt, int ny, int nz, int nxh_rt, int nxh_pad, int RT_rt,
        const float2 *__restrict__ spec, size_t plane, Batch bt) {
   extern __shared__ float2 sm[];
   __shared__ float redf[16];
@@ -379,6 +415,44 @@ k_xinv(XInvArgs a, Axis ax, int nx_rt, int ny, int nz, int nxh_rt, int nxh_pad, 
     if ((a.mode == XSTORE_MAXNORM || a.mode == XSTORE_MAXAXPY) && threadIdx.x == 0) a.maxpart[lb] = 0.f;
     return;
   }
+  float *smf = reinterpret_cast<float *>(sm);
+  if constexpr (ENG == XENG_DENSE) {
+    // x_j = sum_k w_k (cos Re X_k - sin Im X_k), w_0 = 1, else 2 (the table halves
+    // the middle frequency of an even length): the parts of 30 real lines staged as
+    // [k][kDenseLS], real then imaginary, rows nxh .. 2 ks - 1 zero
+    const int KR = 2 * da.ks;
+    float *im = smf + KR * kDenseLS;
+    const int lane = threadIdx.x & 63, hi = lane >> 5, col = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), nw = bdim >> 6;
+    for (int line = wave; line < 3 * kDenseRows; line += nw) {
+      const int q = line / 3, c = line - 3 * q;
+      const float2 *src = spec + c * plane + (size_t)(r0 + q) * nxh_pad;
+      const bool ok = r0 + q < NR;
+      for (int k = lane; k < KR; k += 64) {
+        float2 X = (ok && k < nxh) ? src[k] : make_float2(0.f, 0.f);
+        const float w = k ? 2.f : 1.f;
+        // the imaginary part c2r ignores
+        smf[k * kDenseLS + line] = w * X.x;
+        im[k * kDenseLS + line] = (k == 0 || 2 * k == nx) ? 0.f : w * X.y;
+      }
+    }
+    __syncthreads();
+    v16f P, Q;
+    if (wave < da.tiles)
+      dense_tile<true, false>(smf + hi * kDenseLS + col, im + hi * kDenseLS + col, 2 * kDenseLS,
+                              2 * kDenseLS, da.tab + (size_t)wave * da.ks * 64 + lane, da.ks, P, Q);
+    __syncthreads();  // the staged frequencies are read: the lines take their place
+    const int j = 32 * wave + col;
+    if (wave < da.tiles && j < da.H) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int line = dense_row(i, lane);
+        smf[j * kDenseLS + line] = P[i] - Q[i];
+        if (j > 0 && 2 * j != nx) smf[(nx - j) * kDenseLS + line] = P[i] + Q[i];
+      }
+    }
+    __syncthreads();
+  } else {
 #pragma unroll
   for (int w = threadIdx.x; w < NL * nxh; w += bdim) {
     const int line = w / nxh, k = w - line * nxh;
@@ -396,6 +470,25 @@ k_xinv(XInvArgs a, Axis ax, int nx_rt, int ny, int nz, int nxh_rt, int nxh_pad, 
   __syncthreads();
   if constexpr (NC != 0) ct_fft<NC, 3 * RTC / 2, 3 * RTC / 2 + 1, BDC>(sm, ax.tw, true);
   else lds_fft(sm, ax, NL, LS, true, sm + (size_t)nx * LS);
+  }
+  // the velocity at (q, x) of the block's rows
+  auto vel = [&](int q, int x, float &v0, float &v1, float &v2) {
+    if constexpr (ENG == XENG_DENSE) {
+      const float *o = smf + x * kDenseLS + 3 * q;
+      v0 = o[0];
+      v1 = o[1];
+      v2 = o[2];
+      return;
+    }
+    const int p = q >> 1;
+    if ((q & 1) == 0) {
+      const float2 t = sm[x * LS + 3 * p];
+      v0 = t.x; v1 = t.y; v2 = sm[x * LS + 3 * p + 1].x;
+    } else {
+      const float2 t = sm[x * LS + 3 * p + 2];
+      v0 = t.x; v1 = t.y; v2 = sm[x * LS + 3 * p + 1].y;
+    }
+  };
   float mx = 0.f;
   if (a.mode == XSTORE_COMPOSE) {
     // updateDeformation (GreedyIteratorCPU.cxx:81-95): v *= step; h <- composeHV(h, v, sp, PARTIAL_ID).
@@ -423,15 +516,8 @@ k_xinv(XInvArgs a, Axis ax, int nx_rt, int ny, int nz, int nxh_rt, int nxh_pad, 
       for (int u = 0; u < VP; ++u) {
         const int w = threadIdx.x + u * BDC;
         const int q = w / NC, x = w - q * NC;
-        const int p = q >> 1;
         float v0, v1, v2;
-        if ((q & 1) == 0) {
-          const float2 t = sm[x * LS + 3 * p];
-          v0 = t.x; v1 = t.y; v2 = sm[x * LS + 3 * p + 1].x;
-        } else {
-          const float2 t = sm[x * LS + 3 * p + 2];
-          v0 = t.x; v1 = t.y; v2 = sm[x * LS + 3 * p + 1].y;
-        }
+        vel(q, x, v0, v1, v2);
         px[u] = fmaf(v0 * st, isx, (float)x);
         py[u] = fmaf(v1 * st, isy, (float)(yb + q));
         pz[u] = fmaf(v2 * st, isz, (float)zr);
@@ -499,15 +585,8 @@ k_xinv(XInvArgs a, Axis ax, int nx_rt, int ny, int nz, int nxh_rt, int nxh_pad, 
         row_[u] = (w < RT * nx) ? r0 + q : NR;
         x_[u] = x;
         if (row_[u] < NR) {
-          const int p = q >> 1;
           float v0, v1, v2;
-          if ((q & 1) == 0) {
-            const float2 t = sm[x * LS + 3 * p];
-            v0 = t.x; v1 = t.y; v2 = sm[x * LS + 3 * p + 1].x;
-          } else {
-            const float2 t = sm[x * LS + 3 * p + 2];
-            v0 = t.x; v1 = t.y; v2 = sm[x * LS + 3 * p + 1].y;
-          }
+          vel(q, x, v0, v1, v2);
           const int y = row_[u] % ny, z = row_[u] / ny;
           // explicit fma: the same rounding wherever the position is formed
           px[u] = fmaf(v0 * st, isx, (float)x);
@@ -558,15 +637,8 @@ k_xinv(XInvArgs a, Axis ax, int nx_rt, int ny, int nz, int nxh_rt, int nxh_pad, 
       const int q = w / nx, x = w - q * nx;
       const int row = r0 + q;
       if (row >= NR) continue;
-      const int p = q >> 1;
       float v0, v1, v2;
-      if ((q & 1) == 0) {
-        const float2 t = sm[x * LS + 3 * p];
-        v0 = t.x; v1 = t.y; v2 = sm[x * LS + 3 * p + 1].x;
-      } else {
-        const float2 t = sm[x * LS + 3 * p + 2];
-        v0 = t.x; v1 = t.y; v2 = sm[x * LS + 3 * p + 1].y;
-      }
+      vel(q, x, v0, v1, v2);
       const size_t base = (size_t)row * nx + x;
       if (a.mode == XSTORE_AXPBY) {
         // updateVelocity (LDMMIteratorCPU.cxx:175-190): v = vFac v + uFac u
@@ -692,6 +764,35 @@ k_ypass_reg(const float2 *__restrict__ tw, int nz, int nxh, int nxh_pad, float2 
     energy_block(ra, reinterpret_cast<double *>(sm), TX * (PA > PB ? PA : PB));
   }
 }
+
+// Y pass of a length with a dense plan: a wave per 32 output rows.  Bound by the
+// matrix cores and the spectrum's two passes through memory together.
+__global__ void __launch_bounds__(512)
+k_ypass_dense(DenseAxis ax, int nz, int nxh, int nxh_pad, float2 *__restrict__ spec, size_t plane,
+              int inv, ReduceArgs ra, Batch bt) {
+  extern __shared__ float2 sm[];
+  float *smf = reinterpret_cast<float *>(sm);
+  spec += (long long)blockIdx.y * bt.spec;
+  const int ntile = (nxh + 15) / 16;
+  const int lb = (int)xcd_block();
+  if (lb >= 3 * nz * ntile) return;
+  const int tile = lb % ntile, rest = lb / ntile;
+  const int z = rest % nz, c = rest / nz;
+  const int kx0 = tile * 16, nvalid = min(16, nxh - kx0);
+  float2 *base = spec + c * plane + (size_t)z * ax.n * nxh_pad + kx0;
+  dense_stage(smf, base, (size_t)nxh_pad, ax.n, nvalid);
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  v16f A, B;
+  dense_lines(smf, ax, wave, lane, inv != 0, A, B);
+  dense_store(reinterpret_cast<float *>(base), 2 * (size_t)nxh_pad, ax, wave, lane, nvalid, A, B);
+  if (ra.partials && lb == 0) {
+    __syncthreads();
+    batch_reduce(ra, bt);
+    energy_block(ra, reinterpret_cast<double *>(sm), blockDim.x);
+  }
+}
+
 struct SolveArgs {
   const float *cwx, *swx, *cwy, *swy, *cwz, *swz;
   const float *eig;  // 6 per frequency, or null
@@ -749,6 +850,17 @@ __device__ __forceinline__ void solve_one(const SolveArgs &s, int kx, int ky, in
   b0 = cscale(v0, s.scale);
   b1 = cscale(v1, s.scale);
   b2 = cscale(v2, s.scale);
+}
+
+// solve_one on one part (real or imaginary) of the three components: the operator
+// is real, so the parts do not mix.
+__device__ __forceinline__ void solve_part(const SolveArgs &s, int kx, int ky, int kz, int ny, int nxh,
+                                           float &b0, float &b1, float &b2) {
+  float2 a0 = make_float2(b0, 0.f), a1 = make_float2(b1, 0.f), a2 = make_float2(b2, 0.f);
+  solve_one(s, kx, ky, kz, ny, nxh, a0, a1, a2);
+  b0 = a0.x;
+  b1 = a1.x;
+  b2 = a2.x;
 }
 
 // The three components' z-lines stay in registers through the solve; the
@@ -864,6 +976,59 @@ k_zsolve(Axis az, SolveArgs s, int ny, int nz, int nxh, int nxh_pad, int TX,
   }
 }
 
+// Z pass of a length with a dense plan.  A wave keeps its 32 frequencies and their
+// mirrors of all three components in registers (one real or imaginary part per
+// lane, on which the real operator acts separately); the components go through one
+// LDS buffer in turn, forward and back.
+__global__ void __launch_bounds__(512)
+k_zsolve_dense(DenseAxis az, SolveArgs sa, int ny, int nxh, int nxh_pad, float2 *__restrict__ spec,
+               size_t plane, Batch bt) {
+  extern __shared__ float2 sm[];
+  float *smf = reinterpret_cast<float *>(sm);
+  spec += (long long)blockIdx.y * bt.spec;
+  const int ntile = (nxh + 15) / 16;
+  const int lb = (int)xcd_block();
+  if (lb >= ny * ntile) return;
+  const int tile = lb % ntile, ky = lb / ntile;
+  const int kx0 = tile * 16, nvalid = min(16, nxh - kx0);
+  const size_t zst = (size_t)ny * nxh_pad;
+  float2 *base = spec + (size_t)ky * nxh_pad + kx0;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int col = lane & 31;
+  v16f A[3], B[3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    if (c) __syncthreads();
+    dense_stage(smf, base + c * plane, zst, az.n, nvalid);
+    __syncthreads();
+    dense_lines(smf, az, wave, lane, false, A[c], B[c]);
+  }
+  const int kx = min(kx0 + (col >> 1), nxh - 1);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int k = 32 * wave + dense_row(i, lane);
+    if (k < az.H) {
+      float b0 = A[0][i], b1 = A[1][i], b2 = A[2][i];
+      solve_part(sa, kx, ky, k, ny, nxh, b0, b1, b2);
+      A[0][i] = b0; A[1][i] = b1; A[2][i] = b2;
+      if (k > 0 && 2 * k != az.n) {
+        b0 = B[0][i]; b1 = B[1][i]; b2 = B[2][i];
+        solve_part(sa, kx, ky, az.n - k, ny, nxh, b0, b1, b2);
+        B[0][i] = b0; B[1][i] = b1; B[2][i] = b2;
+      }
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    __syncthreads();
+    dense_store(smf, 32, az, wave, lane, 16, A[c], B[c]);  // row n stays zero
+    __syncthreads();
+    v16f P, Q;
+    dense_lines(smf, az, wave, lane, true, P, Q);
+    dense_store(reinterpret_cast<float *>(base + c * plane), 2 * zst, az, wave, lane, nvalid, P, Q);
+  }
+}
+
 // FP64 table of L^p (symmetric, 6 entries) per frequency for the eigen path
 // (DiffOper::InitializeEigenLookup + PowL, DiffOper.cxx:641-745, 1176-1218).
 // Jacobi rotations on the 3x3 symmetric matrix in double.
@@ -932,12 +1097,16 @@ __global__ void k_eigen_table(float *__restrict__ out, int nx, int ny, int nz, i
 
 // ------------------------------------------------------------------ host
 
-// LDS of the x passes: the row buffer (LS = NL + 1) plus the Bluestein work area.
+// LDS of the x passes: the row buffer (LS = NL + 1) plus the Bluestein work area,
+// or the staged lines (with the zero row) and both parts of the frequencies.
 static size_t x_lds(const AxisPlan &a, int rt) {
+  if (a.dense.tiles) return (size_t)std::max(a.n + 1, 4 * a.dense.ks) * kDenseLS * sizeof(float);
   return ((size_t)a.n * (3 * rt / 2 + 1) + (size_t)a.m * (3 * rt / 2)) * sizeof(float2);
 }
-// LDS of the y / z passes: n lines-per-column * tx lines, plus the work area.
+// LDS of the y / z passes: n lines-per-column * tx lines, plus the work area (dense:
+// 16 columns of n + 1 rows).
 static size_t yz_lds(const AxisPlan &a, int lines) {
+  if (a.dense.tiles) return ((size_t)a.n + 1) * 16 * sizeof(float2);
   return ((size_t)a.n + (size_t)a.m) * lines * sizeof(float2);
 }
 
@@ -945,6 +1114,40 @@ static size_t yz_lds(const AxisPlan &a, int lines) {
 // for the kernels' static reduction arrays (the generic pass kernels are set up
 // for it once; above 64 KiB a block has the CU's LDS to itself)
 constexpr size_t kPassLdsMax = 160 * 1024 - 1024;
+
+// Whether an axis is transformed as a dense product (awk_dense.h): a length with a
+// prime factor above 13, whose LDS stages would be a direct DFT of that prime or a
+// chirp-z transform.  L^-1 at 181 x 217 x 181 4347 -> 576 us, 251 x 241 x 239 7189 ->
+// 1097, 248 x 186 x 155 2611 -> 552, 62^3 184 -> 66, 32 x 31 x 36 63 -> 37, with a
+// smaller error against 64 bits each time.  Lengths of small primes keep their LDS
+// stages: at 200^3 553 us (dense 664), and half as many roundings.
+static bool use_dense(int n, const std::vector<int> &rad) {
+  if (n < kDenseMin || n > kDenseMax) return false;
+  for (int r : rad)
+    if (r > 13 && r != 16) return true;
+  return false;
+}
+
+// The fragment-order table of DenseAxis.  cos and sin of 2 pi m / n once per m.
+static std::vector<float2> dense_table(int n, DenseAxis &d) {
+  d.n = n;
+  d.H = n / 2 + 1;
+  d.tiles = (d.H + 31) / 32;
+  d.ks = ((d.H + 1) / 2 + 3) / 4 * 4;
+  std::vector<float2> cs(n);
+  for (int m = 0; m < n; ++m) {
+    const double a = 2.0 * M_PI * (double)m / (double)n;
+    cs[m] = make_float2((float)cos(a), (2 * m == n || m == 0) ? 0.f : (float)sin(a));
+  }
+  std::vector<float2> t((size_t)d.tiles * d.ks * 64, make_float2(0.f, 0.f));
+  for (int k = 0; k < d.H; ++k)
+    for (int j = 0; j < d.H; ++j) {
+      float2 v = cs[(int)((long long)j * k % n)];
+      if (2 * j == n) v = make_float2(0.5f * v.x, 0.f);
+      t[((size_t)(k / 32) * d.ks + j / 2) * 64 + (j & 1) * 32 + k % 32] = v;
+    }
+  return t;
+}
 
 static int pick_rt(const AxisPlan &a) {
   // the tuned RT if it fits, else the largest even RT <= 8 whose LDS fits 64 KiB
@@ -982,14 +1185,18 @@ awk_status fk_init(FluidKernel &k, int nx, int ny, int nz, const float sp[3]) {
   k.nxh_pad = (k.nxh + 7) / 8 * 8;
   for (int i = 0; i < 3; ++i) k.sp[i] = sp[i];
   const int ns[3] = {nx, ny, nz};
+  std::vector<float2> dense[3];
   for (int i = 0; i < 3; ++i) {
     k.ax[i].n = ns[i];
     k.ax[i].rad = factor(ns[i]);
     k.ax[i].m = 0;
     k.ax[i].mrad.clear();
+    k.ax[i].dense = DenseAxis{nullptr, 0, 0, 0, 0};
     bool big = false;
     for (int r : k.ax[i].rad) big = big || r > 64;
-    if (big) {
+    if (use_dense(ns[i], k.ax[i].rad)) {
+      dense[i] = dense_table(ns[i], k.ax[i].dense);
+    } else if (big) {
       // Bluestein: a power-of-two convolution of length m >= 2n - 1
       int m = 1;
       while (m < 2 * ns[i] - 1) m *= 2;
@@ -1003,13 +1210,14 @@ awk_status fk_init(FluidKernel &k, int nx, int ny, int nz, const float sp[3]) {
     if ((int)k.ax[i].rad.size() > kMaxStages || (int)k.ax[i].mrad.size() > 8)
       return fail(AWK_ERR_INVALID, "fluid kernel: too many FFT stages");
   }
-  k.rt = pick_rt(k.ax[0]);
-  k.tx_y = pick_tx(k.ax[1], 1, 16, tuning().y_tx);
-  k.tx_z = pick_tx(k.ax[2], 3, 8, tuning().z_tx);
+  const DenseAxis *dx[3] = {&k.ax[0].dense, &k.ax[1].dense, &k.ax[2].dense};
+  k.rt = dx[0]->tiles ? kDenseRows : pick_rt(k.ax[0]);
+  k.tx_y = dx[1]->tiles ? 16 : pick_tx(k.ax[1], 1, 16, tuning().y_tx);
+  k.tx_z = dx[2]->tiles ? 16 : pick_tx(k.ax[2], 3, 8, tuning().z_tx);
   if (!k.rt || !k.tx_y || !k.tx_z) return fail(AWK_ERR_UNSUPPORTED, "fluid kernel: axis too long for LDS staging");
-  k.bd_x = pick_bd(k.ax[0].stage_len(), 3 * k.rt / 2);
-  k.bd_y = pick_bd(k.ax[1].stage_len(), k.tx_y);
-  k.bd_z = pick_bd(k.ax[2].stage_len(), 3 * k.tx_z);
+  k.bd_x = dx[0]->tiles ? std::max(256, 64 * dx[0]->tiles) : pick_bd(k.ax[0].stage_len(), 3 * k.rt / 2);
+  k.bd_y = dx[1]->tiles ? 64 * dx[1]->tiles : pick_bd(k.ax[1].stage_len(), k.tx_y);
+  k.bd_z = dx[2]->tiles ? 64 * dx[2]->tiles : pick_bd(k.ax[2].stage_len(), 3 * k.tx_z);
   if (k.bd_x > 1024 || k.bd_y > 1024 || k.bd_z > 1024)
     return fail(AWK_ERR_UNSUPPORTED, "fluid kernel: block too large");
   {
@@ -1020,7 +1228,12 @@ awk_status fk_init(FluidKernel &k, int nx, int ny, int nz, const float sp[3]) {
                            reinterpret_cast<const void *>(&k_xinv<0, 0, 0, 1>),
                            reinterpret_cast<const void *>(&k_xinv<0, 0, 0, 1, false, true>),
                            reinterpret_cast<const void *>(&k_ypass),
-                           reinterpret_cast<const void *>(&k_zsolve)};
+                           reinterpret_cast<const void *>(&k_zsolve),
+                           reinterpret_cast<const void *>(&k_xfwd<0, 0, 0, XENG_DENSE>),
+                           reinterpret_cast<const void *>(&k_xinv<0, 0, 0, 1, false, false, false, XENG_DENSE>),
+                           reinterpret_cast<const void *>(&k_xinv<0, 0, 0, 1, false, true, false, XENG_DENSE>),
+                           reinterpret_cast<const void *>(&k_ypass_dense),
+                           reinterpret_cast<const void *>(&k_zsolve_dense)};
       for (const void *f : fns)
         AWK_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kPassLdsMax));
       lds_attr = true;
@@ -1040,6 +1253,11 @@ awk_status fk_init(FluidKernel &k, int nx, int ny, int nz, const float sp[3]) {
   size_t boff[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
   for (int i = 0; i < 3; ++i)
     if (k.ax[i].m) bluestein_tables(ns[i], k.ax[i].m, tw, boff[i]);
+  size_t doff[3] = {0, 0, 0};
+  for (int i = 0; i < 3; ++i) {
+    doff[i] = tw.size();
+    tw.insert(tw.end(), dense[i].begin(), dense[i].end());
+  }
   const size_t ntw = tw.size();
   const size_t nlut = 2 * (size_t)k.nxh + 2 * (size_t)ny + 2 * (size_t)nz;
   std::vector<float> lut(nlut);
@@ -1070,6 +1288,8 @@ awk_status fk_init(FluidKernel &k, int nx, int ny, int nz, const float sp[3]) {
       k.ax[i].bhat = twd + boff[i][1];
       k.ax[i].mtw = twd + boff[i][2];
     }
+  for (int i = 0; i < 3; ++i)
+    if (k.ax[i].dense.tiles) k.ax[i].dense.tab = twd + doff[i];
   AWK_HIP(hipMalloc(&k.lut, nlut * sizeof(float)));
   AWK_HIP(hipMemcpy(k.lut, lut.data(), nlut * sizeof(float), hipMemcpyHostToDevice));
   k.scratch_bytes = spec_bytes + ntw * sizeof(float2) + nlut * sizeof(float);
@@ -1122,11 +1342,14 @@ awk_status fk_xfwd(FluidKernel &k, const XFwdArgs &a_in, hipStream_t s, int *nbl
   const size_t lds = x_lds(k.ax[0], k.rt);
   const Axis ax = k.ax[0].dev();
 #define AWK_XF(NC, RTC, BDC)                                                                     \
-  AWK_LAUNCH((k_xfwd<NC, RTC, BDC>), dim3(grid, bt.n), dim3(BDC ? BDC : k.bd_x), lds, s, a, ax, \
+  AWK_LAUNCH((k_xfwd<NC, RTC, BDC>), dim3(grid, bt.n), dim3(BDC ? BDC : k.bd_x), lds, s, a, ax, k.ax[0].dense, \
                      k.nx, k.ny, k.nz, k.nxh, k.nxh_pad, k.rt, k.spec, k.spec_plane(), bt)
   // block size = row length selects column mode (128^3 LDMM: 17.2 -> 16.3 us
   // against the generic 256-thread form; the spectrum is the same bit for bit)
-  if (k.nx == 256 && k.rt == 8) AWK_XF(256, 8, 256);
+  if (k.ax[0].dense.tiles)
+    AWK_LAUNCH((k_xfwd<0, 0, 0, XENG_DENSE>), dim3(grid, bt.n), dim3(k.bd_x), lds, s, a, ax, k.ax[0].dense,
+               k.nx, k.ny, k.nz, k.nxh, k.nxh_pad, k.rt, k.spec, k.spec_plane(), bt);
+  else if (k.nx == 256 && k.rt == 8) AWK_XF(256, 8, 256);
   else if (k.nx == 128 && k.rt == 8) AWK_XF(128, 8, 128);
   else if (k.nx == 64 && k.rt == 8) AWK_XF(64, 8, 256);
   else AWK_XF(0, 0, 0);
@@ -1148,7 +1371,11 @@ awk_status fk_ypass(FluidKernel &k, bool inv, hipStream_t s, const ReduceArgs *r
   AWK_LAUNCH((k_ypass_reg<N, RA, RB, 16>), dim3(g16, bt.n), dim3(16 * (N / RA > N / RB ? N / RA : N / RB)), \
                      0, s, tw, k.nz, k.nxh, k.nxh_pad, k.spec, k.spec_plane(),                    \
                      inv ? 1 : tuning().yfwd_rev ? 0 : 2, ra, bt)
-  if (k.ny == 256) AWK_YR(256, 16, 16);
+  if (k.ax[1].dense.tiles)
+    AWK_LAUNCH(k_ypass_dense, dim3(g16, bt.n), dim3(k.bd_y),
+               std::max(yz_lds(k.ax[1], 16), (size_t)k.bd_y * sizeof(double)), s, k.ax[1].dense, k.nz, k.nxh,
+               k.nxh_pad, k.spec, k.spec_plane(), inv ? 1 : 0, ra, bt);
+  else if (k.ny == 256) AWK_YR(256, 16, 16);
   else if (k.ny == 128) AWK_YR(128, 16, 8);
   else if (k.ny == 64) AWK_YR(64, 8, 8);
   else if (k.ny == 32) AWK_YR(32, 8, 4);
@@ -1191,7 +1418,10 @@ awk_status fk_zsolve(FluidKernel &k, bool inverse_op, hipStream_t s, const Batch
 #define AWK_ZR(N, RA, RB)                                                                     \
   AWK_LAUNCH((k_zsolve_reg<N, RA, RB, 16>), dim3(g16, bt.n), dim3(16 * (N / RA > N / RB ? N / RA : N / RB)), \
                      0, s, tw, sa, k.ny, k.nxh, k.nxh_pad, k.spec, k.spec_plane(), bt)
-  if (k.nz == 256) AWK_ZR(256, 16, 16);
+  if (k.ax[2].dense.tiles)
+    AWK_LAUNCH(k_zsolve_dense, dim3(g16, bt.n), dim3(k.bd_z), yz_lds(k.ax[2], 16), s, k.ax[2].dense, sa, k.ny,
+               k.nxh, k.nxh_pad, k.spec, k.spec_plane(), bt);
+  else if (k.nz == 256) AWK_ZR(256, 16, 16);
   else if (k.nz == 128) AWK_ZR(128, 16, 8);
   else if (k.nz == 64) AWK_ZR(64, 8, 8);
   else if (k.nz == 32) AWK_ZR(32, 8, 4);
@@ -1225,12 +1455,12 @@ awk_status fk_xinv(FluidKernel &k, const XInvArgs &a_in, hipStream_t s, int *nbl
   const Axis ax = k.ax[0].dev();
 #define AWK_XI3(NC, RTC, BDC, XU, PR, AP)                                                        \
   AWK_LAUNCH((k_xinv<NC, RTC, BDC, XU, PR, AP>), dim3(grid, bt.n), dim3(BDC ? BDC : k.bd_x), lds, s, a, \
-                     ax, k.nx, k.ny, k.nz, k.nxh, k.nxh_pad, k.rt, k.spec, k.spec_plane(), bt)
+                     ax, k.ax[0].dense, k.nx, k.ny, k.nz, k.nxh, k.nxh_pad, k.rt, k.spec, k.spec_plane(), bt)
 #define AWK_XIS(NC, BD, AP)                                                                      \
-  AWK_LAUNCH((k_xinv<NC, 8, BD, 1, false, AP, true>), dim3(grid, bt.n), dim3(BD), lds, s, a, ax, \
+  AWK_LAUNCH((k_xinv<NC, 8, BD, 1, false, AP, true>), dim3(grid, bt.n), dim3(BD), lds, s, a, ax, k.ax[0].dense, \
                      k.nx, k.ny, k.nz, k.nxh, k.nxh_pad, k.rt, k.spec, k.spec_plane(), bt)
 #define AWK_XI(NC, RTC, BDC, XU)                                                                 \
-  AWK_LAUNCH((k_xinv<NC, RTC, BDC, XU>), dim3(grid, bt.n), dim3(BDC ? BDC : k.bd_x), lds, s, a, ax, \
+  AWK_LAUNCH((k_xinv<NC, RTC, BDC, XU>), dim3(grid, bt.n), dim3(BDC ? BDC : k.bd_x), lds, s, a, ax, k.ax[0].dense, \
                      k.nx, k.ny, k.nz, k.nxh, k.nxh_pad, k.rt, k.spec, k.spec_plane(), bt)
   const int xu = tuning().xinv_unroll;
   // xinv_pairs: waves whose points all lie inside the volume gather the
@@ -1250,7 +1480,13 @@ awk_status fk_xinv(FluidKernel &k, const XInvArgs &a_in, hipStream_t s, int *nbl
   const int sk = tuning().xinv_stage;
   const bool stg = a.mode == XSTORE_COMPOSE && (sk == 1 || (sk == 2 && k.nx <= 128)) && k.rt == 8 &&
                    k.ny % 8 == 0 && (k.nx == 256 || k.nx == 128 || k.nx == 64);
-  if (stg) {
+#define AWK_XID(AP)                                                                              \
+  AWK_LAUNCH((k_xinv<0, 0, 0, 1, false, AP, false, XENG_DENSE>), dim3(grid, bt.n), dim3(k.bd_x), lds, s, \
+                     a, ax, k.ax[0].dense, k.nx, k.ny, k.nz, k.nxh, k.nxh_pad, k.rt, k.spec, k.spec_plane(), bt)
+  if (k.ax[0].dense.tiles) {
+    if (ap) AWK_XID(true);
+    else AWK_XID(false);
+  } else if (stg) {
     lds = std::max(lds, (size_t)3 * (k.rt + 2) * k.nx * sizeof(float));
     if (k.nx == 256) {
       if (ap) AWK_XIS(256, 256, true);
@@ -1286,6 +1522,7 @@ awk_status fk_xinv(FluidKernel &k, const XInvArgs &a_in, hipStream_t s, int *nbl
 #undef AWK_XI
 #undef AWK_XI3
 #undef AWK_XIS
+#undef AWK_XID
   AWK_LAUNCH_CHECK("k_xinv");
   if (nblocks) *nblocks = (int)grid;
   return AWK_OK;

@@ -109,3 +109,50 @@ def test_tuned_fft_plans_match_oracle(shape, knobs):
     op.ApplyInverseOperator(d)
     ref = oracle.diffoper(aos(f), sp=sp, alpha=0.01, beta=0.01, gamma=0.001, inverse=True)
     assert rel_l2(host(d), soa(ref)) <= TOL
+
+
+# A length with a prime factor above 13 is transformed as a matrix product in tiles of
+# 32 outputs k <= n / 2: the first such length, one short of / exactly / one past one,
+# two, four and eight tiles, and the two sides of the longest (511)
+DENSE_LENGTHS = [17, 19, 61, 62, 67, 127, 134, 251, 254, 257, 262, 502, 509, 511, 514]
+
+
+@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("n", DENSE_LENGTHS)
+def test_dense_axis_matches_oracle(n, axis):
+    """L^-1 with one dense axis.  Bar: the two transforms of that axis, each a sum of
+    n / 2 terms in runs of 16 (n = 511: 16 runs, so at most about 2 sqrt(16) roundings
+    of 2^-24 in the mean square and the folds before and after: 6e-7), four short ones
+    and the solve (5e-7): 1.7e-6."""
+    from atlaswerks_amd.fluid import DiffOperGPU, DiffOperParam
+    from gpu_util import aos, host, rel_l2, soa, to_dev
+    shape = [5, 12, 9]
+    shape[axis] = n
+    nz, ny, nx = shape
+    print("fluid dense", shape, flush=True)
+    f = _field(tuple(shape), seed=n + axis)
+    sp = (1.0, 1.25, 0.8)
+    op = DiffOperGPU((nx, ny, nz), sp, DiffOperParam(alpha=0.01, beta=0.01, gamma=0.001))
+    d = to_dev(f)
+    op.ApplyInverseOperator(d)
+    ref = oracle.diffoper(aos(f), sp=sp, alpha=0.01, beta=0.01, gamma=0.001, inverse=True)
+    assert rel_l2(host(d), soa(ref)) <= 1.7e-6
+
+
+@pytest.mark.parametrize("shape", [(23, 19, 37), (34, 20, 62), (17, 29, 67)])
+def test_dense_axes_greedy_matches_oracle(shape):
+    """The force, energy and composition of the greedy step around dense axes, row
+    groups that end inside a plane among them: energies and field as the greedy parity
+    tests' bars (1e-3, relative L2 1e-5), single and back-to-back iterations alike."""
+    import torch
+    from atlaswerks_amd.greedy import GreedyWarp
+    from gpu_util import host, rel_l2, soa
+    print("greedy dense", shape, flush=True)
+    t, h, _ = synth.pair(shape, seed=2, max_disp=1.5)
+    target = oracle.apply(t, np.moveaxis(h, 0, -1), dtype=np.float32)
+    hd, _, _, ed, _ = oracle.greedy_run(t, target, 6)
+    I0, I1 = torch.from_numpy(t).cuda(), torch.from_numpy(target).cuda()
+    w = GreedyWarp(I0, I1, 6)
+    data = w.RunWarp()
+    assert np.max(np.abs(data.energies() - ed) / ed) < 1e-3
+    assert rel_l2(host(data.Def1To0), soa(hd)) <= 1e-5
