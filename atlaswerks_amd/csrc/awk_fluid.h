@@ -119,6 +119,7 @@ struct FluidKernel {
   int tx_y = 16;       // kx columns per y-pass block
   int tx_z = 8;        // kx columns per z-pass block
   int bd_x = 256, bd_y = 256, bd_z = 256;
+  size_t lds_x = 0, lds_y = 0, lds_z = 0;  // dynamic LDS of the any-length passes
   // device buffers
   float2 *spec = nullptr;  // 3 planes of nz*ny*nxh_pad complex
   float *lut = nullptr;    // cwx[nxh] swx[nxh] cwy[ny] swy[ny] cwz[nz] swz[nz]
@@ -145,6 +146,14 @@ awk_status fk_zsolve(FluidKernel &k, bool inverse_op, hipStream_t s, const Batch
 awk_status fk_xinv(FluidKernel &k, const XInvArgs &a, hipStream_t s, int *nblocks,
                    const Batch *b = nullptr);
 int fk_xblocks(const FluidKernel &k);
+// The passes for lengths without a kernel of their own (awk_fluid_any.hip); the
+// callers check the launch.
+struct SolveArgs;
+awk_status any_setup(int lds_max);
+void any_xfwd(FluidKernel &k, const XFwdArgs &a, unsigned grid, hipStream_t s, const Batch &bt);
+void any_xinv(FluidKernel &k, const XInvArgs &a, bool apply, unsigned grid, hipStream_t s, const Batch &bt);
+void any_ypass(FluidKernel &k, bool inv, const ReduceArgs &ra, hipStream_t s, const Batch &bt);
+void any_zsolve(FluidKernel &k, const SolveArgs &sa, hipStream_t s, const Batch &bt);
 
 }  // namespace awk
 

@@ -1,0 +1,224 @@
+// awk_fluid_any.hip -- the passes of the FluidKernelFFT operator for any axis length:
+// LDS stages of mixed radices (chirp-z for large primes), or the dense product on the
+// matrix cores (awk_dense.h).  The powers of two from 32 to 256 have their own kernels
+// in awk_fluid.hip.
+#include "awk_fluid.h"
+#include "awk_fluid_solve.h"
+#include "awk_fluid_x.h"
+
+namespace awk {
+
+// Y pass: complex FFT along y for TX kx columns of one (component, z) slab.
+__global__ void __launch_bounds__(1024)
+k_ypass(Axis ax, int ny, int nz, int nxh, int nxh_pad, int TX, float2 *__restrict__ spec,
+        size_t plane, int inv, ReduceArgs ra, Batch bt) {
+  extern __shared__ float2 sm[];
+  spec += (long long)blockIdx.y * bt.spec;
+  const int ntile = (nxh + TX - 1) / TX;
+  const int lb = (int)xcd_block();
+  if (lb >= 3 * nz * ntile) return;
+  const int tile = lb % ntile, rest = lb / ntile;
+  const int z = rest % nz, c = rest / nz;
+  const int kx0 = tile * TX;
+  float2 *base = spec + c * plane + (size_t)z * ny * nxh_pad + kx0;
+  for (int w = threadIdx.x; w < TX * ny; w += blockDim.x) {
+    const int t = w % TX, y = w / TX;
+    sm[y * TX + t] = (kx0 + t < nxh) ? base[(size_t)y * nxh_pad + t] : make_float2(0.f, 0.f);
+  }
+  __syncthreads();
+  lds_fft(sm, ax, TX, TX, inv != 0, sm + (size_t)ny * TX);
+  for (int w = threadIdx.x; w < TX * ny; w += blockDim.x) {
+    const int t = w % TX, y = w / TX;
+    if (kx0 + t < nxh) base[(size_t)y * nxh_pad + t] = sm[y * TX + t];
+  }
+  if (ra.partials && lb == 0) {
+    __syncthreads();
+    batch_reduce(ra, bt);
+    energy_block(ra, reinterpret_cast<double *>(sm), blockDim.x);
+  }
+}
+
+// Y pass of a length with a dense plan: a wave per 32 output rows.  Bound by the
+// matrix cores and the spectrum's two passes through memory together.
+__global__ void __launch_bounds__(512)
+k_ypass_dense(DenseAxis ax, int nz, int nxh, int nxh_pad, float2 *__restrict__ spec, size_t plane,
+              int inv, ReduceArgs ra, Batch bt) {
+  extern __shared__ float2 sm[];
+  float *smf = reinterpret_cast<float *>(sm);
+  spec += (long long)blockIdx.y * bt.spec;
+  const int ntile = (nxh + 15) / 16;
+  const int lb = (int)xcd_block();
+  if (lb >= 3 * nz * ntile) return;
+  const int tile = lb % ntile, rest = lb / ntile;
+  const int z = rest % nz, c = rest / nz;
+  const int kx0 = tile * 16, nvalid = min(16, nxh - kx0);
+  float2 *base = spec + c * plane + (size_t)z * ax.n * nxh_pad + kx0;
+  dense_stage(smf, base, (size_t)nxh_pad, ax.n, nvalid);
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  v16f A, B;
+  dense_lines(smf, ax, wave, lane, inv != 0, A, B);
+  dense_store(reinterpret_cast<float *>(base), 2 * (size_t)nxh_pad, ax, wave, lane, nvalid, A, B);
+  if (ra.partials && lb == 0) {
+    __syncthreads();
+    batch_reduce(ra, bt);
+    energy_block(ra, reinterpret_cast<double *>(sm), blockDim.x);
+  }
+}
+
+// Z pass: forward FFT along z of 3 components x TX kx columns at one ky, the
+// per-frequency solve, inverse FFT along z.
+__global__ void __launch_bounds__(1024)
+k_zsolve(Axis az, SolveArgs s, int ny, int nz, int nxh, int nxh_pad, int TX,
+         float2 *__restrict__ spec, size_t plane, Batch bt) {
+  extern __shared__ float2 sm[];
+  spec += (long long)blockIdx.y * bt.spec;
+  const int NL = 3 * TX;
+  const int ntile = (nxh + TX - 1) / TX;
+  const int lb = (int)xcd_block();
+  if (lb >= ny * ntile) return;
+  const int tile = lb % ntile, ky = lb / ntile;
+  const int kx0 = tile * TX;
+  for (int w = threadIdx.x; w < NL * nz; w += blockDim.x) {
+    const int t = w % TX, rest = w / TX;
+    const int c = rest % 3, z = rest / 3;
+    sm[z * NL + c * TX + t] = (kx0 + t < nxh)
+                                  ? spec[c * plane + ((size_t)z * ny + ky) * nxh_pad + kx0 + t]
+                                  : make_float2(0.f, 0.f);
+  }
+  __syncthreads();
+  lds_fft(sm, az, NL, NL, false, sm + (size_t)nz * NL);
+  for (int w = threadIdx.x; w < TX * nz; w += blockDim.x) {
+    const int t = w % TX, kz = w / TX;
+    const int kx = kx0 + t;
+    if (kx >= nxh) continue;
+    float2 b0 = sm[kz * NL + t], b1 = sm[kz * NL + TX + t], b2 = sm[kz * NL + 2 * TX + t];
+    solve_one(s, kx, ky, kz, ny, nxh, b0, b1, b2);
+    sm[kz * NL + t] = b0;
+    sm[kz * NL + TX + t] = b1;
+    sm[kz * NL + 2 * TX + t] = b2;
+  }
+  __syncthreads();
+  lds_fft(sm, az, NL, NL, true, sm + (size_t)nz * NL);
+  for (int w = threadIdx.x; w < NL * nz; w += blockDim.x) {
+    const int t = w % TX, rest = w / TX;
+    const int c = rest % 3, z = rest / 3;
+    if (kx0 + t < nxh) spec[c * plane + ((size_t)z * ny + ky) * nxh_pad + kx0 + t] = sm[z * NL + c * TX + t];
+  }
+}
+
+// Z pass of a length with a dense plan.  A wave keeps its 32 frequencies and their
+// mirrors of all three components in registers (one real or imaginary part per
+// lane, on which the real operator acts separately); the components go through one
+// LDS buffer in turn, forward and back.
+__global__ void __launch_bounds__(512)
+k_zsolve_dense(DenseAxis az, SolveArgs sa, int ny, int nxh, int nxh_pad, float2 *__restrict__ spec,
+               size_t plane, Batch bt) {
+  extern __shared__ float2 sm[];
+  float *smf = reinterpret_cast<float *>(sm);
+  spec += (long long)blockIdx.y * bt.spec;
+  const int ntile = (nxh + 15) / 16;
+  const int lb = (int)xcd_block();
+  if (lb >= ny * ntile) return;
+  const int tile = lb % ntile, ky = lb / ntile;
+  const int kx0 = tile * 16, nvalid = min(16, nxh - kx0);
+  const size_t zst = (size_t)ny * nxh_pad;
+  float2 *base = spec + (size_t)ky * nxh_pad + kx0;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int col = lane & 31;
+  v16f A[3], B[3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    if (c) __syncthreads();
+    dense_stage(smf, base + c * plane, zst, az.n, nvalid);
+    __syncthreads();
+    dense_lines(smf, az, wave, lane, false, A[c], B[c]);
+  }
+  const int kx = min(kx0 + (col >> 1), nxh - 1);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int k = 32 * wave + dense_row(i, lane);
+    if (k < az.H) {
+      float b0 = A[0][i], b1 = A[1][i], b2 = A[2][i];
+      solve_part(sa, kx, ky, k, ny, nxh, b0, b1, b2);
+      A[0][i] = b0; A[1][i] = b1; A[2][i] = b2;
+      if (k > 0 && 2 * k != az.n) {
+        b0 = B[0][i]; b1 = B[1][i]; b2 = B[2][i];
+        solve_part(sa, kx, ky, az.n - k, ny, nxh, b0, b1, b2);
+        B[0][i] = b0; B[1][i] = b1; B[2][i] = b2;
+      }
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    __syncthreads();
+    dense_store(smf, 32, az, wave, lane, 16, A[c], B[c]);  // row n stays zero
+    __syncthreads();
+    v16f P, Q;
+    dense_lines(smf, az, wave, lane, true, P, Q);
+    dense_store(reinterpret_cast<float *>(base + c * plane), 2 * zst, az, wave, lane, nvalid, P, Q);
+  }
+}
+
+// ------------------------------------------------------------------ host
+
+awk_status any_setup(int lds_max) {
+  // these kernels may take more than the default 64 KiB of dynamic LDS
+  static bool done = false;
+  if (done) return AWK_OK;
+  const void *fns[] = {reinterpret_cast<const void *>(&k_xfwd<0, 0, 0>),
+                       reinterpret_cast<const void *>(&k_xinv<0, 0, 0, 1>),
+                       reinterpret_cast<const void *>(&k_xinv<0, 0, 0, 1, false, true>),
+                       reinterpret_cast<const void *>(&k_ypass),
+                       reinterpret_cast<const void *>(&k_zsolve),
+                       reinterpret_cast<const void *>(&k_xfwd<0, 0, 0, XENG_DENSE>),
+                       reinterpret_cast<const void *>(&k_xinv<0, 0, 0, 1, false, false, false, XENG_DENSE>),
+                       reinterpret_cast<const void *>(&k_xinv<0, 0, 0, 1, false, true, false, XENG_DENSE>),
+                       reinterpret_cast<const void *>(&k_ypass_dense),
+                       reinterpret_cast<const void *>(&k_zsolve_dense)};
+  for (const void *f : fns) AWK_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds_max));
+  done = true;
+  return AWK_OK;
+}
+
+#define AWK_ANY_X(K, A)                                                                          \
+  AWK_LAUNCH(K, dim3(grid, bt.n), dim3(k.bd_x), k.lds_x, s, A, k.ax[0].dev(), k.ax[0].dense, k.nx, k.ny, \
+             k.nz, k.nxh, k.nxh_pad, k.rt, k.spec, k.spec_plane(), bt)
+
+void any_xfwd(FluidKernel &k, const XFwdArgs &a, unsigned grid, hipStream_t s, const Batch &bt) {
+  if (k.ax[0].dense.tiles) AWK_ANY_X((k_xfwd<0, 0, 0, XENG_DENSE>), a);
+  else AWK_ANY_X((k_xfwd<0, 0, 0>), a);
+}
+
+void any_xinv(FluidKernel &k, const XInvArgs &a, bool apply, unsigned grid, hipStream_t s, const Batch &bt) {
+  if (k.ax[0].dense.tiles) {
+    if (apply) AWK_ANY_X((k_xinv<0, 0, 0, 1, false, true, false, XENG_DENSE>), a);
+    else AWK_ANY_X((k_xinv<0, 0, 0, 1, false, false, false, XENG_DENSE>), a);
+  } else if (apply) AWK_ANY_X((k_xinv<0, 0, 0, 1, false, true>), a);
+  else AWK_ANY_X((k_xinv<0, 0, 0, 1>), a);
+}
+#undef AWK_ANY_X
+
+void any_ypass(FluidKernel &k, bool inv, const ReduceArgs &ra, hipStream_t s, const Batch &bt) {
+  const int ntile = (k.nxh + k.tx_y - 1) / k.tx_y;
+  const unsigned grid = grid_for((long long)3 * k.nz * ntile, 1);
+  if (k.ax[1].dense.tiles)
+    AWK_LAUNCH(k_ypass_dense, dim3(grid, bt.n), dim3(k.bd_y), k.lds_y, s, k.ax[1].dense, k.nz, k.nxh,
+               k.nxh_pad, k.spec, k.spec_plane(), inv ? 1 : 0, ra, bt);
+  else
+    AWK_LAUNCH(k_ypass, dim3(grid, bt.n), dim3(k.bd_y), k.lds_y, s, k.ax[1].dev(), k.ny, k.nz, k.nxh,
+               k.nxh_pad, k.tx_y, k.spec, k.spec_plane(), inv ? 1 : 0, ra, bt);
+}
+
+void any_zsolve(FluidKernel &k, const SolveArgs &sa, hipStream_t s, const Batch &bt) {
+  const int ntile = (k.nxh + k.tx_z - 1) / k.tx_z;
+  const unsigned grid = grid_for((long long)k.ny * ntile, 1);
+  if (k.ax[2].dense.tiles)
+    AWK_LAUNCH(k_zsolve_dense, dim3(grid, bt.n), dim3(k.bd_z), k.lds_z, s, k.ax[2].dense, sa, k.ny, k.nxh,
+               k.nxh_pad, k.spec, k.spec_plane(), bt);
+  else
+    AWK_LAUNCH(k_zsolve, dim3(grid, bt.n), dim3(k.bd_z), k.lds_z, s, k.ax[2].dev(), sa, k.ny, k.nz, k.nxh,
+               k.nxh_pad, k.tx_z, k.spec, k.spec_plane(), bt);
+}
+
+}  // namespace awk
