@@ -5,6 +5,7 @@
 #include <vector>
 
 #include "awk_dense.h"
+#include "awk_radix.h"
 
 namespace awk {
 
@@ -22,8 +23,18 @@ struct AxisPlan {
   const float2 *chirp = nullptr, *bhat = nullptr, *mtw = nullptr;
   // Dense transform on the matrix cores (0 tiles: not used)
   DenseAxis dense{nullptr, 0, 0, 0, 0};
+  // Two radices in registers (ra 0: not used)
+  RadixAxis radix{nullptr, 0, 0, 0};
   // the line length the LDS stages hold (the work area of m when used)
   int stage_len() const { return m > n ? m : n; }
+};
+
+// What the any-length x passes take besides the axis: its dense or radix plan, and the
+// multipliers of div_small for nx and nxh.
+struct XPlan {
+  DenseAxis dense;
+  RadixAxis radix;
+  unsigned mn, mh;
 };
 
 // Epilogue of the inverse x pass.
@@ -114,6 +125,10 @@ struct FluidKernel {
   float alpha = 0, beta = 0, gamma = 0, lpow = 1;
   int flags = 0;
   AxisPlan ax[3];
+  XPlan xplan() const {
+    auto m = [](int n) { return n > 1 ? (unsigned)(((1ull << 32) + n - 1) / n) : 0u; };
+    return XPlan{ax[0].dense, ax[0].radix, m(nx), m(nxh)};
+  }
   // launch shapes
   int rt = 8;          // spatial rows per x-pass block (even)
   int tx_y = 16;       // kx columns per y-pass block

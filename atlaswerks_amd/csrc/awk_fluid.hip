@@ -341,6 +341,16 @@ static bool use_dense(int n, const std::vector<int> &rad) {
   return false;
 }
 
+// Whether an axis is transformed by two radices in registers (awk_radix.h): every
+// length that has such a plan, up to 1024 (along z up to the 424 whose three
+// components fit a block's LDS).  L^-1 against the LDS stages: 160 x 192 x 144 312 ->
+// 171 us, 96^3 125 -> 62, 36^3 43 -> 27, 112^3 279 -> 78, 182^3 2199 -> 222, 240^3 931 ->
+// 527, 200^3 553 -> 382, 300 x 128 x 128 317 -> 173.
+static bool use_radix(int axis, int n) {
+  int ra, rb;
+  return n > 1 && radix_plan(n, ra, rb) && (axis < 2 || (size_t)n * 3 * 16 * sizeof(float2) <= kPassLdsMax);
+}
+
 // The fragment-order table of DenseAxis.  cos and sin of 2 pi m / n once per m.
 static std::vector<float2> dense_table(int n, DenseAxis &d) {
   d.n = n;
@@ -405,6 +415,8 @@ awk_status fk_init(FluidKernel &k, int nx, int ny, int nz, const float sp[3]) {
     k.ax[i].m = 0;
     k.ax[i].mrad.clear();
     k.ax[i].dense = DenseAxis{nullptr, 0, 0, 0, 0};
+    k.ax[i].radix = RadixAxis{nullptr, ns[i], 0, 0};
+    if (use_radix(i, ns[i])) radix_plan(ns[i], k.ax[i].radix.ra, k.ax[i].radix.rb);
     bool big = false;
     for (int r : k.ax[i].rad) big = big || r > 64;
     if (use_dense(ns[i], k.ax[i].rad)) {
@@ -424,13 +436,14 @@ awk_status fk_init(FluidKernel &k, int nx, int ny, int nz, const float sp[3]) {
       return fail(AWK_ERR_INVALID, "fluid kernel: too many FFT stages");
   }
   const DenseAxis *dx[3] = {&k.ax[0].dense, &k.ax[1].dense, &k.ax[2].dense};
-  k.rt = dx[0]->tiles ? kDenseRows : pick_rt(k.ax[0]);
-  k.tx_y = dx[1]->tiles ? 16 : pick_tx(k.ax[1], 1, 16, tuning().y_tx);
-  k.tx_z = dx[2]->tiles ? 16 : pick_tx(k.ax[2], 3, 8, tuning().z_tx);
+  const RadixAxis *rx[3] = {&k.ax[0].radix, &k.ax[1].radix, &k.ax[2].radix};
+  k.rt = rx[0]->ra ? 8 : dx[0]->tiles ? kDenseRows : pick_rt(k.ax[0]);
+  k.tx_y = dx[1]->tiles || rx[1]->ra ? 16 : pick_tx(k.ax[1], 1, 16, tuning().y_tx);
+  k.tx_z = dx[2]->tiles || rx[2]->ra ? 16 : pick_tx(k.ax[2], 3, 8, tuning().z_tx);
   if (!k.rt || !k.tx_y || !k.tx_z) return fail(AWK_ERR_UNSUPPORTED, "fluid kernel: axis too long for LDS staging");
-  k.bd_x = dx[0]->tiles ? std::max(256, 64 * dx[0]->tiles) : pick_bd(k.ax[0].stage_len(), 3 * k.rt / 2);
-  k.bd_y = dx[1]->tiles ? 64 * dx[1]->tiles : pick_bd(k.ax[1].stage_len(), k.tx_y);
-  k.bd_z = dx[2]->tiles ? 64 * dx[2]->tiles : pick_bd(k.ax[2].stage_len(), 3 * k.tx_z);
+  k.bd_x = rx[0]->ra ? std::max(256, (12 * rx[0]->ra + 63) / 64 * 64) : dx[0]->tiles ? std::max(256, 64 * dx[0]->tiles) : pick_bd(k.ax[0].stage_len(), 3 * k.rt / 2);
+  k.bd_y = rx[1]->ra ? 16 * rx[1]->ra : dx[1]->tiles ? 64 * dx[1]->tiles : pick_bd(k.ax[1].stage_len(), k.tx_y);
+  k.bd_z = rx[2]->ra ? 16 * rx[2]->ra : dx[2]->tiles ? 64 * dx[2]->tiles : pick_bd(k.ax[2].stage_len(), 3 * k.tx_z);
   if (k.bd_x > 1024 || k.bd_y > 1024 || k.bd_z > 1024)
     return fail(AWK_ERR_UNSUPPORTED, "fluid kernel: block too large");
   k.lds_x = x_lds(k.ax[0], k.rt);
@@ -480,6 +493,7 @@ awk_status fk_init(FluidKernel &k, int nx, int ny, int nz, const float sp[3]) {
   k.ax[0].tw = twd;
   k.ax[1].tw = twd + nx;
   k.ax[2].tw = twd + nx + ny;
+  for (int i = 0; i < 3; ++i) k.ax[i].radix.tw = k.ax[i].tw;
   for (int i = 0; i < 3; ++i)
     if (k.ax[i].m) {
       k.ax[i].chirp = twd + boff[i][0];
@@ -540,7 +554,7 @@ awk_status fk_xfwd(FluidKernel &k, const XFwdArgs &a_in, hipStream_t s, int *nbl
   const size_t lds = k.lds_x;
   const Axis ax = k.ax[0].dev();
 #define AWK_XF(NC, RTC, BDC)                                                                     \
-  AWK_LAUNCH((k_xfwd<NC, RTC, BDC>), dim3(grid, bt.n), dim3(BDC ? BDC : k.bd_x), lds, s, a, ax, k.ax[0].dense, \
+  AWK_LAUNCH((k_xfwd<NC, RTC, BDC>), dim3(grid, bt.n), dim3(BDC ? BDC : k.bd_x), lds, s, a, ax, k.xplan(), \
                      k.nx, k.ny, k.nz, k.nxh, k.nxh_pad, k.rt, k.spec, k.spec_plane(), bt)
   // block size = row length selects column mode (128^3 LDMM: 17.2 -> 16.3 us
   // against the generic 256-thread form; the spectrum is the same bit for bit)
@@ -631,12 +645,12 @@ awk_status fk_xinv(FluidKernel &k, const XInvArgs &a_in, hipStream_t s, int *nbl
   const Axis ax = k.ax[0].dev();
 #define AWK_XI3(NC, RTC, BDC, XU, PR, AP)                                                        \
   AWK_LAUNCH((k_xinv<NC, RTC, BDC, XU, PR, AP>), dim3(grid, bt.n), dim3(BDC ? BDC : k.bd_x), lds, s, a, \
-                     ax, k.ax[0].dense, k.nx, k.ny, k.nz, k.nxh, k.nxh_pad, k.rt, k.spec, k.spec_plane(), bt)
+                     ax, k.xplan(), k.nx, k.ny, k.nz, k.nxh, k.nxh_pad, k.rt, k.spec, k.spec_plane(), bt)
 #define AWK_XIS(NC, BD, AP)                                                                      \
-  AWK_LAUNCH((k_xinv<NC, 8, BD, 1, false, AP, true>), dim3(grid, bt.n), dim3(BD), lds, s, a, ax, k.ax[0].dense, \
+  AWK_LAUNCH((k_xinv<NC, 8, BD, 1, false, AP, true>), dim3(grid, bt.n), dim3(BD), lds, s, a, ax, k.xplan(), \
                      k.nx, k.ny, k.nz, k.nxh, k.nxh_pad, k.rt, k.spec, k.spec_plane(), bt)
 #define AWK_XI(NC, RTC, BDC, XU)                                                                 \
-  AWK_LAUNCH((k_xinv<NC, RTC, BDC, XU>), dim3(grid, bt.n), dim3(BDC ? BDC : k.bd_x), lds, s, a, ax, k.ax[0].dense, \
+  AWK_LAUNCH((k_xinv<NC, RTC, BDC, XU>), dim3(grid, bt.n), dim3(BDC ? BDC : k.bd_x), lds, s, a, ax, k.xplan(), \
                      k.nx, k.ny, k.nz, k.nxh, k.nxh_pad, k.rt, k.spec, k.spec_plane(), bt)
   const int xu = tuning().xinv_unroll;
   // xinv_pairs: waves whose points all lie inside the volume gather the

@@ -3,6 +3,7 @@
 // matrix cores (awk_dense.h).  The powers of two from 32 to 256 have their own kernels
 // in awk_fluid.hip.
 #include "awk_fluid.h"
+#include "awk_radix.h"
 #include "awk_fluid_solve.h"
 #include "awk_fluid_x.h"
 
@@ -160,6 +161,150 @@ k_zsolve_dense(DenseAxis az, SolveArgs sa, int ny, int nxh, int nxh_pad, float2 
   }
 }
 
+// ------------------------------------------------------------------
+// Lengths n = ra * rb (awk_radix.h).  Thread (t, j): kx column t of 16 (128-byte rows),
+// butterfly j < max(ra, rb).  MAXR: the largest radix compiled in (16, or 32 for
+// lengths past 16 * 16 and the like, which costs registers).
+
+template <int MAXR>
+__global__ void __launch_bounds__(16 * MAXR)
+k_ypass_radix(RadixAxis ax, int nz, int nxh, int nxh_pad, float2 *__restrict__ spec, size_t plane,
+              int inv, ReduceArgs ra, Batch bt) {
+  extern __shared__ float2 sm[];
+  spec += (long long)blockIdx.y * bt.spec;
+  const int t = threadIdx.x & 15, j = threadIdx.x >> 4;
+  const int ntile = (nxh + 15) / 16;
+  const int lb = (int)xcd_block();
+  if (lb >= 3 * nz * ntile) return;
+  const int tile = lb % ntile, rest = lb / ntile;
+  const int z = rest % nz, c = rest / nz;
+  const int kx = tile * 16 + t;
+  const bool valid = kx < nxh, iv = inv != 0;
+  float2 *base = spec + c * plane + (size_t)z * ax.n * nxh_pad + kx;
+  const int RA = ax.ra, RB = ax.rb;
+  with_radix<MAXR>(RA, [&](auto rad) {
+    constexpr int R = decltype(rad)::value;
+    if (j < RB) {
+      float2 v[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[r] = valid ? base[(size_t)(j + r * RB) * nxh_pad] : make_float2(0.f, 0.f);
+      dft_any<R>(v, iv);
+#pragma unroll
+      for (int r = 0; r < R; ++r) sm[(j * R + r) * 16 + t] = v[r];
+    }
+  });
+  __syncthreads();
+  with_radix<MAXR>(RB, [&](auto rad) {
+    constexpr int R = decltype(rad)::value;
+    if (j < RA) {
+      float2 v[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[r] = sm[(j + r * RA) * 16 + t];
+      radix_twiddle<R>(v, ax.tw, j, iv);
+      dft_any<R>(v, iv);
+      if (valid) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) base[(size_t)(j + r * RA) * nxh_pad] = v[r];
+      }
+    }
+  });
+  if (ra.partials && lb == 0) {
+    __syncthreads();
+    batch_reduce(ra, bt);
+    energy_block(ra, reinterpret_cast<double *>(sm), blockDim.x);
+  }
+}
+
+// The three components' lines stay in LDS.  A thread's stage-B slots, its frequencies
+// and the first inverse stage's slots (the forward stages transposed) are the same
+// ones, so between stage A and its transpose nothing is exchanged: two barriers.
+template <int MAXR>
+__global__ void __launch_bounds__(16 * MAXR)
+k_zsolve_radix(RadixAxis az, SolveArgs sa, int ny, int nxh, int nxh_pad, float2 *__restrict__ spec,
+               size_t plane, Batch bt) {
+  extern __shared__ float2 sm[];
+  spec += (long long)blockIdx.y * bt.spec;
+  const int t = threadIdx.x & 15, j = threadIdx.x >> 4;
+  const int ntile = (nxh + 15) / 16;
+  const int lb = (int)xcd_block();
+  if (lb >= ny * ntile) return;
+  const int tile = lb % ntile, ky = lb / ntile;
+  const int kx = tile * 16 + t;
+  const bool valid = kx < nxh;
+  const size_t zst = (size_t)ny * nxh_pad;
+  float2 *base = spec + (size_t)ky * nxh_pad + kx;
+  const int RA = az.ra, RB = az.rb, cs = az.n * 16;  // LDS elements per component
+  with_radix<MAXR>(RA, [&](auto rad) {
+    constexpr int R = decltype(rad)::value;
+    if (j < RB) {
+#pragma unroll 1
+      for (int c = 0; c < 3; ++c) {
+        float2 v[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          v[r] = valid ? base[c * plane + (size_t)(j + r * RB) * zst] : make_float2(0.f, 0.f);
+        dft_any<R>(v, false);
+#pragma unroll
+        for (int r = 0; r < R; ++r) sm[c * cs + (j * R + r) * 16 + t] = v[r];
+      }
+    }
+  });
+  __syncthreads();
+  with_radix<MAXR>(RB, [&](auto rad) {
+    constexpr int R = decltype(rad)::value;
+    if (j < RA) {
+#pragma unroll 1
+      for (int c = 0; c < 3; ++c) {
+        float2 v[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[r] = sm[c * cs + (j + r * RA) * 16 + t];
+        radix_twiddle<R>(v, az.tw, j, false);
+        dft_any<R>(v, false);
+#pragma unroll
+        for (int r = 0; r < R; ++r) sm[c * cs + (j + r * RA) * 16 + t] = v[r];
+      }
+      if (valid) {
+#pragma unroll 2
+        for (int r = 0; r < R; ++r) {
+          float2 *p = sm + (j + r * RA) * 16 + t;
+          float2 b0 = p[0], b1 = p[cs], b2 = p[2 * cs];
+          solve_one(sa, kx, ky, j + r * RA, ny, nxh, b0, b1, b2);
+          p[0] = b0;
+          p[cs] = b1;
+          p[2 * cs] = b2;
+        }
+      }
+#pragma unroll 1
+      for (int c = 0; c < 3; ++c) {
+        float2 v[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[r] = sm[c * cs + (j + r * RA) * 16 + t];
+        dft_any<R>(v, true);
+        radix_twiddle<R>(v, az.tw, j, true);
+#pragma unroll
+        for (int r = 0; r < R; ++r) sm[c * cs + (j + r * RA) * 16 + t] = v[r];
+      }
+    }
+  });
+  __syncthreads();
+  with_radix<MAXR>(RA, [&](auto rad) {
+    constexpr int R = decltype(rad)::value;
+    if (j < RB) {
+#pragma unroll 1
+      for (int c = 0; c < 3; ++c) {
+        float2 v[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[r] = sm[c * cs + (j * R + r) * 16 + t];
+        dft_any<R>(v, true);
+        if (valid) {
+#pragma unroll
+          for (int r = 0; r < R; ++r) base[c * plane + (size_t)(j + r * RB) * zst] = v[r];
+        }
+      }
+    }
+  });
+}
+
 // ------------------------------------------------------------------ host
 
 awk_status any_setup(int lds_max) {
@@ -175,23 +320,37 @@ awk_status any_setup(int lds_max) {
                        reinterpret_cast<const void *>(&k_xinv<0, 0, 0, 1, false, false, false, XENG_DENSE>),
                        reinterpret_cast<const void *>(&k_xinv<0, 0, 0, 1, false, true, false, XENG_DENSE>),
                        reinterpret_cast<const void *>(&k_ypass_dense),
-                       reinterpret_cast<const void *>(&k_zsolve_dense)};
+                       reinterpret_cast<const void *>(&k_zsolve_dense),
+                       reinterpret_cast<const void *>(&k_xfwd<0, 8, 0, XENG_RADIX32>),
+                       reinterpret_cast<const void *>(&k_xinv<0, 8, 0, 1, false, false, false, XENG_RADIX32>),
+                       reinterpret_cast<const void *>(&k_xinv<0, 8, 0, 1, false, true, false, XENG_RADIX32>),
+                       reinterpret_cast<const void *>(&k_zsolve_radix<16>),
+                       reinterpret_cast<const void *>(&k_zsolve_radix<32>),
+                       reinterpret_cast<const void *>(&k_ypass_radix<32>)};
   for (const void *f : fns) AWK_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds_max));
   done = true;
   return AWK_OK;
 }
 
 #define AWK_ANY_X(K, A)                                                                          \
-  AWK_LAUNCH(K, dim3(grid, bt.n), dim3(k.bd_x), k.lds_x, s, A, k.ax[0].dev(), k.ax[0].dense, k.nx, k.ny, \
+  AWK_LAUNCH(K, dim3(grid, bt.n), dim3(k.bd_x), k.lds_x, s, A, k.ax[0].dev(), k.xplan(), k.nx, k.ny, \
              k.nz, k.nxh, k.nxh_pad, k.rt, k.spec, k.spec_plane(), bt)
 
 void any_xfwd(FluidKernel &k, const XFwdArgs &a, unsigned grid, hipStream_t s, const Batch &bt) {
-  if (k.ax[0].dense.tiles) AWK_ANY_X((k_xfwd<0, 0, 0, XENG_DENSE>), a);
+  if (k.ax[0].radix.ra > 16) AWK_ANY_X((k_xfwd<0, 8, 0, XENG_RADIX32>), a);
+  else if (k.ax[0].radix.ra) AWK_ANY_X((k_xfwd<0, 8, 0, XENG_RADIX16>), a);
+  else if (k.ax[0].dense.tiles) AWK_ANY_X((k_xfwd<0, 0, 0, XENG_DENSE>), a);
   else AWK_ANY_X((k_xfwd<0, 0, 0>), a);
 }
 
 void any_xinv(FluidKernel &k, const XInvArgs &a, bool apply, unsigned grid, hipStream_t s, const Batch &bt) {
-  if (k.ax[0].dense.tiles) {
+  if (k.ax[0].radix.ra > 16) {
+    if (apply) AWK_ANY_X((k_xinv<0, 8, 0, 1, false, true, false, XENG_RADIX32>), a);
+    else AWK_ANY_X((k_xinv<0, 8, 0, 1, false, false, false, XENG_RADIX32>), a);
+  } else if (k.ax[0].radix.ra) {
+    if (apply) AWK_ANY_X((k_xinv<0, 8, 0, 1, false, true, false, XENG_RADIX16>), a);
+    else AWK_ANY_X((k_xinv<0, 8, 0, 1, false, false, false, XENG_RADIX16>), a);
+  } else if (k.ax[0].dense.tiles) {
     if (apply) AWK_ANY_X((k_xinv<0, 0, 0, 1, false, true, false, XENG_DENSE>), a);
     else AWK_ANY_X((k_xinv<0, 0, 0, 1, false, false, false, XENG_DENSE>), a);
   } else if (apply) AWK_ANY_X((k_xinv<0, 0, 0, 1, false, true>), a);
@@ -202,23 +361,37 @@ void any_xinv(FluidKernel &k, const XInvArgs &a, bool apply, unsigned grid, hipS
 void any_ypass(FluidKernel &k, bool inv, const ReduceArgs &ra, hipStream_t s, const Batch &bt) {
   const int ntile = (k.nxh + k.tx_y - 1) / k.tx_y;
   const unsigned grid = grid_for((long long)3 * k.nz * ntile, 1);
-  if (k.ax[1].dense.tiles)
+  const RadixAxis r = k.ax[1].radix;
+#define AWK_YX(M)                                                                                \
+  AWK_LAUNCH(k_ypass_radix<M>, dim3(grid, bt.n), dim3(k.bd_y), k.lds_y, s, r, k.nz, k.nxh, k.nxh_pad, k.spec, \
+             k.spec_plane(), inv ? 1 : 0, ra, bt)
+  if (r.ra > 16) AWK_YX(32);
+  else if (r.ra) AWK_YX(16);
+  else if (k.ax[1].dense.tiles)
     AWK_LAUNCH(k_ypass_dense, dim3(grid, bt.n), dim3(k.bd_y), k.lds_y, s, k.ax[1].dense, k.nz, k.nxh,
                k.nxh_pad, k.spec, k.spec_plane(), inv ? 1 : 0, ra, bt);
   else
     AWK_LAUNCH(k_ypass, dim3(grid, bt.n), dim3(k.bd_y), k.lds_y, s, k.ax[1].dev(), k.ny, k.nz, k.nxh,
                k.nxh_pad, k.tx_y, k.spec, k.spec_plane(), inv ? 1 : 0, ra, bt);
+#undef AWK_YX
 }
 
 void any_zsolve(FluidKernel &k, const SolveArgs &sa, hipStream_t s, const Batch &bt) {
   const int ntile = (k.nxh + k.tx_z - 1) / k.tx_z;
   const unsigned grid = grid_for((long long)k.ny * ntile, 1);
-  if (k.ax[2].dense.tiles)
+  const RadixAxis r = k.ax[2].radix;
+#define AWK_ZX(M)                                                                                \
+  AWK_LAUNCH(k_zsolve_radix<M>, dim3(grid, bt.n), dim3(k.bd_z), k.lds_z, s, r, sa, k.ny, k.nxh, k.nxh_pad, \
+             k.spec, k.spec_plane(), bt)
+  if (r.ra > 16) AWK_ZX(32);
+  else if (r.ra) AWK_ZX(16);
+  else if (k.ax[2].dense.tiles)
     AWK_LAUNCH(k_zsolve_dense, dim3(grid, bt.n), dim3(k.bd_z), k.lds_z, s, k.ax[2].dense, sa, k.ny, k.nxh,
                k.nxh_pad, k.spec, k.spec_plane(), bt);
   else
     AWK_LAUNCH(k_zsolve, dim3(grid, bt.n), dim3(k.bd_z), k.lds_z, s, k.ax[2].dev(), sa, k.ny, k.nz, k.nxh,
                k.nxh_pad, k.tx_z, k.spec, k.spec_plane(), bt);
+#undef AWK_ZX
 }
 
 }  // namespace awk

@@ -76,17 +76,59 @@ __device__ __forceinline__ float load_mul(const XFwdArgs &a, size_t i) {
   return __builtin_nontemporal_load(a.i1 + i);
 }
 
-// Which transform an x pass runs: the LDS stages, or the dense product (awk_dense.h),
-// whose lines are the rows' components as real lines [x][kDenseLS].
-enum XEngine { XENG_STAGES = 0, XENG_DENSE = 1 };
+// Which transform an x pass runs: the LDS stages; the dense product (awk_dense.h),
+// whose lines are the rows' components as real lines [x][kDenseLS]; or two radices
+// (awk_radix.h) of up to 16 or 32, a thread per butterfly of the 12 complex lines.
+enum XEngine { XENG_STAGES = 0, XENG_DENSE = 1, XENG_RADIX16 = 2, XENG_RADIX32 = 3 };
+constexpr int x_threads(int eng, int bdc) {
+  return eng == XENG_DENSE || eng == XENG_RADIX32 ? 512 : eng == XENG_RADIX16 ? 256 : bdc ? bdc : 1024;
+}
 constexpr int kDenseLS = 33;   // floats per staged x (an odd stride: no bank conflicts along x)
 constexpr int kDenseRows = 10; // rows per dense x block: 30 of the product's 32 lines
-constexpr int kDenseXThreads = 512;  // at most: a wave per tile, and at least 4 waves
+
+// w / n for 0 <= w < 2^16 and a launch constant n < 2^16: m = ceil(2^32 / n) (0: n = 1).
+__device__ __forceinline__ int div_small(int w, unsigned m) {
+  return m ? (int)__umulhi((unsigned)w, m) : w;
+}
+
+// The 12 lines of an x block (row stride LS) through two radices in LDS.
+template <int MAXR, int NL, int LS>
+__device__ __forceinline__ void radix_lds(float2 *sm, const RadixAxis &ax, bool inv) {
+  const int line = threadIdx.x % NL, j = threadIdx.x / NL, RA = ax.ra, RB = ax.rb;
+  with_radix<MAXR>(RA, [&](auto rad) {
+    constexpr int R = decltype(rad)::value;
+    float2 v[R];
+    if (j < RB) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[r] = sm[(j + r * RB) * LS + line];
+      dft_any<R>(v, inv);
+    }
+    __syncthreads();
+    if (j < RB) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) sm[(j * R + r) * LS + line] = v[r];
+    }
+  });
+  __syncthreads();
+  with_radix<MAXR>(RB, [&](auto rad) {
+    constexpr int R = decltype(rad)::value;
+    if (j < RA) {
+      float2 v[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[r] = sm[(j + r * RA) * LS + line];
+      radix_twiddle<R>(v, ax.tw, j, inv);
+      dft_any<R>(v, inv);
+#pragma unroll
+      for (int r = 0; r < R; ++r) sm[(j + r * RA) * LS + line] = v[r];
+    }
+  });
+  __syncthreads();
+}
 
 // NC, RTC, BDC: compile-time length, rows per block and block size (0 = runtime).
 template <int NC, int RTC, int BDC, int ENG = XENG_STAGES>
-__global__ void __launch_bounds__(ENG == XENG_DENSE ? kDenseXThreads : BDC ? BDC : 1024)
-k_xfwd(XFwdArgs a, Axis ax, DenseAxis da, int nx_rt, int ny, int nz, int nxh_rt, int nxh_pad, int RT_rt,
+__global__ void __launch_bounds__(x_threads(ENG, BDC))
+k_xfwd(XFwdArgs a, Axis ax, XPlan xp, int nx_rt, int ny, int nz, int nxh_rt, int nxh_pad, int RT_rt,
        float2 *__restrict__ spec, size_t plane, Batch bt) {
   extern __shared__ float2 sm[];
   __shared__ double red[16];
@@ -104,6 +146,16 @@ k_xfwd(XFwdArgs a, Axis ax, DenseAxis da, int nx_rt, int ny, int nz, int nxh_rt,
   const int g = band_block(lb, a.band, ny / RT);  // the row group (its SSD partial's index)
   const int r0 = g * RT;
   if (r0 >= NR) return;
+  // y and z of the block's row q: from the first row's, without a division per voxel
+  const int zb = r0 / ny, yb0 = r0 - zb * ny;
+  auto row_yz = [&](int q, int &y, int &z) {
+    y = yb0 + q;
+    z = zb;
+    while (y >= ny) {
+      y -= ny;
+      ++z;
+    }
+  };
   double ssd = 0.0;
   float *smf = reinterpret_cast<float *>(sm);
   auto put = [&](int q, int x, float f0, float f1, float f2) {
@@ -184,7 +236,7 @@ k_xfwd(XFwdArgs a, Axis ax, DenseAxis da, int nx_rt, int ny, int nz, int nxh_rt,
   if (!done) {
 #pragma unroll
   for (int w = threadIdx.x; w < RT * nx; w += bdim) {
-    const int q = w / nx, x = w - q * nx;
+    const int q = NC ? w / nx : div_small(w, xp.mn), x = w - q * nx;
     const int row = r0 + q;
     float f0 = 0.f, f1 = 0.f, f2 = 0.f;
     if (row < NR) {
@@ -197,7 +249,8 @@ k_xfwd(XFwdArgs a, Axis ax, DenseAxis da, int nx_rt, int ny, int nz, int nxh_rt,
         // gradient of the deformed image (Array3DUtils::computeGradient, wrap=false,
         // Array3DUtils.txx:783-901), residual r = I1 - Idef and force r*grad
         // (GreedyIteratorCPU.cxx:108-117).
-        const int y = row % ny, z = row / ny;
+        int y, z;
+        row_yz(q, y, z);
         const float *I = a.idef;
         const float c = I[base];
         float gx = 0.f, gy = 0.f, gz = 0.f;
@@ -233,10 +286,10 @@ k_xfwd(XFwdArgs a, Axis ax, DenseAxis da, int nx_rt, int ny, int nz, int nxh_rt,
     __syncthreads();
     const int lane = threadIdx.x & 63, hi = lane >> 5, col = lane & 31;
     const int tile = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    if (tile < da.tiles) {
+    if (tile < xp.dense.tiles) {
       v16f E, O;
       dense_tile<true, true>(smf + hi * kDenseLS + col, smf + (nx - hi) * kDenseLS + col, 2 * kDenseLS,
-                             -2 * kDenseLS, da.tab + (size_t)tile * da.ks * 64 + lane, da.ks, E, O);
+                             -2 * kDenseLS, xp.dense.tab + (size_t)tile * xp.dense.ks * 64 + lane, xp.dense.ks, E, O);
       const int k = 32 * tile + col;
       if (k < nxh) {
 #pragma unroll
@@ -249,13 +302,15 @@ k_xfwd(XFwdArgs a, Axis ax, DenseAxis da, int nx_rt, int ny, int nz, int nxh_rt,
     }
   } else {
   __syncthreads();
-  if constexpr (NC != 0) ct_fft<NC, 3 * RTC / 2, 3 * RTC / 2 + 1, BDC>(sm, ax.tw, false);
+  if constexpr (ENG == XENG_RADIX16 || ENG == XENG_RADIX32)
+    radix_lds<ENG == XENG_RADIX16 ? 16 : 32, 3 * RTC / 2, 3 * RTC / 2 + 1>(sm, xp.radix, false);
+  else if constexpr (NC != 0) ct_fft<NC, 3 * RTC / 2, 3 * RTC / 2 + 1, BDC>(sm, ax.tw, false);
   else lds_fft(sm, ax, NL, LS, false, sm + (size_t)nx * LS);
 #pragma unroll
   for (int w = threadIdx.x; w < NL * nxh; w += bdim) {
-    const int line = w / nxh, k = w - line * nxh;
+    const int line = NC ? w / nxh : div_small(w, xp.mh), k = w - line * nxh;
     const float2 Z = sm[k * LS + line];
-    const float2 Zc = cconj(sm[((nx - k) % nx) * LS + line]);
+    const float2 Zc = cconj(sm[(k ? nx - k : 0) * LS + line]);
     const float2 A = cscale(cadd(Z, Zc), 0.5f);
     const float2 d = cscale(csub(Z, Zc), 0.5f);
     const float2 B = make_float2(d.y, -d.x);
@@ -288,8 +343,8 @@ k_xfwd(XFwdArgs a, Axis ax, DenseAxis da, int nx_rt, int ny, int nz, int nxh_rt,
 // neighbours staged in LDS.
 template <int NC, int RTC, int BDC, int XU, bool PAIRS = false, bool APPLY = false, bool STG = false,
           int ENG = XENG_STAGES>
-__global__ void __launch_bounds__(ENG == XENG_DENSE ? kDenseXThreads : BDC ? BDC : 1024)
-k_xinv(XInvArgs a, Axis ax, DenseAxis da, int nx_rt, int ny, int nz, int nxh_rt, int nxh_pad, int RT_rt,
+__global__ void __launch_bounds__(x_threads(ENG, BDC))
+k_xinv(XInvArgs a, Axis ax, XPlan xp, int nx_rt, int ny, int nz, int nxh_rt, int nxh_pad, int RT_rt,
        const float2 *__restrict__ spec, size_t plane, Batch bt) {
   extern __shared__ float2 sm[];
   __shared__ float redf[16];
@@ -321,7 +376,7 @@ k_xinv(XInvArgs a, Axis ax, DenseAxis da, int nx_rt, int ny, int nz, int nxh_rt,
     // x_j = sum_k w_k (cos Re X_k - sin Im X_k), w_0 = 1, else 2 (the table halves
     // the middle frequency of an even length): the parts of 30 real lines staged as
     // [k][kDenseLS], real then imaginary, rows nxh .. 2 ks - 1 zero
-    const int KR = 2 * da.ks;
+    const int KR = 2 * xp.dense.ks;
     float *im = smf + KR * kDenseLS;
     const int lane = threadIdx.x & 63, hi = lane >> 5, col = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), nw = bdim >> 6;
@@ -339,12 +394,12 @@ k_xinv(XInvArgs a, Axis ax, DenseAxis da, int nx_rt, int ny, int nz, int nxh_rt,
     }
     __syncthreads();
     v16f P, Q;
-    if (wave < da.tiles)
+    if (wave < xp.dense.tiles)
       dense_tile<true, false>(smf + hi * kDenseLS + col, im + hi * kDenseLS + col, 2 * kDenseLS,
-                              2 * kDenseLS, da.tab + (size_t)wave * da.ks * 64 + lane, da.ks, P, Q);
+                              2 * kDenseLS, xp.dense.tab + (size_t)wave * xp.dense.ks * 64 + lane, xp.dense.ks, P, Q);
     __syncthreads();  // the staged frequencies are read: the lines take their place
     const int j = 32 * wave + col;
-    if (wave < da.tiles && j < da.H) {
+    if (wave < xp.dense.tiles && j < xp.dense.H) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int line = dense_row(i, lane);
@@ -356,7 +411,7 @@ k_xinv(XInvArgs a, Axis ax, DenseAxis da, int nx_rt, int ny, int nz, int nxh_rt,
   } else {
 #pragma unroll
   for (int w = threadIdx.x; w < NL * nxh; w += bdim) {
-    const int line = w / nxh, k = w - line * nxh;
+    const int line = NC ? w / nxh : div_small(w, xp.mh), k = w - line * nxh;
     int rowA, cA, rowB, cB;
     line_targets(line, r0, rowA, cA, rowB, cB);
     float2 A = rowA < NR ? spec[cA * plane + (size_t)rowA * nxh_pad + k] : make_float2(0.f, 0.f);
@@ -369,7 +424,9 @@ k_xinv(XInvArgs a, Axis ax, DenseAxis da, int nx_rt, int ny, int nz, int nxh_rt,
     if (k > 0 && nx - k >= nxh) sm[(nx - k) * LS + line] = make_float2(A.x + B.y, B.x - A.y);  // conj(A) + i conj(B)
   }
   __syncthreads();
-  if constexpr (NC != 0) ct_fft<NC, 3 * RTC / 2, 3 * RTC / 2 + 1, BDC>(sm, ax.tw, true);
+  if constexpr (ENG == XENG_RADIX16 || ENG == XENG_RADIX32)
+    radix_lds<ENG == XENG_RADIX16 ? 16 : 32, 3 * RTC / 2, 3 * RTC / 2 + 1>(sm, xp.radix, true);
+  else if constexpr (NC != 0) ct_fft<NC, 3 * RTC / 2, 3 * RTC / 2 + 1, BDC>(sm, ax.tw, true);
   else lds_fft(sm, ax, NL, LS, true, sm + (size_t)nx * LS);
   }
   // the velocity at (q, x) of the block's rows
@@ -388,6 +445,16 @@ k_xinv(XInvArgs a, Axis ax, DenseAxis da, int nx_rt, int ny, int nz, int nxh_rt,
     } else {
       const float2 t = sm[x * LS + 3 * p + 2];
       v0 = t.x; v1 = t.y; v2 = sm[x * LS + 3 * p + 1].y;
+    }
+  };
+  // y and z of the block's row q: from the first row's, without a division per voxel
+  const int zb = r0 / ny, yb0 = r0 - zb * ny;
+  auto row_yz = [&](int q, int &y, int &z) {
+    y = yb0 + q;
+    z = zb;
+    while (y >= ny) {
+      y -= ny;
+      ++z;
     }
   };
   float mx = 0.f;
@@ -482,13 +549,14 @@ k_xinv(XInvArgs a, Axis ax, DenseAxis da, int nx_rt, int ny, int nz, int nxh_rt,
 #pragma unroll
       for (int u = 0; u < XU; ++u) {
         const int w = w0 + u * bdim;
-        const int q = w / nx, x = w - q * nx;
+        const int q = NC ? w / nx : div_small(w, xp.mn), x = w - q * nx;
         row_[u] = (w < RT * nx) ? r0 + q : NR;
         x_[u] = x;
         if (row_[u] < NR) {
           float v0, v1, v2;
           vel(q, x, v0, v1, v2);
-          const int y = row_[u] % ny, z = row_[u] / ny;
+          int y, z;
+          row_yz(q, y, z);
           // explicit fma: the same rounding wherever the position is formed
           px[u] = fmaf(v0 * st, isx, (float)x);
           py[u] = fmaf(v1 * st, isy, (float)y);
@@ -535,7 +603,7 @@ k_xinv(XInvArgs a, Axis ax, DenseAxis da, int nx_rt, int ny, int nz, int nxh_rt,
     }
 #pragma unroll
     for (int w = threadIdx.x; w < RT * nx; w += bdim) {
-      const int q = w / nx, x = w - q * nx;
+      const int q = NC ? w / nx : div_small(w, xp.mn), x = w - q * nx;
       const int row = r0 + q;
       if (row >= NR) continue;
       float v0, v1, v2;

@@ -78,7 +78,7 @@ enum {
  * subjects per group of one fused launch; read when an atlas iteration is
  * launched or captured); results do not depend on them.  FFT plan knobs read when an operator is created:
  * "fft_order", "x_rt", "y_tx", "z_tx" (another butterfly order or tile, results
- * within FP32 rounding).  Process-wide.  No counterpart in the reference. */
+ * within FP32 rounding; for lengths that neither a two-radix nor a dense plan takes).  Process-wide.  No counterpart in the reference. */
 awk_status awk_tune_set(const char *name, int value);
 awk_status awk_tune_get(const char *name, int *value);
 

@@ -156,3 +156,31 @@ def test_dense_axes_greedy_matches_oracle(shape):
     data = w.RunWarp()
     assert np.max(np.abs(data.energies() - ed) / ed) < 1e-3
     assert rel_l2(host(data.Def1To0), soa(hd)) <= 1e-5
+
+
+# A length with two radices up to 32 (prime factors up to 13) is transformed in
+# registers: every radix as the larger and most as the smaller of the two, one radix
+# alone, and the longest
+RADIX_LENGTHS = [2, 3, 7, 11, 13, 14, 26, 39, 44, 60, 72, 80, 110, 143, 165, 168, 182, 195, 208, 240, 270, 286,
+                 315, 320, 325, 384, 405, 416, 420, 448, 450, 810, 960, 1024]
+
+
+@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("n", RADIX_LENGTHS)
+def test_radix_axis_matches_oracle(n, axis):
+    """L^-1 with one long two-radix axis.  Bar: six transforms of at most 10 levels of
+    butterflies (2^-24 each in the mean square, sqrt(60) in all: 4.6e-7) and the solve
+    (5e-7): 1e-6."""
+    from atlaswerks_amd.fluid import DiffOperGPU, DiffOperParam
+    from gpu_util import aos, host, rel_l2, soa, to_dev
+    shape = [5, 12, 9]
+    shape[axis] = n
+    nz, ny, nx = shape
+    print("fluid radix", shape, flush=True)
+    f = _field(tuple(shape), seed=n + axis)
+    sp = (1.0, 1.25, 0.8)
+    op = DiffOperGPU((nx, ny, nz), sp, DiffOperParam(alpha=0.01, beta=0.01, gamma=0.001))
+    d = to_dev(f)
+    op.ApplyInverseOperator(d)
+    ref = oracle.diffoper(aos(f), sp=sp, alpha=0.01, beta=0.01, gamma=0.001, inverse=True)
+    assert rel_l2(host(d), soa(ref)) <= 1e-6
