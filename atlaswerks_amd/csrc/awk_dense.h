@@ -145,6 +145,32 @@ __device__ __forceinline__ void dense_stage(float *sm, const float2 *__restrict_
   }
 }
 
+// The same for three components (planes `plane` apart), one after the other in LDS.
+__device__ __forceinline__ void dense_stage3(float *sm, const float2 *__restrict__ base, size_t plane,
+                                             size_t st, int n, int nvalid) {
+  const int t = (int)threadIdx.x & 15, j0 = (int)threadIdx.x >> 4, dj = (int)blockDim.x >> 4;
+  float2 *s2 = reinterpret_cast<float2 *>(sm);
+  const bool ok = t < nvalid;
+  for (int j = j0; j <= n; j += 4 * dj) {
+    float2 v[3][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = j + i * dj;
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+        v[c][i] = (ok && r < n) ? base[c * plane + (size_t)r * st + t] : make_float2(0.f, 0.f);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = j + i * dj;
+      if (r <= n) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) s2[(c * (n + 1) + r) * 16 + t] = v[c][i];
+      }
+    }
+  }
+}
+
 // X_k and X_{n-k} of a tile to rows k and n - k of base (row stride st floats), the
 // first nvalid complex columns.
 __device__ __forceinline__ void dense_store(float *base, size_t st, const DenseAxis &ax, int tile,

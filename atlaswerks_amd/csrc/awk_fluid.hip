@@ -443,12 +443,15 @@ awk_status fk_init(FluidKernel &k, int nx, int ny, int nz, const float sp[3]) {
   if (!k.rt || !k.tx_y || !k.tx_z) return fail(AWK_ERR_UNSUPPORTED, "fluid kernel: axis too long for LDS staging");
   k.bd_x = rx[0]->ra ? std::max(256, (12 * rx[0]->ra + 63) / 64 * 64) : dx[0]->tiles ? std::max(256, 64 * dx[0]->tiles) : pick_bd(k.ax[0].stage_len(), 3 * k.rt / 2);
   k.bd_y = rx[1]->ra ? 16 * rx[1]->ra : dx[1]->tiles ? 64 * dx[1]->tiles : pick_bd(k.ax[1].stage_len(), k.tx_y);
-  k.bd_z = rx[2]->ra ? 16 * rx[2]->ra : dx[2]->tiles ? 64 * dx[2]->tiles : pick_bd(k.ax[2].stage_len(), 3 * k.tx_z);
+  // along z a wave per tile and component (or thread group per component) where they fit a block
+  const bool z3 = dx[2]->tiles ? dx[2]->tiles <= 5 : rx[2]->ra <= 16;
+  k.bd_z = (z3 ? 3 : 1) * (rx[2]->ra ? (z3 ? (16 * rx[2]->ra + 63) / 64 * 64 : 16 * rx[2]->ra) : dx[2]->tiles ? 64 * dx[2]->tiles : 0);
+  if (!k.bd_z) k.bd_z = pick_bd(k.ax[2].stage_len(), 3 * k.tx_z);
   if (k.bd_x > 1024 || k.bd_y > 1024 || k.bd_z > 1024)
     return fail(AWK_ERR_UNSUPPORTED, "fluid kernel: block too large");
   k.lds_x = x_lds(k.ax[0], k.rt);
   k.lds_y = std::max(yz_lds(k.ax[1], k.tx_y), (size_t)k.bd_y * sizeof(double));  // (the energy tree)
-  k.lds_z = yz_lds(k.ax[2], 3 * k.tx_z);
+  k.lds_z = yz_lds(k.ax[2], 3 * k.tx_z) * (dx[2]->tiles && z3 ? 3 : 1);
   if (awk_status st = any_setup((int)kPassLdsMax)) return st;
   // twiddles and LUT (double -> float); the Bluestein tables follow the three
   // axes' twiddles in the same allocation
@@ -617,10 +620,11 @@ awk_status fk_zsolve(FluidKernel &k, bool inverse_op, hipStream_t s, const Batch
 #define AWK_ZR(N, RA, RB)                                                                     \
   AWK_LAUNCH((k_zsolve_reg<N, RA, RB, 16>), dim3(g16, bt.n), dim3(16 * (N / RA > N / RB ? N / RA : N / RB)), \
                      0, s, tw, sa, k.ny, k.nxh, k.nxh_pad, k.spec, k.spec_plane(), bt)
+  // 64 and below go through the two-radix kernel, whose thread groups hold one
+  // component each: 11.0 -> 8.2 us at 64^3 and 8.1 -> 6.4 at 32^3; at 128 the line in
+  // registers is the faster (21.3 against 23.8 us)
   if (k.nz == 256) AWK_ZR(256, 16, 16);
   else if (k.nz == 128) AWK_ZR(128, 16, 8);
-  else if (k.nz == 64) AWK_ZR(64, 8, 8);
-  else if (k.nz == 32) AWK_ZR(32, 8, 4);
   else any_zsolve(k, sa, s, bt);
 #undef AWK_ZR
   AWK_LAUNCH_CHECK("k_zsolve");

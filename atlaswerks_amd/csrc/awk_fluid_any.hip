@@ -161,6 +161,50 @@ k_zsolve_dense(DenseAxis az, SolveArgs sa, int ny, int nxh, int nxh_pad, float2 
   }
 }
 
+// The same with the three components in LDS side by side and a wave per 32 frequencies
+// of one component: the loads of all three in flight at once, a third of the serial
+// products per wave, and the frequencies solved in pairs of parts (one factorisation
+// per frequency).  For lengths whose 3 * tiles waves fit a block; 181 x 217 x 91
+// frequencies 216 -> 189 us, about 57 us of it the matrix cores'.
+__global__ void __launch_bounds__(1024, 5)
+k_zsolve_dense3(DenseAxis az, SolveArgs sa, int ny, int nxh, int nxh_pad, float2 *__restrict__ spec,
+                size_t plane, Batch bt) {
+  extern __shared__ float2 sm[];
+  float *smf = reinterpret_cast<float *>(sm);
+  spec += (long long)blockIdx.y * bt.spec;
+  const int ntile = (nxh + 15) / 16;
+  const int lb = (int)xcd_block();
+  if (lb >= ny * ntile) return;
+  const int tile = lb % ntile, ky = lb / ntile;
+  const int kx0 = tile * 16, nvalid = min(16, nxh - kx0);
+  const size_t zst = (size_t)ny * nxh_pad;
+  float2 *base = spec + (size_t)ky * nxh_pad + kx0;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int cs = (az.n + 1) * 32;  // floats per component
+  const int c = wave % 3, w = wave / 3;
+  dense_stage3(smf, base, plane, zst, az.n, nvalid);
+  __syncthreads();
+  v16f A, B;
+  dense_lines(smf + c * cs, az, w, lane, false, A, B);
+  __syncthreads();
+  dense_store(smf + c * cs, 32, az, w, lane, 16, A, B);  // row n stays zero
+  __syncthreads();
+  for (int e = threadIdx.x; e < az.n * 16; e += blockDim.x) {
+    const int t = e & 15, kz = e >> 4;
+    if (t < nvalid) {
+      float2 *p = sm + e;
+      float2 b0 = p[0], b1 = p[cs / 2], b2 = p[cs];
+      solve_one(sa, kx0 + t, ky, kz, ny, nxh, b0, b1, b2);
+      p[0] = b0;
+      p[cs / 2] = b1;
+      p[cs] = b2;
+    }
+  }
+  __syncthreads();
+  dense_lines(smf + c * cs, az, w, lane, true, A, B);
+  dense_store(reinterpret_cast<float *>(base + c * plane), 2 * zst, az, w, lane, nvalid, A, B);
+}
+
 // ------------------------------------------------------------------
 // Lengths n = ra * rb (awk_radix.h).  Thread (t, j): kx column t of 16 (128-byte rows),
 // butterfly j < max(ra, rb).  MAXR: the largest radix compiled in (16, or 32 for
@@ -178,16 +222,19 @@ k_ypass_radix(RadixAxis ax, int nz, int nxh, int nxh_pad, float2 *__restrict__ s
   if (lb >= 3 * nz * ntile) return;
   const int tile = lb % ntile, rest = lb / ntile;
   const int z = rest % nz, c = rest / nz;
-  const int kx = tile * 16 + t;
-  const bool valid = kx < nxh, iv = inv != 0;
-  float2 *base = spec + c * plane + (size_t)z * ax.n * nxh_pad + kx;
+  const bool valid = tile * 16 + t < nxh, iv = inv != 0;
+  // row j + r * step of the slab: a uniform base per r and one lane offset
+  char *base = reinterpret_cast<char *>(spec + c * plane + (size_t)z * ax.n * nxh_pad + tile * 16);
+  const size_t rs = (size_t)nxh_pad * sizeof(float2);
+  const unsigned lo = (unsigned)(j * nxh_pad + t) * (unsigned)sizeof(float2);
+  auto row = [&](int r) -> float2 & { return *reinterpret_cast<float2 *>(base + (size_t)r * rs + lo); };
   const int RA = ax.ra, RB = ax.rb;
   with_radix<MAXR>(RA, [&](auto rad) {
     constexpr int R = decltype(rad)::value;
     if (j < RB) {
       float2 v[R];
 #pragma unroll
-      for (int r = 0; r < R; ++r) v[r] = valid ? base[(size_t)(j + r * RB) * nxh_pad] : make_float2(0.f, 0.f);
+      for (int r = 0; r < R; ++r) v[r] = valid ? row(r * RB) : make_float2(0.f, 0.f);
       dft_any<R>(v, iv);
 #pragma unroll
       for (int r = 0; r < R; ++r) sm[(j * R + r) * 16 + t] = v[r];
@@ -204,7 +251,7 @@ k_ypass_radix(RadixAxis ax, int nz, int nxh, int nxh_pad, float2 *__restrict__ s
       dft_any<R>(v, iv);
       if (valid) {
 #pragma unroll
-        for (int r = 0; r < R; ++r) base[(size_t)(j + r * RA) * nxh_pad] = v[r];
+        for (int r = 0; r < R; ++r) row(r * RA) = v[r];
       }
     }
   });
@@ -217,32 +264,45 @@ k_ypass_radix(RadixAxis ax, int nz, int nxh, int nxh_pad, float2 *__restrict__ s
 
 // The three components' lines stay in LDS.  A thread's stage-B slots, its frequencies
 // and the first inverse stage's slots (the forward stages transposed) are the same
-// ones, so between stage A and its transpose nothing is exchanged: two barriers.
-template <int MAXR>
-__global__ void __launch_bounds__(16 * MAXR)
+// ones, so stage A and its transpose are the only exchanges along z.  CG: component
+// groups of threads; 3 groups each take a component of every transform and a third of
+// the frequencies (three times the loads in flight and a third of the serial chain,
+// which is what small grids wait for), 1 group takes them in turn (radices up to 32,
+// whose three groups would not fit a block).  Measured against one group: 144 x 192 x 81
+// frequencies 54.6 -> 43.3 us (2.6 TB/s), 36 x 31 x 17 9.8 -> 6.7 us.
+template <int MAXR, int CG>
+__global__ void __launch_bounds__(16 * MAXR * CG)
 k_zsolve_radix(RadixAxis az, SolveArgs sa, int ny, int nxh, int nxh_pad, float2 *__restrict__ spec,
                size_t plane, Batch bt) {
   extern __shared__ float2 sm[];
   spec += (long long)blockIdx.y * bt.spec;
-  const int t = threadIdx.x & 15, j = threadIdx.x >> 4;
+  const int RA = az.ra, RB = az.rb, cs = az.n * 16;  // LDS elements per component
+  // whole waves per component group
+  const int gs = CG == 1 ? (int)blockDim.x : (int)blockDim.x / CG;
+  const int c0 = CG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / gs);
+  const int u = (int)threadIdx.x - c0 * gs, t = u & 15, j = u >> 4;
   const int ntile = (nxh + 15) / 16;
   const int lb = (int)xcd_block();
   if (lb >= ny * ntile) return;
   const int tile = lb % ntile, ky = lb / ntile;
   const int kx = tile * 16 + t;
   const bool valid = kx < nxh;
-  const size_t zst = (size_t)ny * nxh_pad;
-  float2 *base = spec + (size_t)ky * nxh_pad + kx;
-  const int RA = az.ra, RB = az.rb, cs = az.n * 16;  // LDS elements per component
+  // row j + r of a component: a uniform base per r and one lane offset
+  char *base = reinterpret_cast<char *>(spec + (size_t)ky * nxh_pad + tile * 16);
+  const size_t rs = (size_t)ny * nxh_pad * sizeof(float2), ps = plane * sizeof(float2);
+  const size_t lo = (size_t)j * rs + t * sizeof(float2);
+  auto row = [&](int c, int r) -> float2 & {
+    return *reinterpret_cast<float2 *>(base + c * ps + (size_t)r * rs + lo);
+  };
   with_radix<MAXR>(RA, [&](auto rad) {
     constexpr int R = decltype(rad)::value;
     if (j < RB) {
 #pragma unroll 1
-      for (int c = 0; c < 3; ++c) {
+      for (int c = c0; c < 3; c += CG) {
         float2 v[R];
 #pragma unroll
         for (int r = 0; r < R; ++r)
-          v[r] = valid ? base[c * plane + (size_t)(j + r * RB) * zst] : make_float2(0.f, 0.f);
+          v[r] = valid ? row(c, r * RB) : make_float2(0.f, 0.f);
         dft_any<R>(v, false);
 #pragma unroll
         for (int r = 0; r < R; ++r) sm[c * cs + (j * R + r) * 16 + t] = v[r];
@@ -252,38 +312,41 @@ k_zsolve_radix(RadixAxis az, SolveArgs sa, int ny, int nxh, int nxh_pad, float2 
   __syncthreads();
   with_radix<MAXR>(RB, [&](auto rad) {
     constexpr int R = decltype(rad)::value;
-    if (j < RA) {
 #pragma unroll 1
-      for (int c = 0; c < 3; ++c) {
-        float2 v[R];
+    for (int c = j < RA ? c0 : 3; c < 3; c += CG) {
+      float2 v[R];
 #pragma unroll
-        for (int r = 0; r < R; ++r) v[r] = sm[c * cs + (j + r * RA) * 16 + t];
-        radix_twiddle<R>(v, az.tw, j, false);
-        dft_any<R>(v, false);
+      for (int r = 0; r < R; ++r) v[r] = sm[c * cs + (j + r * RA) * 16 + t];
+      radix_twiddle<R>(v, az.tw, j, false);
+      dft_any<R>(v, false);
 #pragma unroll
-        for (int r = 0; r < R; ++r) sm[c * cs + (j + r * RA) * 16 + t] = v[r];
-      }
-      if (valid) {
+      for (int r = 0; r < R; ++r) sm[c * cs + (j + r * RA) * 16 + t] = v[r];
+    }
+  });
+  if (CG > 1) __syncthreads();
+  if (valid && j < RA) {
 #pragma unroll 2
-        for (int r = 0; r < R; ++r) {
-          float2 *p = sm + (j + r * RA) * 16 + t;
-          float2 b0 = p[0], b1 = p[cs], b2 = p[2 * cs];
-          solve_one(sa, kx, ky, j + r * RA, ny, nxh, b0, b1, b2);
-          p[0] = b0;
-          p[cs] = b1;
-          p[2 * cs] = b2;
-        }
-      }
+    for (int r = c0; r < RB; r += CG) {
+      float2 *p = sm + (j + r * RA) * 16 + t;
+      float2 b0 = p[0], b1 = p[cs], b2 = p[2 * cs];
+      solve_one(sa, kx, ky, j + r * RA, ny, nxh, b0, b1, b2);
+      p[0] = b0;
+      p[cs] = b1;
+      p[2 * cs] = b2;
+    }
+  }
+  if (CG > 1) __syncthreads();
+  with_radix<MAXR>(RB, [&](auto rad) {
+    constexpr int R = decltype(rad)::value;
 #pragma unroll 1
-      for (int c = 0; c < 3; ++c) {
-        float2 v[R];
+    for (int c = j < RA ? c0 : 3; c < 3; c += CG) {
+      float2 v[R];
 #pragma unroll
-        for (int r = 0; r < R; ++r) v[r] = sm[c * cs + (j + r * RA) * 16 + t];
-        dft_any<R>(v, true);
-        radix_twiddle<R>(v, az.tw, j, true);
+      for (int r = 0; r < R; ++r) v[r] = sm[c * cs + (j + r * RA) * 16 + t];
+      dft_any<R>(v, true);
+      radix_twiddle<R>(v, az.tw, j, true);
 #pragma unroll
-        for (int r = 0; r < R; ++r) sm[c * cs + (j + r * RA) * 16 + t] = v[r];
-      }
+      for (int r = 0; r < R; ++r) sm[c * cs + (j + r * RA) * 16 + t] = v[r];
     }
   });
   __syncthreads();
@@ -291,14 +354,14 @@ k_zsolve_radix(RadixAxis az, SolveArgs sa, int ny, int nxh, int nxh_pad, float2 
     constexpr int R = decltype(rad)::value;
     if (j < RB) {
 #pragma unroll 1
-      for (int c = 0; c < 3; ++c) {
+      for (int c = c0; c < 3; c += CG) {
         float2 v[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) v[r] = sm[c * cs + (j * R + r) * 16 + t];
         dft_any<R>(v, true);
         if (valid) {
 #pragma unroll
-          for (int r = 0; r < R; ++r) base[c * plane + (size_t)(j + r * RB) * zst] = v[r];
+          for (int r = 0; r < R; ++r) row(c, r * RB) = v[r];
         }
       }
     }
@@ -324,8 +387,9 @@ awk_status any_setup(int lds_max) {
                        reinterpret_cast<const void *>(&k_xfwd<0, 8, 0, XENG_RADIX32>),
                        reinterpret_cast<const void *>(&k_xinv<0, 8, 0, 1, false, false, false, XENG_RADIX32>),
                        reinterpret_cast<const void *>(&k_xinv<0, 8, 0, 1, false, true, false, XENG_RADIX32>),
-                       reinterpret_cast<const void *>(&k_zsolve_radix<16>),
-                       reinterpret_cast<const void *>(&k_zsolve_radix<32>),
+                       reinterpret_cast<const void *>(&k_zsolve_dense3),
+                       reinterpret_cast<const void *>(&k_zsolve_radix<16, 3>),
+                       reinterpret_cast<const void *>(&k_zsolve_radix<32, 1>),
                        reinterpret_cast<const void *>(&k_ypass_radix<32>)};
   for (const void *f : fns) AWK_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds_max));
   done = true;
@@ -380,11 +444,14 @@ void any_zsolve(FluidKernel &k, const SolveArgs &sa, hipStream_t s, const Batch 
   const int ntile = (k.nxh + k.tx_z - 1) / k.tx_z;
   const unsigned grid = grid_for((long long)k.ny * ntile, 1);
   const RadixAxis r = k.ax[2].radix;
-#define AWK_ZX(M)                                                                                \
-  AWK_LAUNCH(k_zsolve_radix<M>, dim3(grid, bt.n), dim3(k.bd_z), k.lds_z, s, r, sa, k.ny, k.nxh, k.nxh_pad, \
+#define AWK_ZX(M, CG)                                                                            \
+  AWK_LAUNCH((k_zsolve_radix<M, CG>), dim3(grid, bt.n), dim3(k.bd_z), k.lds_z, s, r, sa, k.ny, k.nxh, k.nxh_pad, \
              k.spec, k.spec_plane(), bt)
-  if (r.ra > 16) AWK_ZX(32);
-  else if (r.ra) AWK_ZX(16);
+  if (r.ra > 16) AWK_ZX(32, 1);
+  else if (r.ra) AWK_ZX(16, 3);
+  else if (k.ax[2].dense.tiles && k.bd_z == 192 * k.ax[2].dense.tiles)
+    AWK_LAUNCH(k_zsolve_dense3, dim3(grid, bt.n), dim3(k.bd_z), k.lds_z, s, k.ax[2].dense, sa, k.ny, k.nxh,
+               k.nxh_pad, k.spec, k.spec_plane(), bt);
   else if (k.ax[2].dense.tiles)
     AWK_LAUNCH(k_zsolve_dense, dim3(grid, bt.n), dim3(k.bd_z), k.lds_z, s, k.ax[2].dense, sa, k.ny, k.nxh,
                k.nxh_pad, k.spec, k.spec_plane(), bt);
