@@ -76,6 +76,62 @@ __device__ __forceinline__ float load_mul(const XFwdArgs &a, size_t i) {
   return __builtin_nontemporal_load(a.i1 + i);
 }
 
+// Column mode of the force: this thread owns column x of CR of the block's rows, q0 ..
+// q0 + CR - 1, which are consecutive y at one z (yb: the block's first).  Each Idef
+// value is loaded once: the column with a one-row halo in y, the two neighbouring z
+// rows, and x +- 1 from the neighbouring lanes (a load only at the wave edges).  Idef
+// and I1 are loaded non-temporally (the halo rows other blocks re-read come from L2):
+// with the apply's hfield loads and the composition's hfield stores also streamed,
+// the memory-side cache keeps this pass's spectrum for the y pass (256^3 greedy
+// iteration: y pass 89 -> 78 us, whole iteration +4 %, measured).
+template <int CR, class Put>
+__device__ __forceinline__ void column_force(const XFwdArgs &a, int nx, int ny, int nz, int z, int yb, int q0,
+                                             int x, Put put, double &ssd) {
+  const int y0 = yb + q0;
+  const size_t sxy = (size_t)nx * ny;
+  const float *col0 = a.idef + (size_t)z * sxy + (size_t)y0 * nx + x;
+  float col[CR + 2], zm[CR], zp[CR], i1v[CR], lft[CR], rgt[CR];
+#pragma unroll
+  for (int k = 0; k < CR + 2; ++k) {
+    const int yy = y0 - 1 + k;
+    col[k] = (yy >= 0 && yy < ny) ? __builtin_nontemporal_load(col0 + (ptrdiff_t)(k - 1) * nx) : 0.f;
+  }
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int q = 0; q < CR; ++q) {
+    zm[q] = (z > 0) ? __builtin_nontemporal_load(col0 + (ptrdiff_t)q * nx - (ptrdiff_t)sxy) : 0.f;
+    zp[q] = (z < nz - 1) ? __builtin_nontemporal_load(col0 + (ptrdiff_t)q * nx + (ptrdiff_t)sxy) : 0.f;
+    i1v[q] = load_mul(a, (size_t)z * sxy + (size_t)(y0 + q) * nx + x);
+    lft[q] = (lane == 0 && x > 0) ? col0[(ptrdiff_t)q * nx - 1] : 0.f;
+    rgt[q] = (lane == 63 && x < nx - 1) ? col0[(ptrdiff_t)q * nx + 1] : 0.f;
+  }
+#pragma unroll
+  for (int q = 0; q < CR; ++q) {
+    const float c = col[q + 1];
+    const float up = __shfl_up(c, 1, 64), dn = __shfl_down(c, 1, 64);
+    const float cl = (lane == 0) ? lft[q] : up;   // value at x - 1
+    const float cr = (lane == 63) ? rgt[q] : dn;  // value at x + 1
+    const int y = y0 + q;
+    // Array3DUtils::computeGradient (Array3DUtils.txx:783-901), wrap = false
+    float gx, gy, gz;
+    if (nx == 1) gx = 0.f;
+    else if (x > 0 && x < nx - 1) gx = div_const((cr - cl), 2.f * a.sp[0], a.r2sp[0]);
+    else if (x == 0) gx = div_const((cr - c), a.sp[0], a.rsp[0]);
+    else gx = div_const((c - cl), a.sp[0], a.rsp[0]);
+    if (ny == 1) gy = 0.f;
+    else if (y > 0 && y < ny - 1) gy = div_const((col[q + 2] - col[q]), 2.f * a.sp[1], a.r2sp[1]);
+    else if (y == 0) gy = div_const((col[q + 2] - c), a.sp[1], a.rsp[1]);
+    else gy = div_const((c - col[q]), a.sp[1], a.rsp[1]);
+    if (nz == 1) gz = 0.f;
+    else if (z > 0 && z < nz - 1) gz = div_const((zp[q] - zm[q]), 2.f * a.sp[2], a.r2sp[2]);
+    else if (z == 0) gz = div_const((zp[q] - c), a.sp[2], a.rsp[2]);
+    else gz = div_const((c - zm[q]), a.sp[2], a.rsp[2]);
+    const float r = (a.mode == XLOAD_FORCE) ? i1v[q] - c : i1v[q];
+    ssd += (double)r * (double)r;
+    put(q0 + q, x, gx * r, gy * r, gz * r);
+  }
+}
+
 // Which transform an x pass runs: the LDS stages; the dense product (awk_dense.h),
 // whose lines are the rows' components as real lines [x][kDenseLS]; or two radices
 // (awk_radix.h) of up to 16 or 32, a thread per butterfly of the 12 complex lines.
@@ -177,59 +233,25 @@ k_xfwd(XFwdArgs a, Axis ax, XPlan xp, int nx_rt, int ny, int nz, int nxh_rt, int
   };
   bool done = false;
   if constexpr (NC != 0 && NC == BDC) {
-    // Column mode: thread x owns column x of the block's RT rows, which are RT
-    // consecutive y at one z.  Each Idef value is loaded once: the column with a
-    // one-row halo in y, the two neighbouring z rows, and x +- 1 from the
-    // neighbouring lanes (a load only at the wave edges).  Idef and I1 are loaded
-    // non-temporally (the halo rows other blocks re-read come from L2): with the
-    // apply's hfield loads and the composition's hfield stores also streamed,
-    // the memory-side cache keeps this pass's spectrum for the y pass (256^3
-    // greedy iteration: y pass 89 -> 78 us, whole iteration +4 %, measured).
     if (a.mode != XLOAD_PLAIN && ny % RTC == 0) {
       done = true;
-      const int x = threadIdx.x;
-      const int z = r0 / ny, y0 = r0 - z * ny;
-      const size_t sxy = (size_t)NC * ny;
-      const float *I = a.idef;
-      const float *col0 = I + (size_t)z * sxy + (size_t)y0 * NC + x;
-      float col[RTC + 2], zm[RTC], zp[RTC], i1v[RTC], lft[RTC], rgt[RTC];
-#pragma unroll
-      for (int k = 0; k < RTC + 2; ++k) {
-        const int yy = y0 - 1 + k;
-        col[k] = (yy >= 0 && yy < ny) ? __builtin_nontemporal_load(col0 + (ptrdiff_t)(k - 1) * NC) : 0.f;
-      }
-      const int lane = threadIdx.x & 63;
-#pragma unroll
-      for (int q = 0; q < RTC; ++q) {
-        zm[q] = (z > 0) ? __builtin_nontemporal_load(col0 + (ptrdiff_t)q * NC - (ptrdiff_t)sxy) : 0.f;
-        zp[q] = (z < nz - 1) ? __builtin_nontemporal_load(col0 + (ptrdiff_t)q * NC + (ptrdiff_t)sxy) : 0.f;
-        i1v[q] = load_mul(a, (size_t)z * sxy + (size_t)(y0 + q) * NC + x);
-        lft[q] = (lane == 0 && x > 0) ? col0[(ptrdiff_t)q * NC - 1] : 0.f;
-        rgt[q] = (lane == 63 && x < NC - 1) ? col0[(ptrdiff_t)q * NC + 1] : 0.f;
-      }
-#pragma unroll
-      for (int q = 0; q < RTC; ++q) {
-        const float c = col[q + 1];
-        const float up = __shfl_up(c, 1, 64), dn = __shfl_down(c, 1, 64);
-        const float cl = (lane == 0) ? lft[q] : up;   // value at x - 1
-        const float cr = (lane == 63) ? rgt[q] : dn;  // value at x + 1
-        const int y = y0 + q;
-        // Array3DUtils::computeGradient (Array3DUtils.txx:783-901), wrap = false
-        float gx, gy, gz;
-        if (x > 0 && x < NC - 1) gx = div_const((cr - cl), 2.f * a.sp[0], a.r2sp[0]);
-        else if (x == 0) gx = div_const((cr - c), a.sp[0], a.rsp[0]);
-        else gx = div_const((c - cl), a.sp[0], a.rsp[0]);
-        if (ny == 1) gy = 0.f;
-        else if (y > 0 && y < ny - 1) gy = div_const((col[q + 2] - col[q]), 2.f * a.sp[1], a.r2sp[1]);
-        else if (y == 0) gy = div_const((col[q + 2] - c), a.sp[1], a.rsp[1]);
-        else gy = div_const((c - col[q]), a.sp[1], a.rsp[1]);
-        if (nz == 1) gz = 0.f;
-        else if (z > 0 && z < nz - 1) gz = div_const((zp[q] - zm[q]), 2.f * a.sp[2], a.r2sp[2]);
-        else if (z == 0) gz = div_const((zp[q] - c), a.sp[2], a.rsp[2]);
-        else gz = div_const((c - zm[q]), a.sp[2], a.rsp[2]);
-        const float r = (a.mode == XLOAD_FORCE) ? i1v[q] - c : i1v[q];
-        ssd += (double)r * (double)r;
-        put(q, x, gx * r, gy * r, gz * r);
+      column_force<RTC>(a, NC, ny, nz, zb, yb0, 0, (int)threadIdx.x, put, ssd);
+    }
+  } else if constexpr (ENG != XENG_STAGES) {
+    // the same for any length where the block's rows lie in one plane and its threads
+    // cover a row: 256 threads take rows of up to 128 in two halves of the block's
+    // rows, up to 64 (and an even half) in four quarters
+    constexpr int RC = ENG == XENG_DENSE ? kDenseRows : 8;
+    if (a.mode != XLOAD_PLAIN && nx <= bdim && yb0 + RC <= ny) {
+      done = true;
+      if (nx <= 64 && RC % 4 == 0) {
+        const int h = threadIdx.x >> 6, x = threadIdx.x & 63;
+        if (x < nx && h < 4) column_force<(RC + 3) / 4>(a, nx, ny, nz, zb, yb0, h * (RC / 4), x, put, ssd);
+      } else if (nx <= 128) {
+        const int h = threadIdx.x >> 7, x = threadIdx.x & 127;
+        if (x < nx && h < 2) column_force<RC / 2>(a, nx, ny, nz, zb, yb0, h * (RC / 2), x, put, ssd);
+      } else if ((int)threadIdx.x < nx) {
+        column_force<RC>(a, nx, ny, nz, zb, yb0, 0, (int)threadIdx.x, put, ssd);
       }
     }
   }

@@ -184,3 +184,22 @@ def test_radix_axis_matches_oracle(n, axis):
     op.ApplyInverseOperator(d)
     ref = oracle.diffoper(aos(f), sp=sp, alpha=0.01, beta=0.01, gamma=0.001, inverse=True)
     assert rel_l2(host(d), soa(ref)) <= 1e-6
+
+
+@pytest.mark.parametrize("shape", [(6, 20, 40), (5, 16, 64), (5, 11, 100), (4, 9, 150), (3, 10, 300), (3, 21, 134),
+                                   (1, 16, 40), (16, 1, 48), (2, 24, 17)])
+def test_force_columns_match_oracle(shape):
+    """The force formed by columns (quarters, halves or all of a block's rows per
+    thread) and voxel by voxel (row groups over a plane's end, rows longer than the
+    block) in one grid: the greedy parity tests' bars."""
+    import torch
+    from atlaswerks_amd.greedy import GreedyWarp
+    from gpu_util import host, rel_l2, soa
+    print("greedy columns", shape, flush=True)
+    t, h, _ = synth.pair(shape, seed=4, max_disp=1.0)
+    target = oracle.apply(t, np.moveaxis(h, 0, -1), dtype=np.float32)
+    sp = (1.2, 0.9, 1.0)
+    hd, _, _, ed, _ = oracle.greedy_run(t, target, 4, sp=sp)
+    data = GreedyWarp(torch.from_numpy(t).cuda(), torch.from_numpy(target).cuda(), 4, spacing=sp).RunWarp()
+    assert np.max(np.abs(data.energies() - ed) / ed) < 1e-3
+    assert rel_l2(host(data.Def1To0), soa(hd)) <= 1e-5
