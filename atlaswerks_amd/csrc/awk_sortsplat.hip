@@ -14,6 +14,8 @@
 //      order (float) over LDS tiles of the sorted pairs: the result is a pure
 //      function of the inputs, identical run to run and to a CPU sequential sum
 //      in stable-sorted order.
+// When the caller does not ask for the sorted pairs, the same sums are formed from the
+// voxels sorted by base cell (below), an eighth of the keys.
 // The reference sums with a parallel CUDPP segmented scan; the keys are the
 // bit-exact target, the sums match to rounding.
 #include <algorithm>
@@ -379,48 +381,118 @@ k_segment_sum(const unsigned *__restrict__ keys, const float *__restrict__ vals,
   }
 }
 
-size_t splat_sorted_scratch_bytes(int nx, int ny, int nz) {
-  const long long M = 8LL * nx * ny * nz;
-  const int ntiles = (int)((M + kTile - 1) / kTile);
-  const long long nh = 2LL * kRadix * ntiles;  // room for a 9-bit pass
-  const int nchunks = (int)((nh + kScanChunk - 1) / kScanChunk);
-  // two key/value buffers, histogram, chunk sums
-  return 2 * (size_t)M * 4 + 2 * (size_t)M * 4 + (size_t)nh * 4 + (size_t)nchunks * 4 + 256;
+// ---------------------------------------------------------------- by base cell
+// The sums without the sorted pairs.  All 8 pairs of a voxel follow from its base cell
+// (its lowest corner), so the N voxels are sorted by base cell instead of the 8N pairs
+// by cell: an eighth of the keys through every radix pass.  A cell's contributions, in
+// the order of the sorted pairs, are those of the four base cells at its own z, by
+// voxel number, then of the four one plane below, by voxel number; each base cell's
+// voxels are in that order already (the sort is stable), so a four-way merge adds
+// them one by one in exactly the sequence of the pairs.  The same bits.
+//
+// Bound by the passes over the voxels; 128^3: 479 -> 307 us.
+
+// Corner weights of a voxel at (x, y, z), as k_create_index forms them.
+__device__ __forceinline__ void base_corner(float x, float y, float z, int truncate, int &xi, int &yi, int &zi) {
+  xi = (int)x;
+  yi = (int)y;
+  zi = (int)z;
+  if (!truncate) {
+    if (x < 0.f && x != (float)xi) --xi;
+    if (y < 0.f && y != (float)yi) --yi;
+    if (z < 0.f && z != (float)zi) --zi;
+  }
 }
 
-awk_status launch_splat_sorted(float *dst, const float *src, const float *vx, const float *vy,
-                               const float *vz, int nx, int ny, int nz, int truncate,
-                               unsigned *keys_out, float *vals_out, hipStream_t s, int absolute,
-                               void *work) {
-  const long long N = (long long)nx * ny * nz;
-  const long long M = 8 * N;
-  int bits = 1;
-  while ((1LL << bits) < N + 1) ++bits;
+__device__ __forceinline__ float4 splat_source(int id, const float *__restrict__ src, const float *__restrict__ vx,
+                                               const float *__restrict__ vy, const float *__restrict__ vz, int w,
+                                               int h, int absolute) {
+  const int i = id % w, rest = id / w, j = rest % h, k = rest / h;
+  return make_float4(absolute ? vx[id] : (float)i + vx[id], absolute ? vy[id] : (float)j + vy[id],
+                     absolute ? vz[id] : (float)k + vz[id], src[id]);
+}
+
+// Base cells -1 .. n - 1 per axis, numbered from 0; `cells` for a voxel without a
+// corner in the volume.
+__global__ void __launch_bounds__(256)
+k_base_index(unsigned *__restrict__ keys, unsigned *__restrict__ ids, const float *__restrict__ src,
+             const float *__restrict__ vx, const float *__restrict__ vy, const float *__restrict__ vz, int w, int h,
+             int l, unsigned cells, int truncate, int absolute, uint2 *__restrict__ ranges) {
+  const int N = w * h * l;
+  const unsigned id = blockIdx.x * blockDim.x + threadIdx.x;
+  if (id < cells) ranges[id] = make_uint2(0u, 0u);
+  if (id >= (unsigned)N) return;
+  const float4 p = splat_source((int)id, src, vx, vy, vz, w, h, absolute);
+  int xi, yi, zi;
+  base_corner(p.x, p.y, p.z, truncate, xi, yi, zi);
+  const bool in = xi >= -1 && xi < w && yi >= -1 && yi < h && zi >= -1 && zi < l;
+  keys[id] = in ? ((unsigned)(zi + 1) * (h + 1) + (yi + 1)) * (w + 1) + (xi + 1) : cells;
+  ids[id] = id;
+}
+
+// Each base cell's run of the sorted voxels, and the voxels' positions and masses in
+// that order (the cells read them 8 times).
+__global__ void __launch_bounds__(256)
+k_base_runs(const unsigned *__restrict__ keys, const unsigned *__restrict__ ids, const float *__restrict__ src,
+            const float *__restrict__ vx, const float *__restrict__ vy, const float *__restrict__ vz, int w, int h,
+            int l, unsigned cells, int absolute, uint2 *__restrict__ ranges, float4 *__restrict__ pos) {
+  const unsigned N = (unsigned)(w * h * l), e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= N) return;
+  const unsigned k = keys[e];
+  if (k >= cells) return;
+  if (e == 0 || keys[e - 1] != k) ranges[k].x = e;
+  if (e + 1 == N || keys[e + 1] != k) ranges[k].y = e + 1;
+  pos[e] = splat_source((int)ids[e], src, vx, vy, vz, w, h, absolute);
+}
+
+__global__ void __launch_bounds__(256)
+k_base_sum(float *__restrict__ dst, const unsigned *__restrict__ ids, const float4 *__restrict__ pos,
+           const uint2 *__restrict__ ranges, int w, int h, int l, int truncate) {
+#pragma clang fp contract(off)  // each contribution is rounded before it is added, as a stored pair is
+  const int N = w * h * l, cell = (int)(xcd_block() * blockDim.x + threadIdx.x);
+  if (cell >= N) return;
+  const int X = cell % w, rest = cell / w, Y = rest % h, Z = rest / h;
+  constexpr unsigned kNone = 0xffffffffu;
+  uint2 run[8];
+#pragma unroll
+  for (int c = 0; c < 8; ++c)
+    run[c] = ranges[((unsigned)(Z + 1 - (c >> 2)) * (h + 1) + (Y + 1 - ((c >> 1) & 1))) * (w + 1) + (X + 1 - (c & 1))];
+  float acc = 0.f;
+#pragma unroll
+  for (int half = 0; half < 2; ++half) {
+    unsigned next[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) next[c] = run[4 * half + c].x < run[4 * half + c].y ? ids[run[4 * half + c].x] : kNone;
+    while (true) {
+      const unsigned m = min(min(next[0], next[1]), min(next[2], next[3]));
+      if (m == kNone) break;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        if (next[c] != m) continue;
+        uint2 &q = run[4 * half + c];
+        const float4 p = pos[q.x];
+        ++q.x;
+        next[c] = q.x < q.y ? ids[q.x] : kNone;
+        int xi, yi, zi;
+        base_corner(p.x, p.y, p.z, truncate, xi, yi, zi);
+        const float dx = 1.f - (p.x - xi), dy = 1.f - (p.y - yi), dz = 1.f - (p.z - zi);
+        const float wx = (c & 1) ? 1.f - dx : dx, wy = (c >> 1) ? 1.f - dy : dy, wz = half ? 1.f - dz : dz;
+        acc += p.w * wx * wy * wz;
+      }
+    }
+  }
+  dst[cell] = acc;
+}
+
+// Stable radix sort of M (key, value) pairs of `bits` key bits, between the two
+// buffer pairs; the sorted pairs are in (ka, va) on return.
+static awk_status radix_sort(unsigned *&ka, unsigned *&kb, float *&va, float *&vb, long long M, int bits,
+                             unsigned *hist, unsigned *sums, hipStream_t s) {
   // 8-bit passes; 9 remaining bits go in one pass (a power-of-two volume's keys,
   // cells 0 .. N - 1 and the outside-volume cell N, need one bit past a multiple of 8)
-  std::vector<int> plan;
-  for (int rem = bits; rem > 0;) {
-    const int b = rem == 9 ? 9 : std::min(rem, kRadixBits);
-    plan.push_back(b);
-    rem -= b;
-  }
   const int ntiles = (int)((M + kTile - 1) / kTile);
-  const long long nh_max = 2LL * kRadix * ntiles;
-  // scratch: the caller's work buffer (splat_sorted_scratch_bytes) or stream-ordered
-  char *scratch = static_cast<char *>(work);
-  if (!scratch) AWK_HIP(hipMallocAsync((void **)&scratch, splat_sorted_scratch_bytes(nx, ny, nz), s));
-  unsigned *ka = reinterpret_cast<unsigned *>(scratch);
-  unsigned *kb = ka + M;
-  float *va = reinterpret_cast<float *>(kb + M);
-  float *vb = va + M;
-  unsigned *hist = reinterpret_cast<unsigned *>(vb + M);
-  unsigned *sums = hist + nh_max;
-  AWK_LAUNCH(k_create_index, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s,
-             reinterpret_cast<uint4 *>(ka), reinterpret_cast<float4 *>(va), src, vx, vy, vz, nx, ny,
-             nz, truncate, absolute);
-  AWK_LAUNCH_CHECK("k_create_index");
-  int shift = 0;
-  for (const int b : plan) {
+  for (int rem = bits, shift = 0; rem > 0;) {
+    const int b = rem == 9 ? 9 : std::min(rem, kRadixBits);
     const long long nh = (long long)(b == 9 ? 2 * kRadix : kRadix) * ntiles;
     const int nchunks = (int)((nh + kScanChunk - 1) / kScanChunk);
     if (b == 9) AWK_LAUNCH(k_radix_hist<9>, dim3(ntiles), dim3(kSortBlock), 0, s, ka, M, shift, ntiles, hist);
@@ -436,15 +508,93 @@ awk_status launch_splat_sorted(float *dst, const float *src, const float *vx, co
                  ntiles, hist);
     AWK_LAUNCH_CHECK("radix pass");
     shift += b;
+    rem -= b;
     std::swap(ka, kb);
     std::swap(va, vb);
   }
+  return AWK_OK;
+}
+
+static int key_bits(long long most) {  // keys 0 .. most
+  int bits = 1;
+  while ((1LL << bits) < most + 1) ++bits;
+  return bits;
+}
+
+// Scratch of a sort of M pairs: two key / value buffers, histogram, chunk sums.
+struct SortScratch {
+  long long M, nh, nchunks;
+  explicit SortScratch(long long m) : M(m) {
+    nh = 2LL * kRadix * ((M + kTile - 1) / kTile);  // room for a 9-bit pass
+    nchunks = (nh + kScanChunk - 1) / kScanChunk;
+  }
+  size_t bytes() const { return (16 * (size_t)M + 4 * (size_t)nh + 4 * (size_t)nchunks + 255) / 256 * 256; }
+};
+
+static long long base_cells(int nx, int ny, int nz) { return (long long)(nx + 1) * (ny + 1) * (nz + 1); }
+
+size_t splat_sorted_scratch_bytes(int nx, int ny, int nz) {
+  const long long N = (long long)nx * ny * nz;
+  return SortScratch(N).bytes() + 16 * (size_t)N + 8 * (size_t)base_cells(nx, ny, nz);
+}
+
+// The sorted pairs themselves are wanted: all 8N of them are made and sorted.
+static awk_status splat_pairs(float *dst, const float *src, const float *vx, const float *vy, const float *vz, int nx,
+                              int ny, int nz, int truncate, unsigned *keys_out, float *vals_out, hipStream_t s,
+                              int absolute) {
+  const long long N = (long long)nx * ny * nz;
+  const long long M = 8 * N;
+  const SortScratch sc(M);
+  char *scratch = nullptr;
+  AWK_HIP(hipMallocAsync((void **)&scratch, sc.bytes(), s));
+  unsigned *ka = reinterpret_cast<unsigned *>(scratch);
+  unsigned *kb = ka + M;
+  float *va = reinterpret_cast<float *>(kb + M);
+  float *vb = va + M;
+  unsigned *hist = reinterpret_cast<unsigned *>(vb + M);
+  AWK_LAUNCH(k_create_index, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s,
+             reinterpret_cast<uint4 *>(ka), reinterpret_cast<float4 *>(va), src, vx, vy, vz, nx, ny,
+             nz, truncate, absolute);
+  AWK_LAUNCH_CHECK("k_create_index");
+  if (awk_status st = radix_sort(ka, kb, va, vb, M, key_bits(N), hist, hist + sc.nh, s)) return st;
   AWK_LAUNCH(k_zero_image, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, dst, N);
   AWK_LAUNCH(k_segment_sum, dim3((unsigned)((M + kSegTile - 1) / kSegTile)), dim3(256), 0, s, ka, va, M,
              (unsigned)N, dst);
   AWK_LAUNCH_CHECK("k_segment_sum");
   if (keys_out) AWK_HIP(hipMemcpyAsync(keys_out, ka, (size_t)M * 4, hipMemcpyDeviceToDevice, s));
   if (vals_out) AWK_HIP(hipMemcpyAsync(vals_out, va, (size_t)M * 4, hipMemcpyDeviceToDevice, s));
+  AWK_HIP(hipFreeAsync(scratch, s));
+  return AWK_OK;
+}
+
+awk_status launch_splat_sorted(float *dst, const float *src, const float *vx, const float *vy,
+                               const float *vz, int nx, int ny, int nz, int truncate,
+                               unsigned *keys_out, float *vals_out, hipStream_t s, int absolute,
+                               void *work) {
+  if (keys_out || vals_out)
+    return splat_pairs(dst, src, vx, vy, vz, nx, ny, nz, truncate, keys_out, vals_out, s, absolute);
+  const long long N = (long long)nx * ny * nz, cells = base_cells(nx, ny, nz);
+  const SortScratch sc(N);
+  // scratch: the caller's work buffer (splat_sorted_scratch_bytes) or stream-ordered
+  char *scratch = static_cast<char *>(work);
+  if (!scratch) AWK_HIP(hipMallocAsync((void **)&scratch, splat_sorted_scratch_bytes(nx, ny, nz), s));
+  float4 *pos = reinterpret_cast<float4 *>(scratch);
+  uint2 *ranges = reinterpret_cast<uint2 *>(pos + N);
+  unsigned *ka = reinterpret_cast<unsigned *>(ranges + cells);
+  unsigned *kb = ka + N;
+  float *va = reinterpret_cast<float *>(kb + N);  // voxel numbers: moved as bits
+  float *vb = va + N;
+  unsigned *hist = reinterpret_cast<unsigned *>(vb + N);
+  const unsigned gN = (unsigned)((N + 255) / 256), gc = (unsigned)((cells + 255) / 256);
+  AWK_LAUNCH(k_base_index, dim3(gc), dim3(256), 0, s, ka, reinterpret_cast<unsigned *>(va), src, vx, vy, vz, nx, ny,
+             nz, (unsigned)cells, truncate, absolute, ranges);
+  AWK_LAUNCH_CHECK("k_base_index");
+  if (awk_status st = radix_sort(ka, kb, va, vb, N, key_bits(cells), hist, hist + sc.nh, s)) return st;
+  AWK_LAUNCH(k_base_runs, dim3(gN), dim3(256), 0, s, ka, reinterpret_cast<unsigned *>(va), src, vx, vy, vz, nx, ny,
+             nz, (unsigned)cells, absolute, ranges, pos);
+  AWK_LAUNCH(k_base_sum, dim3(grid_for(N, 256)), dim3(256), 0, s, dst, reinterpret_cast<unsigned *>(va), pos, ranges,
+             nx, ny, nz, truncate);
+  AWK_LAUNCH_CHECK("k_base_sum");
   if (!work) AWK_HIP(hipFreeAsync(scratch, s));
   return AWK_OK;
 }

@@ -444,7 +444,7 @@ awk_status awk_ldmm_set_gradient(awk_ldmm_t l, int use_orig);
  * 185-247, made order-independent; the default), 1 = the sort/scan splat
  * (cplSplating, cudaSplat.cu:175-238: createIndex keys, stable radix sort,
  * sequential segment sums; positions floored as the atomic splat does).  Both are
- * deterministic.  Mode 1 allocates its scratch here (about 130 bytes per voxel). */
+ * deterministic.  Mode 1 allocates its scratch here (about 40 bytes per voxel). */
 awk_status awk_ldmm_set_splat(awk_ldmm_t l, int mode);
 /* LDMMIteratorGPU::UpdateStepSizeNextIteration: the next iterate only sets the step. */
 awk_status awk_ldmm_update_step_next(awk_ldmm_t l);

@@ -216,3 +216,39 @@ def test_splat_tiled_equals_direct(shape, amp):
         np.testing.assert_array_equal(host(out), direct)
     finally:
         set_knob("splat_tile", old)
+
+
+@pytest.mark.parametrize("kind", ["one_cell", "spread", "outside", "edges", "nonfinite"])
+@pytest.mark.parametrize("trunc", [True, False])
+def test_splat_sorted_without_pairs_bit_exact(kind, trunc):
+    """The sums from the voxels sorted by base cell (no pairs asked for) against the
+    sums over the sorted pairs: the same bits, with every voxel in one cell, spread
+    over the volume and past it, all outside, within a voxel of the faces, and with
+    infinite and NaN displacements."""
+    import torch
+    shape = (19, 21, 23)
+    nz, ny, nx = shape
+    print("splat_sorted base", kind, trunc, flush=True)
+    rng = np.random.default_rng(5)
+    src = rng.standard_normal(shape).astype(np.float32)
+    ident = synth.identity(shape)
+    v = np.zeros((3,) + shape, np.float32)
+    if kind == "one_cell":
+        v = (np.array([7.25, 9.5, 3.125], np.float32)[:, None, None, None] - ident).astype(np.float32)
+    elif kind == "spread":
+        v = rng.uniform(-30, 30, v.shape).astype(np.float32)
+    elif kind == "outside":
+        v[:] = 1000.0
+    elif kind == "edges":
+        to = rng.uniform(-1.5, 0.5, v.shape) + np.where(rng.random(v.shape) < 0.5, 0, 1) * (np.array([nx, ny, nz]) + 0.5)[:, None, None, None]
+        v = (to - ident).astype(np.float32)
+    else:
+        v = rng.uniform(-2, 2, v.shape).astype(np.float32)
+        v[:, 3, 4, 5], v[:, 6, 7, 8], v[1, 2, 2, 2] = np.inf, -np.inf, np.nan
+    S, V = torch.from_numpy(src).cuda(), torch.from_numpy(np.ascontiguousarray(v)).cuda()
+    keys = torch.empty(8 * src.size, dtype=torch.int32, device="cuda")
+    vals = torch.empty(8 * src.size, dtype=torch.float32, device="cuda")
+    a, b = torch.full_like(S, 7.0), torch.full_like(S, -3.0)
+    hfield.splat_sorted(a, S, V, reference_truncation=trunc, keys=keys, vals=vals)
+    hfield.splat_sorted(b, S, V, reference_truncation=trunc)
+    np.testing.assert_array_equal(a.cpu().numpy(), b.cpu().numpy())
