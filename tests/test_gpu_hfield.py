@@ -226,6 +226,7 @@ def test_splat_sorted_without_pairs_bit_exact(kind, trunc):
     over the volume and past it, all outside, within a voxel of the faces, and with
     infinite and NaN displacements."""
     import torch
+    from atlaswerks_amd import hfield
     shape = (19, 21, 23)
     nz, ny, nx = shape
     print("splat_sorted base", kind, trunc, flush=True)
