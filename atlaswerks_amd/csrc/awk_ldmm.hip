@@ -103,7 +103,7 @@ k_ldmm_bwd(float *__restrict__ nx_, float *__restrict__ ny_, float *__restrict__
   const int N = d.nx * d.ny * d.nz;
   SplatPosLdmm p{hx, hy, hz, make_buf(vx, N), make_buf(vy, N), make_buf(vz, N), d, sx, sy, sz,
                  nx_, ny_, nz_};
-  splat_tile<SplatShapeLdmm>(p, diff, acc, d);
+  splat_tile<SplatShape16>(p, diff, acc, d);
 }
 
 // composeVHInv(v_t, h, PARTIAL_ZERO) alone, for the sort/scan splat: the same
@@ -583,7 +583,7 @@ awk_status awk::ldmm_new_iterate(awk_ldmm *l, const float *I0, const float *I1, 
                                     nullptr, s, 1, l->sort_work)))
         return st;
     } else {
-      AWK_LAUNCH(k_ldmm_bwd, dim3(splat_tile_grid<SplatShapeLdmm>(nx, ny, nz)), dim3(kSplatTileThreads), 0, s, hs,
+      AWK_LAUNCH(k_ldmm_bwd, dim3(splat_tile_grid<SplatShape16>(nx, ny, nz)), dim3(kSplatTileThreads), 0, s, hs,
                  hs + N, hs + 2 * N, h, h + N, h + 2 * N, v[3 * t], v[3 * t + 1], v[3 * t + 2],
                  l->diff, reinterpret_cast<unsigned long long *>(l->acc), d, sx, sy, sz);
       AWK_LAUNCH_CHECK("k_ldmm_bwd");

@@ -58,7 +58,7 @@ __global__ void __launch_bounds__(kSplatTileThreads)
 k_splat_tiled(unsigned long long *__restrict__ acc, const float *__restrict__ src,
               const float *__restrict__ hx, const float *__restrict__ hy,
               const float *__restrict__ hz, Dims d) {
-  splat_tile<SplatShapeEntry>(SplatPosH{hx, hy, hz}, src, acc, d);
+  splat_tile<SplatShape16>(SplatPosH{hx, hy, hz}, src, acc, d);
 }
 
 template <class T>
@@ -67,12 +67,13 @@ __global__ void k_fill(T *__restrict__ p, long long n, T v) {
   if (i < n) p[i] = v;
 }
 
-// dst = acc * 2^-32 in float; the accumulator is left cleared for its next use.
+// dst = acc * 2^-32 in float; CLEAR: the accumulator is left cleared for its next use.
+template <bool CLEAR>
 __global__ void k_fixed64_to_float(float *__restrict__ dst, long long *__restrict__ acc, int N) {
   const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   if (i >= N) return;
   const long long q = acc[i];
-  acc[i] = 0;
+  if (CLEAR) acc[i] = 0;
   dst[i] = splat_unq(q);
 }
 
@@ -95,17 +96,20 @@ awk_status clear_splat_acc(unsigned long long *acc, long long n, hipStream_t s) 
 
 awk_status launch_splat_acc(float *dst, const float *src, const float *hx, const float *hy,
                             const float *hz, int nx, int ny, int nz, unsigned long long *acc,
-                            hipStream_t s) {
+                            bool clear, hipStream_t s) {
   const long long N = (long long)nx * ny * nz;
   if (tuning().splat_tile)
-    AWK_LAUNCH(k_splat_tiled, dim3(splat_tile_grid<SplatShapeEntry>(nx, ny, nz)),
+    AWK_LAUNCH(k_splat_tiled, dim3(splat_tile_grid<SplatShape16>(nx, ny, nz)),
                dim3(kSplatTileThreads), 0, s, acc, src, hx, hy, hz, Dims{nx, ny, nz});
   else
     AWK_LAUNCH(k_splat<AWK_SPLAT_FIXED64>, dim3(grid_for(N, kSplatBlock)), dim3(kSplatBlock), 0,
                s, (void *)acc, src, hx, hy, hz, nx, ny, nz);
   AWK_LAUNCH_CHECK("k_splat<FIXED64>");
-  AWK_LAUNCH(k_fixed64_to_float, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, dst,
-             reinterpret_cast<long long *>(acc), (int)N);
+  const dim3 cgrid((unsigned)((N + 255) / 256));
+  if (clear)
+    AWK_LAUNCH(k_fixed64_to_float<true>, cgrid, dim3(256), 0, s, dst, reinterpret_cast<long long *>(acc), (int)N);
+  else
+    AWK_LAUNCH(k_fixed64_to_float<false>, cgrid, dim3(256), 0, s, dst, reinterpret_cast<long long *>(acc), (int)N);
   AWK_LAUNCH_CHECK("k_fixed64_to_float");
   return AWK_OK;
 }
@@ -123,7 +127,7 @@ awk_status launch_splat(float *dst, const float *src, const float *hx, const flo
     awk_status st = clear_splat_acc(reinterpret_cast<unsigned long long *>(acc), N, s);
     if (st == AWK_OK)
       st = launch_splat_acc(dst, src, hx, hy, hz, nx, ny, nz,
-                            reinterpret_cast<unsigned long long *>(acc), s);
+                            reinterpret_cast<unsigned long long *>(acc), false, s);
     hipError_t e = hipFreeAsync(acc, s);
     if (st != AWK_OK) return st;
     AWK_HIP(e);
@@ -212,7 +216,7 @@ extern "C" awk_status awk_splat_noalloc(float *dst, const float *src, const floa
   int dev = -1;
   awk_status st = noalloc_scratch(s, &acc, &dev);
   if (st != AWK_OK) return st;
-  st = launch_splat_acc(dst, src, hx, hy, hz, nx, ny, nz, acc, s);
+  st = launch_splat_acc(dst, src, hx, hy, hz, nx, ny, nz, acc, true, s);
   if (st != AWK_OK) {
     std::lock_guard<std::mutex> lock(g_scratch_mu);
     g_scratch_dirty[dev] = true;

@@ -8,8 +8,8 @@
 // direct kernel) with LDS atomics and one flush adds the non-zero window cells to
 // the global accumulator; otherwise pass B adds straight to global memory.
 // Integer sums commute, so the result is bit-identical to the direct splat for
-// any tiling or scheduling.  Each thread handles the same voxels in both passes,
-// so a position it stored in pass A is read back by the same thread.
+// any tiling or scheduling.  Each thread handles the same few voxels in both passes
+// and keeps their positions and masses in registers between them.
 //
 // Tile shapes: a tile's footprint is the tile itself widened by the variation of
 // the displacement across it.  For smooth fields of up to 8 voxels at 256^3 a
@@ -34,10 +34,10 @@ struct SplatShape {
   static_assert(TX * TY * TZ % kSplatTileThreads == 0, "tile must be a multiple of the block");
   static_assert((TX & (TX - 1)) == 0 && (TY & (TY - 1)) == 0, "power-of-two tile rows");
 };
-// the splat entry points (1,024 voxels, 32 KiB window: five blocks per CU)
-using SplatShapeEntry = SplatShape<16, 8, 8, 4096>;
-// the LDMM backward sweep (4,096 voxels, 56 KiB window), as measured there
-using SplatShapeLdmm = SplatShape<64, 8, 8, 7168>;
+// 1,024 voxels, 32 KiB window: five blocks per CU.  The LDMM backward sweep had tiles of
+// 64 x 8 x 8 with a 56 KiB window, 160 blocks for a 96 x 80 x 64 grid:
+// 51 us per step there, {LDMM} with these.
+using SplatShape16 = SplatShape<16, 8, 8, 4096>;
 
 template <class S>
 inline unsigned splat_tile_grid(int nx, int ny, int nz) {
@@ -48,19 +48,18 @@ inline unsigned splat_tile_grid(int nx, int ny, int nz) {
 // Positions given by an hfield.
 struct SplatPosH {
   const float *hx, *hy, *hz;
-  __device__ __forceinline__ float3 first(int i) const { return make_float3(hx[i], hy[i], hz[i]); }
-  __device__ __forceinline__ float3 again(int i) const { return make_float3(hx[i], hy[i], hz[i]); }
+  __device__ __forceinline__ float3 at(int i) const { return make_float3(hx[i], hy[i], hz[i]); }
 };
 
-// LDMM backward step: h' = h - v(h)/sp (composeVHInv, PARTIAL_ZERO), stored to
-// (ox, oy, oz) in pass A and read back by the same thread in pass B.
+// LDMM backward step: h' = h - v(h)/sp (composeVHInv, PARTIAL_ZERO), also stored to
+// (ox, oy, oz) for the next step.
 struct SplatPosLdmm {
   const float *gx, *gy, *gz;
   BufLoad vx, vy, vz;
   Dims d;
   float sx, sy, sz;
   float *ox, *oy, *oz;
-  __device__ __forceinline__ float3 first(int i) const {
+  __device__ __forceinline__ float3 at(int i) const {
     const float a = gx[i], b = gy[i], c = gz[i];
     const float3 o = trilerp3g<AWK_BG_PARTIAL_ZERO>(vx, vy, vz, d, a, b, c);
     const float x = o.x / -sx + a, y = o.y / -sy + b, z = o.z / -sz + c;
@@ -69,7 +68,6 @@ struct SplatPosLdmm {
     oz[i] = z;
     return make_float3(x, y, z);
   }
-  __device__ __forceinline__ float3 again(int i) const { return make_float3(ox[i], oy[i], oz[i]); }
 };
 
 __device__ __forceinline__ int wave_min(int v) {
@@ -96,14 +94,24 @@ __device__ void splat_tile(const P &pos, const float *__restrict__ mass,
   const int x0 = (b % ntx) * kSTX, y0 = ((b / ntx) % nty) * kSTY, z0 = (b / (ntx * nty)) * kSTZ;
   const int t = (int)threadIdx.x;
   int mn[3] = {INT_MAX, INT_MAX, INT_MAX}, mx[3] = {INT_MIN, INT_MIN, INT_MIN};
-  // pass A: destinations and their bounding box
-#pragma unroll 4
+  // pass A: destinations (kept in registers, with the masses) and their bounding box
+  float3 p[kSplatTileVPT];
+  float m[kSplatTileVPT];
+  bool live[kSplatTileVPT];
+#pragma unroll
   for (int v = 0; v < kSplatTileVPT; ++v) {
     const int lin = v * kSplatTileThreads + t;
     const int x = x0 + (lin & (kSTX - 1)), y = y0 + ((lin / kSTX) & (kSTY - 1)), z = z0 + lin / (kSTX * kSTY);
-    if (x >= d.nx || y >= d.ny || z >= d.nz) continue;
-    const float3 p = pos.first((z * d.ny + y) * d.nx + x);
-    const int xi = (int)floorf(p.x), yi = (int)floorf(p.y), zi = (int)floorf(p.z);
+    live[v] = x < d.nx && y < d.ny && z < d.nz;
+    if (!live[v]) continue;
+    const int i = (z * d.ny + y) * d.nx + x;
+    p[v] = pos.at(i);
+    m[v] = mass[i];
+  }
+#pragma unroll
+  for (int v = 0; v < kSplatTileVPT; ++v) {
+    if (!live[v]) continue;
+    const int xi = (int)floorf(p[v].x), yi = (int)floorf(p[v].y), zi = (int)floorf(p[v].z);
     mn[0] = min(mn[0], xi); mx[0] = max(mx[0], xi);
     mn[1] = min(mn[1], yi); mx[1] = max(mx[1], yi);
     mn[2] = min(mn[2], zi); mx[2] = max(mx[2], zi);
@@ -143,24 +151,19 @@ __device__ void splat_tile(const P &pos, const float *__restrict__ mass,
     __syncthreads();
   }
   // pass B: contributions
-#pragma unroll 2
+#pragma unroll
   for (int v = 0; v < kSplatTileVPT; ++v) {
-    const int lin = v * kSplatTileThreads + t;
-    const int x = x0 + (lin & (kSTX - 1)), y = y0 + ((lin / kSTX) & (kSTY - 1)), z = z0 + lin / (kSTX * kSTY);
-    if (x >= d.nx || y >= d.ny || z >= d.nz) continue;
-    const int i = (z * d.ny + y) * d.nx + x;
-    const float3 p = pos.again(i);
-    const float m = mass[i];
-    const float fx = floorf(p.x), fy = floorf(p.y), fz = floorf(p.z);
+    if (!live[v]) continue;
+    const float fx = floorf(p[v].x), fy = floorf(p[v].y), fz = floorf(p[v].z);
     const int xi = (int)fx, yi = (int)fy, zi = (int)fz;
-    const float dx = 1.f - (p.x - fx), dy = 1.f - (p.y - fy), dz = 1.f - (p.z - fz);
+    const float dx = 1.f - (p[v].x - fx), dy = 1.f - (p[v].y - fy), dz = 1.f - (p[v].z - fz);
     const float wx[2] = {dx, 1.f - dx}, wy[2] = {dy, 1.f - dy}, wz[2] = {dz, 1.f - dz};
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
       const int ox = c & 1, oy = (c >> 1) & 1, oz = c >> 2;
       const int X = xi + ox, Y = yi + oy, Z = zi + oz;
       if (X < 0 || X >= d.nx || Y < 0 || Y >= d.ny || Z < 0 || Z >= d.nz) continue;
-      const unsigned long long q = splat_q(m * wx[ox] * wy[oy] * wz[oz]);
+      const unsigned long long q = splat_q(m[v] * wx[ox] * wy[oy] * wz[oz]);
       if (use_lds)
         atomicAdd(&win[((Z - lo[2]) * W[1] + (Y - lo[1])) * W[0] + (X - lo[0])], q);
       else
