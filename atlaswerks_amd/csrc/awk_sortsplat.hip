@@ -392,7 +392,7 @@ k_segment_sum(const unsigned *__restrict__ keys, const float *__restrict__ vals,
 //
 // Bound by the passes over the voxels; 128^3: 479 -> 307 us.
 
-// Corner weights of a voxel at (x, y, z), as k_create_index forms them.
+// The base cell of a voxel at (x, y, z), as k_create_index forms it.
 __device__ __forceinline__ void base_corner(float x, float y, float z, int truncate, int &xi, int &yi, int &zi) {
   xi = (int)x;
   yi = (int)y;
@@ -430,58 +430,130 @@ k_base_index(unsigned *__restrict__ keys, unsigned *__restrict__ ids, const floa
   ids[id] = id;
 }
 
-// Each base cell's run of the sorted voxels, and the voxels' positions and masses in
-// that order (the cells read them 8 times).
+// Each base cell's run of the sorted voxels, and the voxels' low-corner weights and
+// masses in that order (the cells read them 8 times).
 __global__ void __launch_bounds__(256)
 k_base_runs(const unsigned *__restrict__ keys, const unsigned *__restrict__ ids, const float *__restrict__ src,
             const float *__restrict__ vx, const float *__restrict__ vy, const float *__restrict__ vz, int w, int h,
-            int l, unsigned cells, int absolute, uint2 *__restrict__ ranges, float4 *__restrict__ pos) {
+            int l, unsigned cells, int truncate, int absolute, uint2 *__restrict__ ranges,
+            float4 *__restrict__ pos) {
   const unsigned N = (unsigned)(w * h * l), e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= N) return;
   const unsigned k = keys[e];
   if (k >= cells) return;
   if (e == 0 || keys[e - 1] != k) ranges[k].x = e;
   if (e + 1 == N || keys[e + 1] != k) ranges[k].y = e + 1;
-  pos[e] = splat_source((int)ids[e], src, vx, vy, vz, w, h, absolute);
+  const float4 p = splat_source((int)ids[e], src, vx, vy, vz, w, h, absolute);
+  int xi, yi, zi;
+  base_corner(p.x, p.y, p.z, truncate, xi, yi, zi);
+  pos[e] = make_float4(1.f - (p.x - xi), 1.f - (p.y - yi), 1.f - (p.z - zi), p.w);
 }
 
-__global__ void __launch_bounds__(256)
+// One block per 128 cells of a row.  The runs of the row's base cells are four
+// consecutive stretches of the sorted voxels (its own row and the three before it in y
+// and z), staged in LDS with coalesced loads when they fit: the merge's loads depend
+// on each other (128^3: 134 us from memory, {SUM} staged).
+constexpr int kSumBlock = 128, kSumCap = 6 * kSumBlock;
+__global__ void __launch_bounds__(kSumBlock)
 k_base_sum(float *__restrict__ dst, const unsigned *__restrict__ ids, const float4 *__restrict__ pos,
-           const uint2 *__restrict__ ranges, int w, int h, int l, int truncate) {
+           const uint2 *__restrict__ ranges, int w, int h, int l) {
 #pragma clang fp contract(off)  // each contribution is rounded before it is added, as a stored pair is
-  const int N = w * h * l, cell = (int)(xcd_block() * blockDim.x + threadIdx.x);
-  if (cell >= N) return;
-  const int X = cell % w, rest = cell / w, Y = rest % h, Z = rest / h;
   constexpr unsigned kNone = 0xffffffffu;
-  uint2 run[8];
+  __shared__ unsigned lo[4], hi[4], sid[kSumCap];
+  __shared__ float4 spos[kSumCap];
+  const int nseg = (w + kSumBlock - 1) / kSumBlock;
+  const int b = (int)xcd_block();
+  if (b >= h * l * nseg) return;
+  const int row = b / nseg, Y = row % h, Z = row / h;
+  const int X = (b - row * nseg) * kSumBlock + (int)threadIdx.x, lane = threadIdx.x & 63;
+  if (threadIdx.x < 4) {
+    lo[threadIdx.x] = kNone;
+    hi[threadIdx.x] = 0u;
+  }
+  uint2 run[8];  // corner c = 4 (z below) + 2 (y below) + (x below)
 #pragma unroll
   for (int c = 0; c < 8; ++c)
-    run[c] = ranges[((unsigned)(Z + 1 - (c >> 2)) * (h + 1) + (Y + 1 - ((c >> 1) & 1))) * (w + 1) + (X + 1 - (c & 1))];
-  float acc = 0.f;
+    run[c] = X < w ? ranges[((unsigned)(Z + 1 - (c >> 2)) * (h + 1) + (Y + 1 - ((c >> 1) & 1))) * (w + 1) +
+                            (X + 1 - (c & 1))]
+                   : make_uint2(0u, 0u);
+  __syncthreads();
 #pragma unroll
-  for (int half = 0; half < 2; ++half) {
-    unsigned next[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) next[c] = run[4 * half + c].x < run[4 * half + c].y ? ids[run[4 * half + c].x] : kNone;
-    while (true) {
-      const unsigned m = min(min(next[0], next[1]), min(next[2], next[3]));
-      if (m == kNone) break;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        if (next[c] != m) continue;
-        uint2 &q = run[4 * half + c];
-        const float4 p = pos[q.x];
-        ++q.x;
-        next[c] = q.x < q.y ? ids[q.x] : kNone;
-        int xi, yi, zi;
-        base_corner(p.x, p.y, p.z, truncate, xi, yi, zi);
-        const float dx = 1.f - (p.x - xi), dy = 1.f - (p.y - yi), dz = 1.f - (p.z - zi);
-        const float wx = (c & 1) ? 1.f - dx : dx, wy = (c >> 1) ? 1.f - dy : dy, wz = half ? 1.f - dz : dz;
-        acc += p.w * wx * wy * wz;
+  for (int r = 0; r < 4; ++r) {
+    // runs ascend with x: the stretch is from the first lane's first voxel to the last's last
+    const bool n1 = run[2 * r + 1].x < run[2 * r + 1].y, n0 = run[2 * r].x < run[2 * r].y;
+    const unsigned f = n1 ? run[2 * r + 1].x : run[2 * r].x, e = n0 ? run[2 * r].y : run[2 * r + 1].y;
+    const unsigned long long any = __ballot(n0 || n1);
+    if (any) {
+      const unsigned fw = __builtin_amdgcn_readlane(f, __builtin_ctzll(any));
+      const unsigned ew = __builtin_amdgcn_readlane(e, 63 - __builtin_clzll(any));
+      if (lane == 0) {
+        atomicMin(&lo[r], fw);
+        atomicMax(&hi[r], ew);
       }
     }
   }
-  dst[cell] = acc;
+  __syncthreads();
+  unsigned shift[4], total = 0;  // sorted index + shift = staged index
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const unsigned n = hi[r] > lo[r] ? hi[r] - lo[r] : 0u;
+    shift[r] = total - (n ? lo[r] : 0u);
+    total += n;
+  }
+  const bool staged = total <= (unsigned)kSumCap;
+  if (staged) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      for (unsigned e = lo[r] + threadIdx.x; e < hi[r]; e += kSumBlock) {
+        sid[e + shift[r]] = ids[e];
+        spos[e + shift[r]] = pos[e];
+      }
+    __syncthreads();
+  }
+  if (X >= w) return;
+  auto merge = [&](const unsigned *id, const float4 *at, bool moved) {
+    float acc = 0.f;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      unsigned next[4];
+      uint2 q[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        q[c] = run[4 * half + c];
+        if (moved) {
+          q[c].x += shift[2 * half + (c >> 1)];
+          q[c].y += shift[2 * half + (c >> 1)];
+        }
+        next[c] = q[c].x != q[c].y ? id[q[c].x] : kNone;
+      }
+      while (true) {
+        const unsigned m = min(min(next[0], next[1]), min(next[2], next[3]));
+        if (m == kNone) break;
+        // the run that m heads, by selects: a branch per run costs a wave all four
+        int c = 3;
+        unsigned i = q[3].x, e = q[3].y;
+#pragma unroll
+        for (int k = 2; k >= 0; --k) {
+          const bool is = next[k] == m;
+          c = is ? k : c;
+          i = is ? q[k].x : i;
+          e = is ? q[k].y : e;
+        }
+        const float4 p = at[i];
+        ++i;
+        const unsigned after = i != e ? id[i] : kNone;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          q[k].x = c == k ? i : q[k].x;
+          next[k] = c == k ? after : next[k];
+        }
+        const float wx = (c & 1) ? 1.f - p.x : p.x, wy = (c >> 1) ? 1.f - p.y : p.y, wz = half ? 1.f - p.z : p.z;
+        acc += p.w * wx * wy * wz;
+      }
+    }
+    return acc;
+  };
+  dst[((size_t)Z * h + Y) * w + X] = staged ? merge(sid, spos, true) : merge(ids, pos, false);
 }
 
 // Stable radix sort of M (key, value) pairs of `bits` key bits, between the two
@@ -591,9 +663,9 @@ awk_status launch_splat_sorted(float *dst, const float *src, const float *vx, co
   AWK_LAUNCH_CHECK("k_base_index");
   if (awk_status st = radix_sort(ka, kb, va, vb, N, key_bits(cells), hist, hist + sc.nh, s)) return st;
   AWK_LAUNCH(k_base_runs, dim3(gN), dim3(256), 0, s, ka, reinterpret_cast<unsigned *>(va), src, vx, vy, vz, nx, ny,
-             nz, (unsigned)cells, absolute, ranges, pos);
-  AWK_LAUNCH(k_base_sum, dim3(grid_for(N, 256)), dim3(256), 0, s, dst, reinterpret_cast<unsigned *>(va), pos, ranges,
-             nx, ny, nz, truncate);
+             nz, (unsigned)cells, truncate, absolute, ranges, pos);
+  AWK_LAUNCH(k_base_sum, dim3(grid_for((long long)ny * nz * ((nx + kSumBlock - 1) / kSumBlock), 1)), dim3(kSumBlock), 0, s, dst, reinterpret_cast<unsigned *>(va), pos, ranges,
+             nx, ny, nz);
   AWK_LAUNCH_CHECK("k_base_sum");
   if (!work) AWK_HIP(hipFreeAsync(scratch, s));
   return AWK_OK;
