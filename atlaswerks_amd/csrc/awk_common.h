@@ -87,6 +87,21 @@ inline hipError_t load_scalar_sync(T *host, const T *dev, hipStream_t s) {
   return e;
 }
 
+// Device memory kept between handles, and stream-ordered scratch of one call
+// (awk_mem.hip).  dev_free waits for the device and takes null pointers.
+hipError_t dev_alloc_bytes(void **p, size_t bytes);
+template <class T>
+inline hipError_t dev_alloc(T **p, size_t bytes) {
+  return dev_alloc_bytes(reinterpret_cast<void **>(p), bytes);
+}
+void dev_free(void *const *blocks, int n);
+hipError_t scratch_alloc_bytes(void **p, size_t bytes, hipStream_t s);
+template <class T>
+inline hipError_t scratch_alloc(T **p, size_t bytes, hipStream_t s) {
+  return scratch_alloc_bytes(reinterpret_cast<void **>(p), bytes, s);
+}
+hipError_t scratch_free(void *p, hipStream_t s);
+
 // Kernel-attached timing events: while set, launches go through
 // hipExtLaunchKernelGGL with these start/stop events, which the dispatch itself
 // timestamps (kernel duration only, the figure rocprof reports).

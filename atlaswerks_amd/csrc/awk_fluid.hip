@@ -489,9 +489,9 @@ awk_status fk_init(FluidKernel &k, int nx, int ny, int nz, const float sp[3]) {
     }
   }
   const size_t spec_bytes = 3 * k.spec_plane() * sizeof(float2);
-  AWK_HIP(hipMalloc(&k.spec, spec_bytes));
+  AWK_HIP(dev_alloc(&k.spec, spec_bytes));
   float2 *twd = nullptr;
-  AWK_HIP(hipMalloc(&twd, ntw * sizeof(float2)));
+  AWK_HIP(dev_alloc(&twd, ntw * sizeof(float2)));
   AWK_HIP(hipMemcpy(twd, tw.data(), ntw * sizeof(float2), hipMemcpyHostToDevice));
   k.ax[0].tw = twd;
   k.ax[1].tw = twd + nx;
@@ -505,17 +505,15 @@ awk_status fk_init(FluidKernel &k, int nx, int ny, int nz, const float sp[3]) {
     }
   for (int i = 0; i < 3; ++i)
     if (k.ax[i].dense.tiles) k.ax[i].dense.tab = twd + doff[i];
-  AWK_HIP(hipMalloc(&k.lut, nlut * sizeof(float)));
+  AWK_HIP(dev_alloc(&k.lut, nlut * sizeof(float)));
   AWK_HIP(hipMemcpy(k.lut, lut.data(), nlut * sizeof(float), hipMemcpyHostToDevice));
   k.scratch_bytes = spec_bytes + ntw * sizeof(float2) + nlut * sizeof(float);
   return AWK_OK;
 }
 
 void fk_release(FluidKernel &k) {
-  if (k.spec) (void)hipFree(k.spec);
-  if (k.ax[0].tw) (void)hipFree(k.ax[0].tw);
-  if (k.lut) (void)hipFree(k.lut);
-  if (k.eig) (void)hipFree(k.eig);
+  void *const blocks[] = {k.spec, const_cast<float2 *>(k.ax[0].tw), k.lut, k.eig};
+  dev_free(blocks, 4);
   k.spec = nullptr;
   k.ax[0].tw = k.ax[1].tw = k.ax[2].tw = nullptr;
   k.lut = nullptr;
@@ -526,7 +524,7 @@ awk_status fk_prepare_eigen(FluidKernel &k, int dir, hipStream_t s) {
   if (k.eig && k.eig_dir == dir) return AWK_OK;
   const size_t nf = (size_t)k.nxh * k.ny * k.nz;
   if (!k.eig) {
-    AWK_HIP(hipMalloc(&k.eig, nf * 6 * sizeof(float)));
+    AWK_HIP(dev_alloc(&k.eig, nf * 6 * sizeof(float)));
     k.scratch_bytes += nf * 6 * sizeof(float);
   }
   const double p = dir > 0 ? (double)k.lpow : -(double)k.lpow;

@@ -97,15 +97,8 @@ static void greedy_free(awk_greedy *g) {
   g->ev.clear();
   g->ev_mask.clear();
   fk_release(g->k);
-  if (g->idef) (void)hipFree(g->idef);
-  if (g->v) (void)hipFree(g->v);
-  if (g->hbuf) (void)hipFree(g->hbuf);
-  if (g->partials) (void)hipFree(g->partials);
-  if (g->maxpart) (void)hipFree(g->maxpart);
-  if (g->step) (void)hipFree(g->step);
-  if (g->prev) (void)hipFree(g->prev);
-  if (g->have_prev) (void)hipFree(g->have_prev);
-  if (g->flags) (void)hipFree(g->flags);
+  void *const blocks[] = {g->idef, g->v, g->hbuf, g->partials, g->maxpart, g->step, g->prev, g->have_prev, g->flags};
+  dev_free(blocks, 9);
 }
 
 extern "C" {
@@ -138,15 +131,15 @@ awk_status awk_greedy_create(awk_greedy_t *out, int nx, int ny, int nz, float sp
   const size_t N = (size_t)nx * ny * nz;
   g->nblk = fk_xblocks(g->k);
   hipError_t e = hipSuccess;
-  if (e == hipSuccess) e = hipMalloc(&g->idef, N * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&g->v, 3 * N * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&g->hbuf, 3 * N * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&g->partials, (size_t)g->nblk * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&g->maxpart, (size_t)g->nblk * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&g->step, sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&g->prev, sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&g->have_prev, sizeof(int));
-  if (e == hipSuccess) e = hipMalloc(&g->flags, sizeof(unsigned));
+  if (e == hipSuccess) e = dev_alloc(&g->idef, N * sizeof(float));
+  if (e == hipSuccess) e = dev_alloc(&g->v, 3 * N * sizeof(float));
+  if (e == hipSuccess) e = dev_alloc(&g->hbuf, 3 * N * sizeof(float));
+  if (e == hipSuccess) e = dev_alloc(&g->partials, (size_t)g->nblk * sizeof(double));
+  if (e == hipSuccess) e = dev_alloc(&g->maxpart, (size_t)g->nblk * sizeof(float));
+  if (e == hipSuccess) e = dev_alloc(&g->step, sizeof(float));
+  if (e == hipSuccess) e = dev_alloc(&g->prev, sizeof(double));
+  if (e == hipSuccess) e = dev_alloc(&g->have_prev, sizeof(int));
+  if (e == hipSuccess) e = dev_alloc(&g->flags, sizeof(unsigned));
   if (e == hipSuccess) e = hipMemset(g->flags, 0, sizeof(unsigned));
   if (e == hipSuccess) e = hipMemset(g->step, 0, sizeof(float));
   if (e == hipSuccess) e = hipMemset(g->prev, 0, sizeof(double));

@@ -352,10 +352,9 @@ using namespace awk;
 
 void awk::ldmm_release(awk_ldmm *l) {
   fk_release(l->k);
-  void *bufs[] = {l->h,      l->hs,     l->J,  l->diff,      l->acc,   l->partials, l->maxpart,
+  void *const bufs[] = {l->h,      l->hs,     l->J,  l->diff,      l->acc,   l->partials, l->maxpart,
                   l->step,   l->energy, l->jt, l->jd, l->sort_work, l->msplat, l->flags};
-  for (void *b : bufs)
-    if (b) (void)hipFree(b);
+  dev_free(bufs, (int)(sizeof(bufs) / sizeof(bufs[0])));
 }
 
 awk_status awk::ldmm_init(awk_ldmm *l, int nx, int ny, int nz, const float sp[3], float alpha,
@@ -379,20 +378,20 @@ awk_status awk::ldmm_init(awk_ldmm *l, int nx, int ny, int nz, const float sp[3]
   l->nblk = fk_xblocks(l->k);
   l->egrid = (int)grid_for((long long)N, kLdmmBlock);
   hipError_t e = hipSuccess;
-  if (e == hipSuccess) e = hipMalloc(&l->h, 3 * N * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&l->hs, 3 * N * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&l->J, (size_t)l->nt * N * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&l->diff, N * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&l->acc, N * sizeof(long long));
-  if (e == hipSuccess) e = hipMalloc(&l->partials, (size_t)l->egrid * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&l->maxpart, (size_t)l->nt * l->nblk * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&l->step, sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&l->energy, 3 * sizeof(double));
-  if (terms && e == hipSuccess) e = hipMalloc(&l->jt, (size_t)l->nt * N * sizeof(float));
-  if (terms && e == hipSuccess) e = hipMalloc(&l->jd, (size_t)l->nt * N * sizeof(float));
+  if (e == hipSuccess) e = dev_alloc(&l->h, 3 * N * sizeof(float));
+  if (e == hipSuccess) e = dev_alloc(&l->hs, 3 * N * sizeof(float));
+  if (e == hipSuccess) e = dev_alloc(&l->J, (size_t)l->nt * N * sizeof(float));
+  if (e == hipSuccess) e = dev_alloc(&l->diff, N * sizeof(float));
+  if (e == hipSuccess) e = dev_alloc(&l->acc, N * sizeof(long long));
+  if (e == hipSuccess) e = dev_alloc(&l->partials, (size_t)l->egrid * sizeof(double));
+  if (e == hipSuccess) e = dev_alloc(&l->maxpart, (size_t)l->nt * l->nblk * sizeof(float));
+  if (e == hipSuccess) e = dev_alloc(&l->step, sizeof(float));
+  if (e == hipSuccess) e = dev_alloc(&l->energy, 3 * sizeof(double));
+  if (terms && e == hipSuccess) e = dev_alloc(&l->jt, (size_t)l->nt * N * sizeof(float));
+  if (terms && e == hipSuccess) e = dev_alloc(&l->jd, (size_t)l->nt * N * sizeof(float));
   if (e == hipSuccess) e = hipMemset(l->acc, 0, N * sizeof(long long));
   if (e == hipSuccess) e = hipMemset(l->step, 0, sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&l->flags, sizeof(unsigned));
+  if (e == hipSuccess) e = dev_alloc(&l->flags, sizeof(unsigned));
   if (e == hipSuccess) e = hipMemset(l->flags, 0, sizeof(unsigned));
   return e == hipSuccess ? AWK_OK : hip_check(e, "LDMM iterator allocation");
 }
@@ -667,8 +666,8 @@ awk_status awk_ldmm_set_splat(awk_ldmm_t l, int mode) {
   if (mode == 1 && !l->sort_work) {
     const size_t N = (size_t)l->nx * l->ny * l->nz;
     if (8 * N > (size_t)((1LL << 31) - 1)) return fail(AWK_ERR_INVALID, "awk_ldmm_set_splat: sort/scan splat takes at most 2^28 voxels");
-    AWK_HIP(hipMalloc(&l->sort_work, splat_sorted_scratch_bytes(l->nx, l->ny, l->nz)));
-    AWK_HIP(hipMalloc(&l->msplat, N * sizeof(float)));
+    AWK_HIP(dev_alloc(&l->sort_work, splat_sorted_scratch_bytes(l->nx, l->ny, l->nz)));
+    AWK_HIP(dev_alloc(&l->msplat, N * sizeof(float)));
   }
   l->splat_mode = mode;
   return AWK_OK;

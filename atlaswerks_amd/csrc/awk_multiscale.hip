@@ -193,11 +193,11 @@ awk_status awk_gaussian_filter(float *out, const float *in, int nx, int ny, int 
   hipStream_t s = as_stream(stream);
   const size_t N = (size_t)nx * ny * nz;
   float *tmp = nullptr;
-  AWK_HIP(hipMallocAsync((void **)&tmp, N * sizeof(float), s));
+  AWK_HIP(scratch_alloc(&tmp, N * sizeof(float), s));
   const float sg[3] = {sigma_x, sigma_y, sigma_z};
   const int hk[3] = {half_x, half_y, half_z};
   awk_status st = gauss_passes(out, in, tmp, nx, ny, nz, sg, hk, s);
-  (void)hipFreeAsync(tmp, s);
+  (void)scratch_free(tmp, s);
   return st;
 }
 
@@ -217,7 +217,7 @@ awk_status awk_gaussian_downsample(float *out, int onx, int ony, int onz, const 
     hk[a] = 2 * (int)std::ceil(sd);
   }
   float *buf = nullptr;
-  AWK_HIP(hipMallocAsync((void **)&buf, 2 * N * sizeof(float), s));
+  AWK_HIP(scratch_alloc(&buf, 2 * N * sizeof(float), s));
   awk_status st = gauss_passes(buf, in, buf + N, nx, ny, nz, sg, hk, s);
   if (!st) {
     const unsigned grid = (unsigned)(((long long)onx * ony * onz + 255) / 256);
@@ -226,7 +226,7 @@ awk_status awk_gaussian_downsample(float *out, int onx, int ony, int onz, const 
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) st = hip_check(e, "k_resample_image");
   }
-  (void)hipFreeAsync(buf, s);
+  (void)scratch_free(buf, s);
   return st;
 }
 

@@ -123,12 +123,12 @@ awk_status launch_splat(float *dst, const float *src, const float *hx, const flo
     // a stream-ordered allocation: after the first call the pool hands the same
     // block back without a device allocation
     void *acc = nullptr;
-    AWK_HIP(hipMallocAsync(&acc, (size_t)N * 8, s));
+    AWK_HIP(scratch_alloc(&acc, (size_t)N * 8, s));
     awk_status st = clear_splat_acc(reinterpret_cast<unsigned long long *>(acc), N, s);
     if (st == AWK_OK)
       st = launch_splat_acc(dst, src, hx, hy, hz, nx, ny, nz,
                             reinterpret_cast<unsigned long long *>(acc), false, s);
-    hipError_t e = hipFreeAsync(acc, s);
+    hipError_t e = scratch_free(acc, s);
     if (st != AWK_OK) return st;
     AWK_HIP(e);
   } else if (mode == AWK_SPLAT_FIXED20) {

@@ -218,12 +218,15 @@ class GreedyWarp:
             if n_iter > 0:
                 it.UpdateStepSizeNextIteration()
                 it.Iterate(data, stream)
-                self.step_history.append(it.StepSize(stream))
+                if self.auto_step_reduce:  # later iterations may change it
+                    self.step_history.append(it.StepSize(stream))
             if self.compute_inverse:
                 for k in range(1, n_iter):
                     it.Iterate(data, stream)
             else:
                 it.IterateN(data, n_iter - 1, stream)
+            if n_iter > 0 and not self.auto_step_reduce:
+                self.step_history.append(it.StepSize(stream))
             flags = it.GetFlags(stream=stream)
             self.flags |= flags
             if flags & _lib.FLAG_NAN_ENERGY:
