@@ -354,33 +354,59 @@ k_pool_bwd(bf16 *__restrict__ dz, const bf16 *__restrict__ dp, const bf16 *__res
   *reinterpret_cast<bf16x8 *>(dz + p * C + gi * 8) = o;
 }
 
-// Adam (fp32 master weights); the gradient is cleared for the next step.
-__global__ void __launch_bounds__(256)
-k_adam(float *__restrict__ w, float *__restrict__ g, float *__restrict__ m, float *__restrict__ v,
-       long long n, float lr, float b1, float b2, float eps, float c1, float c2) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i];
-  const float mi = b1 * m[i] + (1.f - b1) * gi;
-  const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  w[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-  g[i] = 0.f;
-}
+// Where each layer's weights and biases go: the forward layout W[co][tap*cin + ci], the
+// gradient layout Wd[ci][(26 - tap)*cout + co] (layer 0 has none), both bf16, the fp32
+// biases and the head.  woff / boff: the blob offsets of the weights and of the bias.
+struct PackLayer {
+  bf16 *wf, *wd;
+  float *bias;
+  int woff, boff, cout, cin, cinb, kpad, kpad_d;
+};
+struct PackArgs {
+  PackLayer l[14];
+  float *head_w, *head_b;
+  int hoff, n;
+};
 
-// fp32 OIDHW weights -> the forward layout W[co][tap*cin + ci] and the gradient
-// layout Wd[ci][(26 - tap)*cout + co], both bf16.
+// ADAM: one Adam step on the fp32 master weights (the gradient is cleared for the next
+// one); either way the copies the convolutions read are refreshed.  One launch for the
+// update and all layers instead of 14 repacks and 16 small copies: 64^3 step 1.13 ->
+// 1.07 ms.
+template <bool ADAM>
 __global__ void __launch_bounds__(256)
-k_repack(bf16 *__restrict__ wf, bf16 *__restrict__ wd, const float *__restrict__ w, int cout,
-         int cin, int cinb, int kpad, int kpad_d) {
-  const int n = cout * cinb * 27;
+k_adam_pack(float *__restrict__ w, float *__restrict__ g, float *__restrict__ m, float *__restrict__ v, PackArgs a,
+            float lr, float b1, float b2, float eps, float c1, float c2) {
   const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (i >= n) return;
-  const int tap = i % 27, r = i / 27, ci = r % cinb, co = r / cinb;
-  const bf16 v = (bf16)w[i];
-  wf[(size_t)co * kpad + tap * cin + ci] = v;
-  if (wd) wd[(size_t)ci * kpad_d + (26 - tap) * cout + co] = v;
+  if (i >= a.n) return;
+  float wi = w[i];
+  if (ADAM) {
+    const float gi = g[i];
+    const float mi = b1 * m[i] + (1.f - b1) * gi;
+    const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
+    m[i] = mi;
+    v[i] = vi;
+    wi -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    w[i] = wi;
+    g[i] = 0.f;
+  }
+  if (i >= a.hoff) {
+    const int j = i - a.hoff;
+    if (j < 48) a.head_w[j] = wi;
+    else a.head_b[j - 48] = wi;
+    return;
+  }
+  int l = 0;
+#pragma unroll
+  for (int k = 1; k < 14; ++k) l = i >= a.l[k].woff ? k : l;
+  const PackLayer &L = a.l[l];
+  if (i >= L.boff) {
+    L.bias[i - L.boff] = wi;
+    return;
+  }
+  const int j = i - L.woff, tap = j % 27, r = j / 27, co = r / L.cinb, ci = r - co * L.cinb;
+  const bf16 h = (bf16)wi;
+  L.wf[(size_t)co * L.kpad + tap * L.cin + ci] = h;
+  if (L.wd) L.wd[(size_t)ci * L.kpad_d + (26 - tap) * L.cout + co] = h;
 }
 
 }  // namespace awk
@@ -416,19 +442,19 @@ static void trainer_free(awk_unet_trainer *t) {
     if (t->wd[l]) (void)hipFree(t->wd[l]);
 }
 
-static awk_status repack_all(awk_unet_trainer *t, hipStream_t s) {
-  awk_unet *u = t->net;
+static PackArgs pack_args(const awk_unet_trainer *t) {
+  const awk_unet *u = t->net;
+  PackArgs a;
   for (int l = 0; l < 14; ++l) {
     const LayerSpec &L = kUnetLayers[l];
-    const int n = L.cout * kUnetBlobCin[l] * 27;
-    AWK_LAUNCH(k_repack, dim3((n + 255) / 256), dim3(256), 0, s, u->w[l], t->wd[l], t->w + t->woff[l],
-               L.cout, L.cin, kUnetBlobCin[l], u->kpad[l], t->kpad_d[l]);
-    AWK_HIP(hipMemcpyAsync(u->bias[l], t->w + t->boff[l], L.cout * sizeof(float), hipMemcpyDeviceToDevice, s));
+    a.l[l] = PackLayer{u->w[l], t->wd[l], u->bias[l], (int)t->woff[l], (int)t->boff[l], L.cout, L.cin,
+                       kUnetBlobCin[l], u->kpad[l], t->kpad_d[l]};
   }
-  AWK_HIP(hipMemcpyAsync(u->head_w, t->w + t->hoff, 48 * sizeof(float), hipMemcpyDeviceToDevice, s));
-  AWK_HIP(hipMemcpyAsync(u->head_b, t->w + t->hoff + 48, 3 * sizeof(float), hipMemcpyDeviceToDevice, s));
-  AWK_LAUNCH_CHECK("k_repack");
-  return AWK_OK;
+  a.head_w = u->head_w;
+  a.head_b = u->head_b;
+  a.hoff = (int)t->hoff;
+  a.n = (int)t->nw;
+  return a;
 }
 
 // dX = conv^T(dZ) of layer l: the output has cin_l channels, scaled by the
@@ -641,7 +667,12 @@ awk_status awk_unet_trainer_create(awk_unet_trainer_t *out, awk_unet_t net, cons
     e = hipMalloc(&t->ws2, (kWgWsFloats / kWgSumRows + max_ne + (size_t)kWgMaxBlocks * 128) * sizeof(float));
   awk_status st = AWK_OK;
   if (e != hipSuccess) st = hip_check(e, "awk_unet_trainer_create: allocation");
-  if (!st) st = repack_all(t, nullptr);
+  if (!st) {
+    AWK_LAUNCH(k_adam_pack<false>, dim3((unsigned)((t->nw + 255) / 256)), dim3(256), 0, nullptr, t->w, t->g, t->m,
+               t->v, pack_args(t), 0.f, 0.f, 0.f, 0.f, 1.f, 1.f);
+    const hipError_t le = hipGetLastError();
+    if (le != hipSuccess) st = hip_check(le, "k_adam_pack");
+  }
   if (!st) {
     hipError_t se = hipDeviceSynchronize();
     if (se != hipSuccess) st = hip_check(se, "awk_unet_trainer_create: repack");
@@ -671,14 +702,14 @@ awk_status awk_unet_trainer_step(awk_unet_trainer_t t, const float *templ, const
   hipStream_t s = as_stream(stream);
   awk_status st;
   if ((st = train_backward(t, templ, subject, target, loss_dev, s))) return st;
-  // Adam, then the bf16 copies the convolutions read
+  // Adam and the copies the convolutions read
   ++t->t;
   const float b1c = 0.9f, b2c = 0.999f;
   const float c1c = 1.f - std::pow(b1c, (float)t->t), c2c = 1.f - std::pow(b2c, (float)t->t);
-  AWK_LAUNCH(k_adam, dim3((unsigned)((t->nw + 255) / 256)), dim3(256), 0, s, t->w, t->g, t->m, t->v,
-             (long long)t->nw, lr, b1c, b2c, 1e-8f, c1c, c2c);
-  AWK_LAUNCH_CHECK("k_adam");
-  return repack_all(t, s);
+  AWK_LAUNCH(k_adam_pack<true>, dim3((unsigned)((t->nw + 255) / 256)), dim3(256), 0, s, t->w, t->g, t->m, t->v,
+             pack_args(t), lr, b1c, b2c, 1e-8f, c1c, c2c);
+  AWK_LAUNCH_CHECK("k_adam_pack");
+  return AWK_OK;
 }
 
 awk_status awk_unet_trainer_gradients(awk_unet_trainer_t t, const float *templ, const float *subject,
