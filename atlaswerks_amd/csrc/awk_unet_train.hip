@@ -413,6 +413,8 @@ k_adam_pack(float *__restrict__ w, float *__restrict__ g, float *__restrict__ m,
 
 using namespace awk;
 
+constexpr int kWgForks = 8;
+
 struct awk_unet_trainer {
   awk_unet *net = nullptr;
   size_t nw = 0;
@@ -430,6 +432,10 @@ struct awk_unet_trainer {
   float *hpart = nullptr; // head-gradient block partials [blocks][52]
   float *ws = nullptr;    // weight-gradient block partials (kWgWsFloats + bias partials)
   float *ws2 = nullptr;   // their first reduction stage
+  // the weight gradients' own stream, forked from the caller's each time an output
+  // gradient is ready and joined before the update
+  hipStream_t side = nullptr;
+  hipEvent_t fork[kWgForks] = {}, join = nullptr;
 };
 
 static void trainer_free(awk_unet_trainer *t) {
@@ -440,6 +446,10 @@ static void trainer_free(awk_unet_trainer *t) {
     if (p) (void)hipFree(p);
   for (int l = 0; l < 14; ++l)
     if (t->wd[l]) (void)hipFree(t->wd[l]);
+  for (hipEvent_t e : t->fork)
+    if (e) (void)hipEventDestroy(e);
+  if (t->join) (void)hipEventDestroy(t->join);
+  if (t->side) (void)hipStreamDestroy(t->side);
 }
 
 static PackArgs pack_args(const awk_unet_trainer *t) {
@@ -552,52 +562,70 @@ static awk_status train_backward(awk_unet_trainer *t, const float *templ, const 
   AWK_LAUNCH_CHECK("k_head_bwd");
   const float sl = kUnetSlope;
   auto blocks = [](long long n) { return dim3((unsigned)((n + 255) / 256)); };
+  // The chain of output gradients stays on the caller's stream; the weight gradients,
+  // which nothing in it reads, follow on their own stream and fill the chip beside it
+  // (64^3: most launches of either are fewer blocks than the chip holds).  They share
+  // the workspace, so they stay in order among themselves.
+  int forks = 0;
+  auto fork = [&]() -> awk_status {
+    hipEvent_t e = t->fork[forks++];
+    AWK_HIP(hipEventRecord(e, s));
+    AWK_HIP(hipStreamWaitEvent(t->side, e, 0));
+    return AWK_OK;
+  };
+  struct Wg {
+    int l;
+    const bf16 *dz, *x;
+    int nx, ny, nz;
+  };
+  auto wgrads = [&](std::initializer_list<Wg> list) -> awk_status {
+    awk_status r = fork();
+    for (const Wg &g : list)
+      if (!r) r = wgrad(t, g.l, g.dz, g.x, g.nx, g.ny, g.nz, t->side);
+    return r;
+  };
   // decoder level 0
-  if ((st = wgrad(t, 13, t->dz13, u->d0a, nx, ny, nz, s))) return st;
   if ((st = dgrad(t, 13, t->dz13, u->d0a, t->dz12, nx, ny, nz, s))) return st;
-  if ((st = wgrad(t, 12, t->dz12, u->c0, nx, ny, nz, s))) return st;
+  if ((st = wgrads({{13, t->dz13, u->d0a, nx, ny, nz}, {12, t->dz12, u->c0, nx, ny, nz}}))) return st;
   if ((st = dgrad(t, 12, t->dz12, nullptr, t->dc0, nx, ny, nz, s))) return st;
   AWK_LAUNCH(k_upcat_bwd, blocks((long long)(n0 / 8) * 4), dim3(256), 0, s, t->dz11, t->dc0, u->d1, 32, 48,
              nx, ny, nz, sl);
   // decoder level 1
-  if ((st = wgrad(t, 11, t->dz11, u->d1a, a1, b1, c1, s))) return st;
   if ((st = dgrad(t, 11, t->dz11, u->d1a, t->dz10, a1, b1, c1, s))) return st;
-  if ((st = wgrad(t, 10, t->dz10, u->c1, a1, b1, c1, s))) return st;
+  if ((st = wgrads({{11, t->dz11, u->d1a, a1, b1, c1}, {10, t->dz10, u->c1, a1, b1, c1}}))) return st;
   if ((st = dgrad(t, 10, t->dz10, nullptr, t->dc1, a1, b1, c1, s))) return st;
   AWK_LAUNCH(k_upcat_bwd, blocks((long long)(n0 / 64) * 8), dim3(256), 0, s, t->dz9, t->dc1, u->d2, 64, 96,
              a1, b1, c1, sl);
   // decoder level 2
-  if ((st = wgrad(t, 9, t->dz9, u->d2a, a2, b2, c2, s))) return st;
   if ((st = dgrad(t, 9, t->dz9, u->d2a, t->dz8, a2, b2, c2, s))) return st;
-  if ((st = wgrad(t, 8, t->dz8, u->c2, a2, b2, c2, s))) return st;
+  if ((st = wgrads({{9, t->dz9, u->d2a, a2, b2, c2}, {8, t->dz8, u->c2, a2, b2, c2}}))) return st;
   if ((st = dgrad(t, 8, t->dz8, nullptr, t->dc2, a2, b2, c2, s))) return st;
   AWK_LAUNCH(k_upcat_bwd, blocks((long long)(n0 / 512) * 16), dim3(256), 0, s, t->dz7, t->dc2, u->s3, 128,
              192, a2, b2, c2, sl);
   // bottom
-  if ((st = wgrad(t, 7, t->dz7, u->t3, a3, b3, c3, s))) return st;
   if ((st = dgrad(t, 7, t->dz7, u->t3, t->dz6, a3, b3, c3, s))) return st;
-  if ((st = wgrad(t, 6, t->dz6, u->p2, a3, b3, c3, s))) return st;
+  if ((st = wgrads({{7, t->dz7, u->t3, a3, b3, c3}, {6, t->dz6, u->p2, a3, b3, c3}}))) return st;
   if ((st = dgrad(t, 6, t->dz6, nullptr, t->dp2, a3, b3, c3, s))) return st;
   // encoder level 2: pooled gradient + skip from the level-2 concatenation
   AWK_LAUNCH(k_pool_bwd, blocks((long long)(n0 / 64) * 8), dim3(256), 0, s, t->dz5, t->dp2, t->dc2, 192,
              128, u->s2, 64, a2, b2, c2, sl);
-  if ((st = wgrad(t, 5, t->dz5, u->t2, a2, b2, c2, s))) return st;
   if ((st = dgrad(t, 5, t->dz5, u->t2, t->dz4, a2, b2, c2, s))) return st;
-  if ((st = wgrad(t, 4, t->dz4, u->p1, a2, b2, c2, s))) return st;
+  if ((st = wgrads({{5, t->dz5, u->t2, a2, b2, c2}, {4, t->dz4, u->p1, a2, b2, c2}}))) return st;
   if ((st = dgrad(t, 4, t->dz4, nullptr, t->dp1, a2, b2, c2, s))) return st;
   // encoder level 1
   AWK_LAUNCH(k_pool_bwd, blocks((long long)(n0 / 8) * 4), dim3(256), 0, s, t->dz3, t->dp1, t->dc1, 96, 64,
              u->s1, 32, a1, b1, c1, sl);
-  if ((st = wgrad(t, 3, t->dz3, u->t1, a1, b1, c1, s))) return st;
   if ((st = dgrad(t, 3, t->dz3, u->t1, t->dz2, a1, b1, c1, s))) return st;
-  if ((st = wgrad(t, 2, t->dz2, u->p0, a1, b1, c1, s))) return st;
+  if ((st = wgrads({{3, t->dz3, u->t1, a1, b1, c1}, {2, t->dz2, u->p0, a1, b1, c1}}))) return st;
   if ((st = dgrad(t, 2, t->dz2, nullptr, t->dp0, a1, b1, c1, s))) return st;
   // encoder level 0
   AWK_LAUNCH(k_pool_bwd, blocks((long long)n0 * 2), dim3(256), 0, s, t->dz1, t->dp0, t->dc0, 48, 32,
              u->s0, 16, nx, ny, nz, sl);
-  if ((st = wgrad(t, 1, t->dz1, u->t0, nx, ny, nz, s))) return st;
+  if ((st = wgrads({{1, t->dz1, u->t0, nx, ny, nz}}))) return st;
   if ((st = dgrad(t, 1, t->dz1, u->t0, t->dz0, nx, ny, nz, s))) return st;
-  if ((st = wgrad(t, 0, t->dz0, u->x0, nx, ny, nz, s))) return st;
+  if ((st = wgrads({{0, t->dz0, u->x0, nx, ny, nz}}))) return st;
+  AWK_HIP(hipEventRecord(t->join, t->side));
+  AWK_HIP(hipStreamWaitEvent(s, t->join, 0));
   AWK_LAUNCH_CHECK("backward");
   return AWK_OK;
 }
@@ -665,6 +693,10 @@ awk_status awk_unet_trainer_create(awk_unet_trainer_t *out, awk_unet_t net, cons
   }
   if (e == hipSuccess)
     e = hipMalloc(&t->ws2, (kWgWsFloats / kWgSumRows + max_ne + (size_t)kWgMaxBlocks * 128) * sizeof(float));
+  if (e == hipSuccess) e = hipStreamCreateWithFlags(&t->side, hipStreamNonBlocking);
+  for (hipEvent_t &ev : t->fork)
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+  if (e == hipSuccess) e = hipEventCreateWithFlags(&t->join, hipEventDisableTiming);
   awk_status st = AWK_OK;
   if (e != hipSuccess) st = hip_check(e, "awk_unet_trainer_create: allocation");
   if (!st) {
