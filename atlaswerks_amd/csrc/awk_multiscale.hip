@@ -44,18 +44,8 @@ static GaussTab make_tab(float sigma, int k) {
   return t;
 }
 
-// One axis of the separable filter: out(p) from in along `axis` (stride s, length n).
-__global__ void __launch_bounds__(256)
-k_gauss_axis(float *__restrict__ out, const float *__restrict__ in, int nx, int ny, int nz,
-             int axis, GaussTab t) {
-  const int N = nx * ny * nz;
-  const int id = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (id >= N) return;
-  const int x = id % nx, r = id / nx, y = r % ny, z = r / ny;
-  const int p = axis == 0 ? x : axis == 1 ? y : z;
-  const int n = axis == 0 ? nx : axis == 1 ? ny : nz;
-  const int s = axis == 0 ? 1 : axis == 1 ? nx : nx * ny;
-  const float *c = in + id;
+// The filtered value at position p of a line (c: its element p, stride s, length n).
+__device__ __forceinline__ float gauss_at(const float *__restrict__ c, int p, int n, int s, const GaussTab &t) {
   const int k = t.k;
   float acc;
   if (p >= k && p < n - k) {
@@ -74,7 +64,41 @@ k_gauss_axis(float *__restrict__ out, const float *__restrict__ in, int nx, int 
     for (int i = 1; i <= q; ++i) acc += (c[i * s] + c[-i * s]) * g[i];
     for (int i = q + 1; i <= k; ++i) acc += c[-i * s] * g[i];
   }
-  out[id] = acc;
+  return acc;
+}
+
+// One axis of the separable filter: out(p) from in along `axis` (stride s, length n).
+__global__ void __launch_bounds__(256)
+k_gauss_axis(float *__restrict__ out, const float *__restrict__ in, int nx, int ny, int nz,
+             int axis, GaussTab t) {
+  const int N = nx * ny * nz;
+  const int id = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (id >= N) return;
+  const int x = id % nx, r = id / nx, y = r % ny, z = r / ny;
+  const int p = axis == 0 ? x : axis == 1 ? y : z;
+  const int n = axis == 0 ? nx : axis == 1 ? ny : nz;
+  const int s = axis == 0 ? 1 : axis == 1 ? nx : nx * ny;
+  out[id] = gauss_at(in + id, p, n, s, t);
+}
+
+// One axis of the downsampling, filter and resampling together: both are separable, so
+// only the two filtered values that an output position reads are formed, and each
+// axis's output is already the smaller one.  in: [A][n][B], out: [A][m][B]; output j
+// reads f j + (f - 1)/2 (f >= 1, so inside the line).  Bound by the first axis's read of
+// the image: 160 x 192 x 144 by 2, three passes 75 us and a copy and a gather before,
+// 35 us in all now.
+__global__ void __launch_bounds__(256)
+k_gauss_down_axis(float *__restrict__ out, const float *__restrict__ in, int n, int m, int B, int total, double f,
+                  GaussTab t) {
+  const int id = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (id >= total) return;
+  const int b = id % B, r = id / B, j = r % m, a = r / m;
+  const float pos = (float)(f * j + (f - 1.0) / 2.0), fl = floorf(pos), w = pos - fl;
+  const int p = (int)fl;
+  const float *c = in + ((size_t)a * n + p) * B + b;
+  const float v0 = gauss_at(c, p, n, B, t);
+  const float v1 = p + 1 < n ? gauss_at(c + B, p + 1, n, B, t) : 0.f;
+  out[id] = fmaf(w, v1, (1.f - w) * v0);
 }
 
 // resampleNew of the filtered image: output voxel x reads the source at
@@ -149,6 +173,24 @@ k_affine_displace(float *hx, float *hy, float *hz, const float *ux, const float 
   hz[id] = c;
 }
 
+// The half size as GaussianFilter3D.cxx:178-184 clips it, to n/2 - 1; below 2 voxels
+// (where the reference's unsigned arithmetic skips the clip) no filtering.
+static int clip_half(int half, int n) {
+  const int kmax = n / 2 - 1 > 0 ? n / 2 - 1 : 0;
+  return half < 0 ? 0 : (half > kmax ? kmax : half);
+}
+
+static awk_status gauss_down_axis(float *out, const float *in, int n, int m, int B, int A, float sigma, int half,
+                                  hipStream_t s) {
+  const int k = clip_half(half, n);
+  if (k > kMaxHalf) return fail(AWK_ERR_UNSUPPORTED, "gaussian filter: half kernel size above 15");
+  const int total = A * m * B;
+  AWK_LAUNCH(k_gauss_down_axis, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, out, in, n, m, B, total,
+             (double)n / m, make_tab(sigma, k));
+  AWK_LAUNCH_CHECK("k_gauss_down_axis");
+  return AWK_OK;
+}
+
 static awk_status gauss_passes(float *out, const float *in, float *tmp, int nx, int ny, int nz,
                                const float sigma[3], const int half[3], hipStream_t s) {
   const int N = nx * ny * nz;
@@ -158,10 +200,7 @@ static awk_status gauss_passes(float *out, const float *in, float *tmp, int nx, 
   const float *src[3] = {in, tmp, out};
   float *dst[3] = {tmp, out, tmp};
   for (int a = 0; a < 3; ++a) {
-    // GaussianFilter3D.cxx:178-184 clips the half size to n/2 - 1; below 2 voxels
-    // (where the reference's unsigned arithmetic skips the clip) no filtering
-    const int kmax = dims[a] / 2 - 1 > 0 ? dims[a] / 2 - 1 : 0;
-    const int k = half[a] < 0 ? 0 : (half[a] > kmax ? kmax : half[a]);
+    const int k = clip_half(half[a], dims[a]);
     if (k > kMaxHalf) return fail(AWK_ERR_UNSUPPORTED, "gaussian filter: half kernel size above 15");
     const GaussTab t = make_tab(sigma[a], k);
     AWK_LAUNCH(k_gauss_axis, dim3(grid), dim3(256), 0, s, dst[a], src[a], nx, ny, nz, a, t);
@@ -218,6 +257,15 @@ awk_status awk_gaussian_downsample(float *out, int onx, int ony, int onz, const 
   }
   float *buf = nullptr;
   AWK_HIP(scratch_alloc(&buf, 2 * N * sizeof(float), s));
+  if (onx <= nx && ony <= ny && onz <= nz) {
+    // axis by axis, the longest stride first: z, y, x
+    float *mid = buf + (size_t)nx * ny * onz;
+    awk_status st = gauss_down_axis(buf, in, nz, onz, nx * ny, 1, sg[2], hk[2], s);
+    if (!st) st = gauss_down_axis(mid, buf, ny, ony, nx, onz, sg[1], hk[1], s);
+    if (!st) st = gauss_down_axis(out, mid, nx, onx, 1, onz * ony, sg[0], hk[0], s);
+    (void)scratch_free(buf, s);
+    return st;
+  }
   awk_status st = gauss_passes(buf, in, buf + N, nx, ny, nz, sg, hk, s);
   if (!st) {
     const unsigned grid = (unsigned)(((long long)onx * ony * onz + 255) / 256);

@@ -113,3 +113,17 @@ def test_atlas_multiscale_runs_and_descends():
     for a0, a1 in ((0, 6), (6, 12), (12, 16)):
         assert np.all(np.diff(e[a0:a1]) < 0)
     assert b.level_size() == (32, 32, 32)
+
+
+@pytest.mark.parametrize("shape,new", [((9, 33, 10), (9, 7, 5)), ((5, 64, 3), (5, 4, 1)), ((8, 6, 5), (10, 6, 4)),
+                                       ((40, 17, 130), (13, 17, 65))])
+def test_gaussian_downsample_axes(shape, new):
+    """Axis by axis where every axis shrinks or stays (odd ratios, a factor of 16, an
+    axis left as it is), the filtered volume where one grows: the same bar."""
+    import torch
+    from atlaswerks_amd import hfield
+    from gpu_util import host, rel_l2, to_dev
+    a = np.random.default_rng(3).standard_normal(shape).astype(np.float32)
+    out = torch.empty(new, dtype=torch.float32, device="cuda")
+    hfield.gaussianDownsample(out, to_dev(a))
+    assert rel_l2(host(out), oracle.gaussian_downsample(a, new)) <= 1e-6
