@@ -43,7 +43,8 @@ enum XStore {
   XSTORE_MAXNORM = 1,  // write v and a per-block max |v|
   XSTORE_COMPOSE = 2,  // h_new(x) = h(x + step * v(x) / sp) (PARTIAL_ID); v not written
   XSTORE_AXPBY = 3,    // out = (1 - 2 step) out + (2 step / sigma^2) v   (LDMM velocity update)
-  XSTORE_MAXAXPY = 4   // per-block max |2 out - (2 / sigma^2) v|; out not written
+  XSTORE_MAXAXPY = 4,  // per-block max |2 out - (2 / sigma^2) v|; out not written
+  XSTORE_DOT = 5       // per-block FP64 sums of out . v (LDMM vector energy); out not written
 };
 
 // Prologue of the forward x pass.
@@ -93,6 +94,7 @@ struct XInvArgs {
   int mode;
   float *out[3];            // PLAIN / MAXNORM: output planes
   float *maxpart;           // MAXNORM: one float per block
+  double *dotpart;          // DOT: one double per block
   const float *h[3];        // COMPOSE: current hfield
   float *hnew[3];           // COMPOSE: updated hfield
   const float *step;        // COMPOSE / AXPBY: step size (device scalar)

@@ -391,6 +391,7 @@ k_xinv(XInvArgs a, Axis ax, XPlan xp, int nx_rt, int ny, int nz, int nxh_rt, int
   if (r0 >= NR) {
     // a padding block of the grid: its max partial is still read
     if ((a.mode == XSTORE_MAXNORM || a.mode == XSTORE_MAXAXPY) && threadIdx.x == 0) a.maxpart[lb] = 0.f;
+    if (a.mode == XSTORE_DOT && threadIdx.x == 0) a.dotpart[lb] = 0.0;
     return;
   }
   float *smf = reinterpret_cast<float *>(sm);
@@ -480,6 +481,7 @@ k_xinv(XInvArgs a, Axis ax, XPlan xp, int nx_rt, int ny, int nz, int nxh_rt, int
     }
   };
   float mx = 0.f;
+  double dot = 0.0;
   if (a.mode == XSTORE_COMPOSE) {
     // updateDeformation (GreedyIteratorCPU.cxx:81-95): v *= step; h <- composeHV(h, v, sp, PARTIAL_ID).
     // XU voxels per step: their 24*XU gathers are in flight together.
@@ -642,12 +644,30 @@ k_xinv(XInvArgs a, Axis ax, XPlan xp, int nx_rt, int ny, int nz, int nxh_rt, int
         const float q1 = 2.f * a.out[1][base] + cua * v1;
         const float q2 = 2.f * a.out[2][base] + cua * v2;
         mx = fmaxf(mx, sqrtf(q0 * q0 + q1 * q1 + q2 * q2));
+      } else if (a.mode == XSTORE_DOT) {
+        dot += (double)v0 * a.out[0][base];
+        dot += (double)v1 * a.out[1][base];
+        dot += (double)v2 * a.out[2][base];
       } else {
         a.out[0][base] = v0;
         a.out[1][base] = v1;
         a.out[2][base] = v2;
         if (a.mode == XSTORE_MAXNORM) mx = fmaxf(mx, sqrtf(v0 * v0 + v1 * v1 + v2 * v2));
       }
+    }
+  }
+  if (a.mode == XSTORE_DOT) {
+    __shared__ double redd[16];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) dot += __shfl_down(dot, off, 64);
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    if (lane == 0) redd[wave] = dot;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      double t = 0.0;
+      const int nw = (bdim + 63) >> 6;
+      for (int i = 0; i < nw; ++i) t += redd[i];
+      a.dotpart[lb] = t;
     }
   }
   if (a.mode == XSTORE_MAXNORM || a.mode == XSTORE_MAXAXPY) {

@@ -19,6 +19,7 @@
 //             pass updates v_t = (1 - 2 eps) v_t + (2 eps / sigma^2) u in place
 //             (or, on the step-size call, takes max |2 v_t - 2/sigma^2 u|).
 // No host synchronisation; energies stay on the device (FP64, fixed order).
+#include <algorithm>
 #include <cstring>
 #include <new>
 #include <utility>
@@ -144,21 +145,6 @@ k_ldmm_alpha(float *__restrict__ alpha, long long *__restrict__ acc, int N, floa
 __global__ void __launch_bounds__(kLdmmBlock) k_ldmm_zero(long long *__restrict__ acc, int N) {
   const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   if (i < N) acc[i] = 0;
-}
-
-// FP64 dot product partials of two 3-plane fields: sum_c a_c . b_c
-__global__ void __launch_bounds__(kLdmmBlock)
-k_ldmm_dot(const float *__restrict__ a, const float *__restrict__ b0, const float *__restrict__ b1,
-           const float *__restrict__ b2, int N, double *__restrict__ partials) {
-  const int lb = (int)xcd_block();
-  const int i = lb * kLdmmBlock + (int)threadIdx.x;
-  double s = 0.0;
-  if (i < N) {
-    s = (double)a[i] * b0[i];
-    s += (double)a[N + i] * b1[i];
-    s += (double)a[2 * N + i] * b2[i];
-  }
-  block_sum_store(s, partials, lb);
 }
 
 // energy[0] = Prod(sp) * sum(diff^2) / sigma^2 (LDMMIteratorGPU.cxx:276-283,
@@ -383,7 +369,7 @@ awk_status awk::ldmm_init(awk_ldmm *l, int nx, int ny, int nz, const float sp[3]
   if (e == hipSuccess) e = dev_alloc(&l->J, (size_t)l->nt * N * sizeof(float));
   if (e == hipSuccess) e = dev_alloc(&l->diff, N * sizeof(float));
   if (e == hipSuccess) e = dev_alloc(&l->acc, N * sizeof(long long));
-  if (e == hipSuccess) e = dev_alloc(&l->partials, (size_t)l->egrid * sizeof(double));
+  if (e == hipSuccess) e = dev_alloc(&l->partials, (size_t)std::max(l->egrid, l->nblk) * sizeof(double));
   if (e == hipSuccess) e = dev_alloc(&l->maxpart, (size_t)l->nt * l->nblk * sizeof(float));
   if (e == hipSuccess) e = dev_alloc(&l->step, sizeof(float));
   if (e == hipSuccess) e = dev_alloc(&l->energy, 3 * sizeof(double));
@@ -396,33 +382,28 @@ awk_status awk::ldmm_init(awk_ldmm *l, int nx, int ny, int nz, const float sp[3]
   return e == hipSuccess ? AWK_OK : hip_check(e, "LDMM iterator allocation");
 }
 
-// energy[1] += Prod(sp) <L v_t, v_t> / T, with L applied to a copy of v_t in lv (3N).
-static awk_status vec_energy_step(awk_ldmm *l, float *const v[], int t, float *lv, double *energy,
-                                  hipStream_t s) {
-  const int N = l->nx * l->ny * l->nz;
+// energy[1] += Prod(sp) <L v_t, v_t> / T.  The operator reads v_t in place and its last
+// pass takes the products with v_t instead of storing L v_t: no copy of v_t, no field
+// written and read back (96 x 80 x 64: three 5 us copies and a 5 us dot product per t).
+static awk_status vec_energy_step(awk_ldmm *l, float *const v[], int t, double *energy, hipStream_t s) {
   const double vol = (double)l->sp[0] * l->sp[1] * l->sp[2];
   awk_status st;
   int nb = 0;
-  for (int c = 0; c < 3; ++c)
-    AWK_HIP(hipMemcpyAsync(lv + (size_t)c * N, v[3 * t + c], (size_t)N * sizeof(float),
-                           hipMemcpyDeviceToDevice, s));
   XFwdArgs pa;
   std::memset(&pa, 0, sizeof(pa));
   pa.mode = XLOAD_PLAIN;
-  for (int c = 0; c < 3; ++c) pa.in[c] = lv + (size_t)c * N;
+  for (int c = 0; c < 3; ++c) pa.in[c] = v[3 * t + c];
   if ((st = fk_xfwd(l->k, pa, s, &nb))) return st;
   if ((st = fk_ypass(l->k, false, s, nullptr))) return st;
   if ((st = fk_zsolve(l->k, false, s))) return st;
   if ((st = fk_ypass(l->k, true, s, nullptr))) return st;
   XInvArgs pi;
   std::memset(&pi, 0, sizeof(pi));
-  pi.mode = XSTORE_PLAIN;
-  for (int c = 0; c < 3; ++c) pi.out[c] = lv + (size_t)c * N;
+  pi.mode = XSTORE_DOT;
+  for (int c = 0; c < 3; ++c) pi.out[c] = v[3 * t + c];
+  pi.dotpart = l->partials;
   if ((st = fk_xinv(l->k, pi, s, &nb))) return st;
-  AWK_LAUNCH(k_ldmm_dot, dim3(l->egrid), dim3(kLdmmBlock), 0, s, lv, v[3 * t], v[3 * t + 1],
-             v[3 * t + 2], N, l->partials);
-  AWK_LAUNCH(k_ldmm_vec_energy, dim3(1), dim3(256), 0, s, l->partials, l->egrid, vol / l->nt,
-             energy, l->flags);
+  AWK_LAUNCH(k_ldmm_vec_energy, dim3(1), dim3(256), 0, s, l->partials, nb, vol / l->nt, energy, l->flags);
   AWK_LAUNCH_CHECK("vector energy");
   return AWK_OK;
 }
@@ -514,7 +495,7 @@ awk_status awk::ldmm_orig_forward(awk_ldmm *l, const float *I0, const float *I1,
                  vol * inv_sig2, energy, l->flags);
       AWK_LAUNCH_CHECK("k_orig_image_energy");
     }
-    if (!alpha && !step_call && vec_energy && (st = vec_energy_step(l, v, t, hs, energy, s)))
+    if (!alpha && !step_call && vec_energy && (st = vec_energy_step(l, v, t, energy, s)))
       return st;
   }
   if (step_call) {
@@ -603,8 +584,7 @@ awk_status awk::ldmm_new_iterate(awk_ldmm *l, const float *I0, const float *I1, 
                            sorted ? l->msplat : nullptr, sorted ? nullptr : l->acc, step, step_call,
                            s)))
       return st;
-    // <L v_t, v_t> with L applied to a copy of v_t in the free hfield buffer
-    if (!step_call && vec_energy && (st = vec_energy_step(l, v, t, hs, energy, s))) return st;
+    if (!step_call && vec_energy && (st = vec_energy_step(l, v, t, energy, s))) return st;
   }
   if (step_call) {
     if ((st = launch_step_from_max(l->maxpart, T * l->nblk, l->max_pert, step, l->flags, s)))

@@ -136,3 +136,23 @@ def test_ldmm_warp_scale_levels_vs_oracle():
     np.testing.assert_allclose(w.energy_history[0][:, 0], eic, rtol=1e-4)
     np.testing.assert_allclose(w.energy_history[1][:, 0], eif, rtol=1e-4)
     np.testing.assert_allclose(w.energy_history[1][:, 1], evf, rtol=1e-4)
+
+
+@pytest.mark.parametrize("shape", [(9, 40, 5), (6, 21, 31), (5, 18, 128), (4, 9, 256)])
+@pytest.mark.parametrize("orig", GRADIENTS)
+def test_ldmm_vector_energy_rows(shape, orig):
+    """The vector energy summed by the operator's last pass: rows so short that a block
+    has fewer voxels than threads, a dense and two specialised row lengths, row groups
+    past the volume's end.  The energy bar above (1e-5)."""
+    import torch
+    from atlaswerks_amd import ldmm
+    from gpu_util import to_dev
+    print("ldmm energy", shape, orig, flush=True)
+    I0, I1 = _pair(shape, seed=9, disp=0.8)
+    v_ref, ei, ev, st = _oracle_run(orig)(I0, I1, 2, 2, sigma=0.1, max_pert=0.1)
+    prm = ldmm.LDMMIteratorParam(sigma=0.1, max_pert=0.1, use_orig_gradient=orig)
+    w = ldmm.LDMMWarp(to_dev(I0), to_dev(I1), n_time_steps=2, n_iter=2, param=prm)
+    e = w.RunWarp(vec_energy=True)
+    torch.cuda.synchronize()
+    np.testing.assert_allclose(e.energies()[:, 1], ev, rtol=1e-5)
+    np.testing.assert_allclose(e.energies()[:, 0], ei, rtol=1e-5)
