@@ -331,9 +331,9 @@ constexpr size_t kPassLdsMax = 160 * 1024 - 1024;
 // Whether an axis is transformed as a dense product (awk_dense.h): a length with a
 // prime factor above 13, whose LDS stages would be a direct DFT of that prime or a
 // chirp-z transform.  L^-1 at 181 x 217 x 181 4347 -> 576 us, 251 x 241 x 239 7189 ->
-// 1097, 248 x 186 x 155 2611 -> 552, 62^3 184 -> 66, 32 x 31 x 36 63 -> 37, with a
-// smaller error against 64 bits each time.  Lengths of small primes keep their LDS
-// stages: at 200^3 553 us (dense 664), and half as many roundings.
+// 1085, 248 x 186 x 155 2611 -> 546, 62^3 184 -> 47, 32 x 31 x 36 63 -> 25, with a
+// smaller error against 64 bits each time.  Lengths of small primes are faster, and
+// round half as often, as radices: at 200^3 382 us (dense 664).
 static bool use_dense(int n, const std::vector<int> &rad) {
   if (n < kDenseMin || n > kDenseMax) return false;
   for (int r : rad)
