@@ -51,6 +51,14 @@ struct SplatPosH {
   __device__ __forceinline__ float3 at(int i) const { return make_float3(hx[i], hy[i], hz[i]); }
 };
 
+// h at voxel i; hx null: the identity.
+__device__ __forceinline__ float3 voxel_or(const float *__restrict__ hx, const float *__restrict__ hy,
+                                           const float *__restrict__ hz, int i, Dims d) {
+  if (hx) return make_float3(hx[i], hy[i], hz[i]);
+  const int x = i % d.nx, r = i / d.nx;
+  return make_float3((float)x, (float)(r % d.ny), (float)(r / d.ny));
+}
+
 // LDMM backward step: h' = h - v(h)/sp (composeVHInv, PARTIAL_ZERO), also stored to
 // (ox, oy, oz) for the next step.
 struct SplatPosLdmm {
@@ -60,7 +68,8 @@ struct SplatPosLdmm {
   float sx, sy, sz;
   float *ox, *oy, *oz;
   __device__ __forceinline__ float3 at(int i) const {
-    const float a = gx[i], b = gy[i], c = gz[i];
+    const float3 g = voxel_or(gx, gy, gz, i, d);
+    const float a = g.x, b = g.y, c = g.z;
     const float3 o = trilerp3g<AWK_BG_PARTIAL_ZERO>(vx, vy, vz, d, a, b, c);
     const float x = o.x / -sx + a, y = o.y / -sy + b, z = o.z / -sz + c;
     ox[i] = x;
