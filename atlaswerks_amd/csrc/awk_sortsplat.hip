@@ -556,10 +556,40 @@ k_base_sum(float *__restrict__ dst, const unsigned *__restrict__ ids, const floa
   dst[((size_t)Z * h + Y) * w + X] = staged ? merge(sid, spos, true) : merge(ids, pos, false);
 }
 
+// Scratch of a sort of M pairs: two key / value buffers, histogram, chunk sums, each at
+// a multiple of 16 bytes from the scratch's start (k_radix_hist loads keys 16 bytes at a
+// time), whatever M is.
+struct SortScratch {
+  long long M, nh, nchunks;
+  struct Bufs {
+    unsigned *ka, *kb;
+    float *va, *vb;
+    unsigned *hist, *sums;
+  };
+  explicit SortScratch(long long m) : M(m) {
+    nh = 2LL * kRadix * ((M + kTile - 1) / kTile);  // room for a 9-bit pass
+    nchunks = (nh + kScanChunk - 1) / kScanChunk;
+  }
+  static size_t up16(size_t bytes) { return (bytes + 15) / 16 * 16; }
+  size_t bytes() const {
+    return (4 * up16(4 * (size_t)M) + up16(4 * (size_t)nh) + 4 * (size_t)nchunks + 255) / 256 * 256;
+  }
+  Bufs at(char *p) const {
+    const size_t m = up16(4 * (size_t)M);
+    Bufs b;
+    b.ka = reinterpret_cast<unsigned *>(p);
+    b.kb = reinterpret_cast<unsigned *>(p + m);
+    b.va = reinterpret_cast<float *>(p + 2 * m);
+    b.vb = reinterpret_cast<float *>(p + 3 * m);
+    b.hist = reinterpret_cast<unsigned *>(p + 4 * m);
+    b.sums = reinterpret_cast<unsigned *>(p + 4 * m + up16(4 * (size_t)nh));
+    return b;
+  }
+};
+
 // Stable radix sort of M (key, value) pairs of `bits` key bits, between the two
 // buffer pairs; the sorted pairs are in (ka, va) on return.
-static awk_status radix_sort(unsigned *&ka, unsigned *&kb, float *&va, float *&vb, long long M, int bits,
-                             unsigned *hist, unsigned *sums, hipStream_t s) {
+static awk_status radix_sort(SortScratch::Bufs &q, long long M, int bits, hipStream_t s) {
   // 8-bit passes; 9 remaining bits go in one pass (a power-of-two volume's keys,
   // cells 0 .. N - 1 and the outside-volume cell N, need one bit past a multiple of 8)
   const int ntiles = (int)((M + kTile - 1) / kTile);
@@ -567,22 +597,22 @@ static awk_status radix_sort(unsigned *&ka, unsigned *&kb, float *&va, float *&v
     const int b = rem == 9 ? 9 : std::min(rem, kRadixBits);
     const long long nh = (long long)(b == 9 ? 2 * kRadix : kRadix) * ntiles;
     const int nchunks = (int)((nh + kScanChunk - 1) / kScanChunk);
-    if (b == 9) AWK_LAUNCH(k_radix_hist<9>, dim3(ntiles), dim3(kSortBlock), 0, s, ka, M, shift, ntiles, hist);
-    else AWK_LAUNCH(k_radix_hist<8>, dim3(ntiles), dim3(kSortBlock), 0, s, ka, M, shift, ntiles, hist);
-    AWK_LAUNCH(k_scan_reduce, dim3(nchunks), dim3(kSortBlock), 0, s, hist, nh, sums);
-    AWK_LAUNCH(k_scan_top, dim3(1), dim3(kSortBlock), 0, s, sums, nchunks);
-    AWK_LAUNCH(k_scan_down, dim3(nchunks), dim3(kSortBlock), 0, s, hist, nh, sums);
+    if (b == 9) AWK_LAUNCH(k_radix_hist<9>, dim3(ntiles), dim3(kSortBlock), 0, s, q.ka, M, shift, ntiles, q.hist);
+    else AWK_LAUNCH(k_radix_hist<8>, dim3(ntiles), dim3(kSortBlock), 0, s, q.ka, M, shift, ntiles, q.hist);
+    AWK_LAUNCH(k_scan_reduce, dim3(nchunks), dim3(kSortBlock), 0, s, q.hist, nh, q.sums);
+    AWK_LAUNCH(k_scan_top, dim3(1), dim3(kSortBlock), 0, s, q.sums, nchunks);
+    AWK_LAUNCH(k_scan_down, dim3(nchunks), dim3(kSortBlock), 0, s, q.hist, nh, q.sums);
     if (b == 9)
-      AWK_LAUNCH(k_radix_scatter<9>, dim3(ntiles), dim3(kSortBlock), 0, s, ka, va, kb, vb, M, shift,
-                 ntiles, hist);
+      AWK_LAUNCH(k_radix_scatter<9>, dim3(ntiles), dim3(kSortBlock), 0, s, q.ka, q.va, q.kb, q.vb, M, shift,
+                 ntiles, q.hist);
     else
-      AWK_LAUNCH(k_radix_scatter<8>, dim3(ntiles), dim3(kSortBlock), 0, s, ka, va, kb, vb, M, shift,
-                 ntiles, hist);
+      AWK_LAUNCH(k_radix_scatter<8>, dim3(ntiles), dim3(kSortBlock), 0, s, q.ka, q.va, q.kb, q.vb, M, shift,
+                 ntiles, q.hist);
     AWK_LAUNCH_CHECK("radix pass");
     shift += b;
     rem -= b;
-    std::swap(ka, kb);
-    std::swap(va, vb);
+    std::swap(q.ka, q.kb);
+    std::swap(q.va, q.vb);
   }
   return AWK_OK;
 }
@@ -593,21 +623,16 @@ static int key_bits(long long most) {  // keys 0 .. most
   return bits;
 }
 
-// Scratch of a sort of M pairs: two key / value buffers, histogram, chunk sums.
-struct SortScratch {
-  long long M, nh, nchunks;
-  explicit SortScratch(long long m) : M(m) {
-    nh = 2LL * kRadix * ((M + kTile - 1) / kTile);  // room for a 9-bit pass
-    nchunks = (nh + kScanChunk - 1) / kScanChunk;
-  }
-  size_t bytes() const { return (16 * (size_t)M + 4 * (size_t)nh + 4 * (size_t)nchunks + 255) / 256 * 256; }
-};
-
 static long long base_cells(int nx, int ny, int nz) { return (long long)(nx + 1) * (ny + 1) * (nz + 1); }
+
+// Scratch by base cell: the positions, the cells' runs, then the sort's.
+static size_t base_sort_offset(long long N, long long cells) {
+  return SortScratch::up16(16 * (size_t)N + 8 * (size_t)cells);
+}
 
 size_t splat_sorted_scratch_bytes(int nx, int ny, int nz) {
   const long long N = (long long)nx * ny * nz;
-  return SortScratch(N).bytes() + 16 * (size_t)N + 8 * (size_t)base_cells(nx, ny, nz);
+  return base_sort_offset(N, base_cells(nx, ny, nz)) + SortScratch(N).bytes();
 }
 
 // The sorted pairs themselves are wanted: all 8N of them are made and sorted.
@@ -619,22 +644,18 @@ static awk_status splat_pairs(float *dst, const float *src, const float *vx, con
   const SortScratch sc(M);
   char *scratch = nullptr;
   AWK_HIP(scratch_alloc(&scratch, sc.bytes(), s));
-  unsigned *ka = reinterpret_cast<unsigned *>(scratch);
-  unsigned *kb = ka + M;
-  float *va = reinterpret_cast<float *>(kb + M);
-  float *vb = va + M;
-  unsigned *hist = reinterpret_cast<unsigned *>(vb + M);
+  SortScratch::Bufs q = sc.at(scratch);
   AWK_LAUNCH(k_create_index, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s,
-             reinterpret_cast<uint4 *>(ka), reinterpret_cast<float4 *>(va), src, vx, vy, vz, nx, ny,
+             reinterpret_cast<uint4 *>(q.ka), reinterpret_cast<float4 *>(q.va), src, vx, vy, vz, nx, ny,
              nz, truncate, absolute);
   AWK_LAUNCH_CHECK("k_create_index");
-  if (awk_status st = radix_sort(ka, kb, va, vb, M, key_bits(N), hist, hist + sc.nh, s)) return st;
+  if (awk_status st = radix_sort(q, M, key_bits(N), s)) return st;
   AWK_LAUNCH(k_zero_image, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, dst, N);
-  AWK_LAUNCH(k_segment_sum, dim3((unsigned)((M + kSegTile - 1) / kSegTile)), dim3(256), 0, s, ka, va, M,
+  AWK_LAUNCH(k_segment_sum, dim3((unsigned)((M + kSegTile - 1) / kSegTile)), dim3(256), 0, s, q.ka, q.va, M,
              (unsigned)N, dst);
   AWK_LAUNCH_CHECK("k_segment_sum");
-  if (keys_out) AWK_HIP(hipMemcpyAsync(keys_out, ka, (size_t)M * 4, hipMemcpyDeviceToDevice, s));
-  if (vals_out) AWK_HIP(hipMemcpyAsync(vals_out, va, (size_t)M * 4, hipMemcpyDeviceToDevice, s));
+  if (keys_out) AWK_HIP(hipMemcpyAsync(keys_out, q.ka, (size_t)M * 4, hipMemcpyDeviceToDevice, s));
+  if (vals_out) AWK_HIP(hipMemcpyAsync(vals_out, q.va, (size_t)M * 4, hipMemcpyDeviceToDevice, s));
   AWK_HIP(scratch_free(scratch, s));
   return AWK_OK;
 }
@@ -652,19 +673,16 @@ awk_status launch_splat_sorted(float *dst, const float *src, const float *vx, co
   if (!scratch) AWK_HIP(scratch_alloc(&scratch, splat_sorted_scratch_bytes(nx, ny, nz), s));
   float4 *pos = reinterpret_cast<float4 *>(scratch);
   uint2 *ranges = reinterpret_cast<uint2 *>(pos + N);
-  unsigned *ka = reinterpret_cast<unsigned *>(ranges + cells);
-  unsigned *kb = ka + N;
-  float *va = reinterpret_cast<float *>(kb + N);  // voxel numbers: moved as bits
-  float *vb = va + N;
-  unsigned *hist = reinterpret_cast<unsigned *>(vb + N);
+  SortScratch::Bufs q = sc.at(scratch + base_sort_offset(N, cells));
+  // the values are voxel numbers, moved as bits
   const unsigned gN = (unsigned)((N + 255) / 256), gc = (unsigned)((cells + 255) / 256);
-  AWK_LAUNCH(k_base_index, dim3(gc), dim3(256), 0, s, ka, reinterpret_cast<unsigned *>(va), src, vx, vy, vz, nx, ny,
+  AWK_LAUNCH(k_base_index, dim3(gc), dim3(256), 0, s, q.ka, reinterpret_cast<unsigned *>(q.va), src, vx, vy, vz, nx, ny,
              nz, (unsigned)cells, truncate, absolute, ranges);
   AWK_LAUNCH_CHECK("k_base_index");
-  if (awk_status st = radix_sort(ka, kb, va, vb, N, key_bits(cells), hist, hist + sc.nh, s)) return st;
-  AWK_LAUNCH(k_base_runs, dim3(gN), dim3(256), 0, s, ka, reinterpret_cast<unsigned *>(va), src, vx, vy, vz, nx, ny,
+  if (awk_status st = radix_sort(q, N, key_bits(cells), s)) return st;
+  AWK_LAUNCH(k_base_runs, dim3(gN), dim3(256), 0, s, q.ka, reinterpret_cast<unsigned *>(q.va), src, vx, vy, vz, nx, ny,
              nz, (unsigned)cells, truncate, absolute, ranges, pos);
-  AWK_LAUNCH(k_base_sum, dim3(grid_for((long long)ny * nz * ((nx + kSumBlock - 1) / kSumBlock), 1)), dim3(kSumBlock), 0, s, dst, reinterpret_cast<unsigned *>(va), pos, ranges,
+  AWK_LAUNCH(k_base_sum, dim3(grid_for((long long)ny * nz * ((nx + kSumBlock - 1) / kSumBlock), 1)), dim3(kSumBlock), 0, s, dst, reinterpret_cast<unsigned *>(q.va), pos, ranges,
              nx, ny, nz);
   AWK_LAUNCH_CHECK("k_base_sum");
   if (!work) AWK_HIP(scratch_free(scratch, s));

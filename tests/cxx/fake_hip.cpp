@@ -1,0 +1,212 @@
+// A HIP runtime that only keeps books: what libawk_hip.so allocates, launches and
+// records, in order, on memory that does not exist.  Loaded ahead of the real runtime
+// (tests/fake_hip.py), it shows on the CPU what the host code does at an allocation or
+// a launch that fails, under capture, and with which pointers and grids it launches.
+#include <hip/hip_runtime_api.h>
+
+#include <cstdint>
+#include <cstring>
+#include <map>
+#include <string>
+#include <vector>
+
+namespace {
+struct Pool {
+  std::multimap<size_t, uintptr_t> idle;
+};
+struct Block {
+  size_t size;
+  Pool *pool;  // null: hipMalloc, or the runtime's own pool (which keeps nothing)
+};
+size_t g_budget = SIZE_MAX, g_used = 0;
+uintptr_t g_next = 0x100000000ull;
+std::map<uintptr_t, Block> g_live;
+std::map<const void *, std::string> g_names;
+std::string g_log, g_fail_name;
+int g_fail_skip = 0;
+bool g_capturing = false;
+hipError_t g_last = hipSuccess;
+std::vector<void *> g_call;
+dim3 g_grid, g_block;
+size_t g_shmem;
+hipStream_t g_stream;
+uintptr_t g_handle = 0x1000;
+
+hipError_t ret(hipError_t e) {
+  if (e != hipSuccess) g_last = e;
+  return e;
+}
+void note(const std::string &s) { g_log += s + "\n"; }
+std::string num(uintptr_t v) { return std::to_string((unsigned long long)v); }
+template <class T>
+std::string num(T *p) {
+  return num(reinterpret_cast<uintptr_t>(p));
+}
+
+hipError_t take(void **p, size_t n, Pool *pool) {
+  if (pool) {
+    auto it = pool->idle.lower_bound(n);
+    if (it != pool->idle.end()) {
+      *p = reinterpret_cast<void *>(it->second);
+      g_live[it->second] = Block{it->first, pool};
+      pool->idle.erase(it);
+      return hipSuccess;
+    }
+  }
+  if (n > g_budget - g_used) return ret(hipErrorOutOfMemory);
+  g_used += n;
+  *p = reinterpret_cast<void *>(g_next);
+  g_live[g_next] = Block{n, pool};
+  g_next += (n + 0xffff) / 0x10000 * 0x10000 + 0x10000;
+  return hipSuccess;
+}
+hipError_t give(void *p) {
+  if (!p) return hipSuccess;
+  auto it = g_live.find(reinterpret_cast<uintptr_t>(p));
+  if (it == g_live.end()) return ret(hipErrorInvalidValue);
+  if (it->second.pool) it->second.pool->idle.emplace(it->second.size, it->first);
+  else g_used -= it->second.size;
+  g_live.erase(it);
+  return hipSuccess;
+}
+hipError_t launch(const void *f, dim3 g, dim3 b, void **args, hipStream_t s) {
+  const std::string &name = g_names[f];
+  if (!g_fail_name.empty() && name.find(g_fail_name) != std::string::npos && g_fail_skip-- == 0) {
+    note("failed " + name);
+    return ret(hipErrorLaunchFailure);
+  }
+  // the documented limit: fewer than 2^32 threads along an axis
+  if ((unsigned long long)g.x * b.x >> 32 || (unsigned long long)g.y * b.y >> 32 || (unsigned long long)g.z * b.z >> 32)
+    return ret(hipErrorInvalidConfiguration);
+  note("launch " + name + " " + num((uintptr_t)g.x) + " " + num((uintptr_t)g.y) + " " + num((uintptr_t)b.x) + " " +
+       num(s) + " " + num(*static_cast<uintptr_t *>(args[0])));
+  return hipSuccess;
+}
+}  // namespace
+
+extern "C" {
+
+// ---- the test's side
+void fake_budget(unsigned long long bytes) { g_budget = bytes; }
+unsigned long long fake_used() { return g_used; }
+void fake_fail(const char *name, int skip) {
+  g_fail_name = name;
+  g_fail_skip = skip;
+}
+void fake_capture(int on) { g_capturing = on != 0; }
+const char *fake_log() { return g_log.c_str(); }
+void fake_clear() { g_log.clear(); }
+
+// ---- the runtime's side
+void **__hipRegisterFatBinary(const void *) {
+  static void *module = nullptr;
+  return &module;
+}
+void __hipUnregisterFatBinary(void **) {}
+void __hipRegisterFunction(void **, const void *host, char *, const char *name, unsigned, void *, void *, dim3 *, dim3 *,
+                           int *) {
+  g_names[host] = name;
+}
+void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t shmem, hipStream_t s) {
+  g_grid = g;
+  g_block = b;
+  g_shmem = shmem;
+  g_stream = s;
+  return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *shmem, hipStream_t *s) {
+  *g = g_grid;
+  *b = g_block;
+  *shmem = g_shmem;
+  *s = g_stream;
+  return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **args, size_t, hipStream_t s) {
+  return launch(f, g, b, args, s);
+}
+hipError_t hipExtLaunchKernel(const void *f, dim3 g, dim3 b, void **args, size_t, hipStream_t s, hipEvent_t, hipEvent_t,
+                              int) {
+  return launch(f, g, b, args, s);
+}
+hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
+hipError_t hipGetDevice(int *d) {
+  *d = 0;
+  return hipSuccess;
+}
+hipError_t hipGetLastError() {
+  const hipError_t e = g_last;
+  g_last = hipSuccess;
+  return e;
+}
+const char *hipGetErrorString(hipError_t) { return "fake"; }
+hipError_t hipDeviceSynchronize() {
+  note("sync");
+  return g_capturing ? ret(hipErrorStreamCaptureUnsupported) : hipSuccess;
+}
+hipError_t hipMalloc(void **p, size_t n) {
+  if (g_capturing) return ret(hipErrorStreamCaptureUnsupported);
+  return take(p, n, nullptr);
+}
+hipError_t hipFree(void *p) { return give(p); }
+hipError_t hipMallocAsync(void **p, size_t n, hipStream_t) { return take(p, n, nullptr); }
+hipError_t hipFreeAsync(void *p, hipStream_t) { return give(p); }
+hipError_t hipMemPoolCreate(hipMemPool_t *p, const hipMemPoolProps *) {
+  *p = reinterpret_cast<hipMemPool_t>(new Pool());
+  return hipSuccess;
+}
+hipError_t hipMemPoolSetAttribute(hipMemPool_t, hipMemPoolAttr, void *) { return hipSuccess; }
+hipError_t hipMallocFromPoolAsync(void **p, size_t n, hipMemPool_t pool, hipStream_t) {
+  return take(p, n, reinterpret_cast<Pool *>(pool));
+}
+hipError_t hipMemPoolTrimTo(hipMemPool_t pool, size_t) {  // (to zero: all that is asked here)
+  Pool *q = reinterpret_cast<Pool *>(pool);
+  for (const auto &b : q->idle) g_used -= b.first;
+  q->idle.clear();
+  return hipSuccess;
+}
+hipError_t hipMemcpy(void *dst, const void *, size_t n, hipMemcpyKind k) {
+  if (k == hipMemcpyDeviceToHost) std::memset(dst, 0, n);
+  return g_capturing ? ret(hipErrorStreamCaptureUnsupported) : hipSuccess;
+}
+hipError_t hipMemcpyAsync(void *dst, const void *, size_t n, hipMemcpyKind k, hipStream_t) {
+  if (k == hipMemcpyDeviceToHost) std::memset(dst, 0, n);
+  return hipSuccess;
+}
+hipError_t hipMemset(void *, int, size_t) { return g_capturing ? ret(hipErrorStreamCaptureUnsupported) : hipSuccess; }
+hipError_t hipMemsetAsync(void *, int, size_t, hipStream_t) { return hipSuccess; }
+hipError_t hipGetSymbolAddress(void **p, const void *) {
+  *p = reinterpret_cast<void *>(uintptr_t{0x10000});
+  return hipSuccess;
+}
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) {
+  *s = reinterpret_cast<hipStream_t>(g_handle += 16);
+  return hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *c) {
+  *c = g_capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+  return hipSuccess;
+}
+hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
+  note("wait " + num(s) + " " + num(e));
+  return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
+  *e = reinterpret_cast<hipEvent_t>(g_handle += 16);
+  return hipSuccess;
+}
+hipError_t hipEventCreate(hipEvent_t *e) { return hipEventCreateWithFlags(e, 0); }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+  note("record " + num(e) + " " + num(s));
+  return hipSuccess;
+}
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) {
+  *ms = 0.f;
+  return hipSuccess;
+}
+
+}  // extern "C"
