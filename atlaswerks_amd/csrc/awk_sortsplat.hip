@@ -449,10 +449,11 @@ k_base_runs(const unsigned *__restrict__ keys, const unsigned *__restrict__ ids,
   pos[e] = make_float4(1.f - (p.x - xi), 1.f - (p.y - yi), 1.f - (p.z - zi), p.w);
 }
 
-// One block per 128 cells of a row.  The runs of the row's base cells are four
-// consecutive stretches of the sorted voxels (its own row and the three before it in y
-// and z), staged in LDS with coalesced loads when they fit: the merge's loads depend
-// on each other (128^3: 134 us from memory, 82 staged and without a branch per run).
+// One block per 128 consecutive cells (of one row, or of several short ones).  The runs
+// of their base cells are four stretches of the sorted voxels that ascend with the cell
+// (its own base row and the three before it in y and z), staged in LDS with coalesced
+// loads when they fit: the merge's loads depend on each other (128^3: 134 us from
+// memory, 82 staged and without a branch per run).
 constexpr int kSumBlock = 128, kSumCap = 6 * kSumBlock;
 __global__ void __launch_bounds__(kSumBlock)
 k_base_sum(float *__restrict__ dst, const unsigned *__restrict__ ids, const float4 *__restrict__ pos,
@@ -461,11 +462,27 @@ k_base_sum(float *__restrict__ dst, const unsigned *__restrict__ ids, const floa
   constexpr unsigned kNone = 0xffffffffu;
   __shared__ unsigned lo[4], hi[4], sid[kSumCap];
   __shared__ float4 spos[kSumCap];
-  const int nseg = (w + kSumBlock - 1) / kSumBlock;
-  const int b = (int)xcd_block();
-  if (b >= h * l * nseg) return;
-  const int row = b / nseg, Y = row % h, Z = row / h;
-  const int X = (b - row * nseg) * kSumBlock + (int)threadIdx.x, lane = threadIdx.x & 63;
+  const int N = w * h * l, i0 = (int)xcd_block() * kSumBlock, lane = threadIdx.x & 63;
+  if (i0 >= N) return;
+  // cell i0 + thread: from the block's first cell, whose divisions are the block's
+  const int row0 = i0 / w, Z0 = row0 / h;
+  int X = i0 - row0 * w + (int)threadIdx.x, Y = row0 - Z0 * h, Z = Z0;
+  if (w >= kSumBlock) {
+    if (X >= w) {
+      X -= w;
+      ++Y;
+    }
+    if (Y >= h) {
+      Y -= h;
+      ++Z;
+    }
+  } else {
+    Y += X / w;
+    X %= w;
+    Z += Y / h;
+    Y %= h;
+  }
+  const bool live = i0 + (int)threadIdx.x < N;
   if (threadIdx.x < 4) {
     lo[threadIdx.x] = kNone;
     hi[threadIdx.x] = 0u;
@@ -473,13 +490,13 @@ k_base_sum(float *__restrict__ dst, const unsigned *__restrict__ ids, const floa
   uint2 run[8];  // corner c = 4 (z below) + 2 (y below) + (x below)
 #pragma unroll
   for (int c = 0; c < 8; ++c)
-    run[c] = X < w ? ranges[((unsigned)(Z + 1 - (c >> 2)) * (h + 1) + (Y + 1 - ((c >> 1) & 1))) * (w + 1) +
-                            (X + 1 - (c & 1))]
-                   : make_uint2(0u, 0u);
+    run[c] = live ? ranges[((unsigned)(Z + 1 - (c >> 2)) * (h + 1) + (Y + 1 - ((c >> 1) & 1))) * (w + 1) +
+                          (X + 1 - (c & 1))]
+                  : make_uint2(0u, 0u);
   __syncthreads();
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    // runs ascend with x: the stretch is from the first lane's first voxel to the last's last
+    // runs ascend with the cell: the stretch is from the first lane's first voxel to the last's last
     const bool n1 = run[2 * r + 1].x < run[2 * r + 1].y, n0 = run[2 * r].x < run[2 * r].y;
     const unsigned f = n1 ? run[2 * r + 1].x : run[2 * r].x, e = n0 ? run[2 * r].y : run[2 * r + 1].y;
     const unsigned long long any = __ballot(n0 || n1);
@@ -510,7 +527,7 @@ k_base_sum(float *__restrict__ dst, const unsigned *__restrict__ ids, const floa
       }
     __syncthreads();
   }
-  if (X >= w) return;
+  if (!live) return;
   auto merge = [&](const unsigned *id, const float4 *at, bool moved) {
     float acc = 0.f;
 #pragma unroll
@@ -553,7 +570,7 @@ k_base_sum(float *__restrict__ dst, const unsigned *__restrict__ ids, const floa
     }
     return acc;
   };
-  dst[((size_t)Z * h + Y) * w + X] = staged ? merge(sid, spos, true) : merge(ids, pos, false);
+  dst[i0 + threadIdx.x] = staged ? merge(sid, spos, true) : merge(ids, pos, false);
 }
 
 // Scratch of a sort of M pairs: two key / value buffers, histogram, chunk sums, each at
@@ -682,8 +699,8 @@ awk_status launch_splat_sorted(float *dst, const float *src, const float *vx, co
   if (awk_status st = radix_sort(q, N, key_bits(cells), s)) return st;
   AWK_LAUNCH(k_base_runs, dim3(gN), dim3(256), 0, s, q.ka, reinterpret_cast<unsigned *>(q.va), src, vx, vy, vz, nx, ny,
              nz, (unsigned)cells, truncate, absolute, ranges, pos);
-  AWK_LAUNCH(k_base_sum, dim3(grid_for((long long)ny * nz * ((nx + kSumBlock - 1) / kSumBlock), 1)), dim3(kSumBlock), 0, s, dst, reinterpret_cast<unsigned *>(q.va), pos, ranges,
-             nx, ny, nz);
+  AWK_LAUNCH(k_base_sum, dim3(grid_for(N, kSumBlock)), dim3(kSumBlock), 0, s, dst,
+             reinterpret_cast<unsigned *>(q.va), pos, ranges, nx, ny, nz);
   AWK_LAUNCH_CHECK("k_base_sum");
   if (!work) AWK_HIP(scratch_free(scratch, s));
   return AWK_OK;

@@ -253,3 +253,29 @@ def test_splat_sorted_without_pairs_bit_exact(kind, trunc):
     hfield.splat_sorted(a, S, V, reference_truncation=trunc, keys=keys, vals=vals)
     hfield.splat_sorted(b, S, V, reference_truncation=trunc)
     np.testing.assert_array_equal(a.cpu().numpy(), b.cpu().numpy())
+
+
+# blocks of 128 consecutive cells: rows of one, two, just under / at / over one and two
+# blocks, many short rows to a block (whole planes among them), blocks across planes
+@pytest.mark.parametrize("shape", [(3, 5, 127), (3, 5, 128), (3, 5, 129), (4, 3, 200), (2, 3, 300), (3, 40, 1),
+                                   (70, 3, 2), (400, 1, 1), (5, 1, 130), (1, 1, 257), (9, 17, 7)])
+@pytest.mark.parametrize("disp", [0.7, 6.0])
+def test_splat_sorted_row_lengths_bit_exact(shape, disp):
+    """The base-cell sums against the sums over the sorted pairs, bit for bit, with fields
+    that leave a block's voxels in its staged stretches (0.7) and that pile them up past
+    what is staged (6, on a field contracted towards the middle)."""
+    import torch
+    from atlaswerks_amd import hfield
+    nz, ny, nx = shape
+    print("splat_sorted rows", shape, disp, flush=True)
+    rng = np.random.default_rng(nx)
+    src = rng.standard_normal(shape).astype(np.float32)
+    v = rng.uniform(-disp, disp, (3,) + shape).astype(np.float32)
+    if disp > 1:
+        v -= (0.9 * (synth.identity(shape) - np.array([nx, ny, nz], np.float32)[:, None, None, None] / 2)).astype(np.float32)
+    S, V = torch.from_numpy(src).cuda(), torch.from_numpy(v).cuda()
+    vals = torch.empty(8 * src.size, dtype=torch.float32, device="cuda")
+    a, b = torch.full_like(S, 7.0), torch.full_like(S, -3.0)
+    hfield.splat_sorted(a, S, V, vals=vals)
+    hfield.splat_sorted(b, S, V)
+    np.testing.assert_array_equal(a.cpu().numpy(), b.cpu().numpy())

@@ -31,3 +31,15 @@ print(len(rows), sum(int(r[-1]) %% 16 != 0 for r in rows))
 """ % (size,))
     n, bad = map(int, out.split())
     assert n >= 4 and bad == 0, (n, bad)
+
+
+@pytest.mark.parametrize("size", [(1, 1, 1 << 26), (1, 1 << 13, 1 << 13), (2, 4096, 4096), (1, 1, (1 << 28) - 1)])
+def test_sorted_splat_of_short_rows_launches(fake, size):
+    """Volumes of many short rows: every launch stays below 2^32 threads (a block per row
+    of one or two voxels does not)."""
+    fake_hip.run(fake, """
+p = P(0x4000)
+rc = lib.awk_splat_sorted(p, p, p, p, p, *%r, 1, None, None, None)
+assert rc == 0, lib.awk_last_error()
+assert any("k_base_sum" in r[1] for r in log("launch"))
+""" % (size,))
