@@ -462,12 +462,12 @@ awk_status awk_atlas_create(awk_atlas_t *out, int nx, int ny, int nz, float spx,
   const int nblk = fk_xblocks(a->k);
   hipError_t e = hipSuccess;
   const size_t ns = (size_t)n_subjects;
-  if (e == hipSuccess) e = hipMalloc(&a->hslab[0], ns * 3 * N * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&a->hslab[1], ns * 3 * N * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&a->idef_slab, ns * N * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&a->step_slab, ns * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&a->prev_slab, ns * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&a->have_prev_slab, ns * sizeof(int));
+  if (e == hipSuccess) e = device_malloc(&a->hslab[0], ns * 3 * N * sizeof(float));
+  if (e == hipSuccess) e = device_malloc(&a->hslab[1], ns * 3 * N * sizeof(float));
+  if (e == hipSuccess) e = device_malloc(&a->idef_slab, ns * N * sizeof(float));
+  if (e == hipSuccess) e = device_malloc(&a->step_slab, ns * sizeof(float));
+  if (e == hipSuccess) e = device_malloc(&a->prev_slab, ns * sizeof(double));
+  if (e == hipSuccess) e = device_malloc(&a->have_prev_slab, ns * sizeof(int));
   if (e == hipSuccess) e = hipMemset(a->step_slab, 0, ns * sizeof(float));
   if (e == hipSuccess) e = hipMemset(a->have_prev_slab, 0, ns * sizeof(int));
   if (e == hipSuccess)
@@ -488,24 +488,24 @@ awk_status awk_atlas_create(awk_atlas_t *out, int nx, int ny, int nz, float spx,
   {
     const size_t sb = 3 * a->k.spec_plane() * sizeof(float2);
     size_t cap = std::min(ns, std::max<size_t>(1, (8ull << 30) / sb));
-    if (e == hipSuccess) e = hipMalloc(&a->bspec, cap * sb);
-    if (e == hipSuccess) e = hipMalloc(&a->bpart, cap * (size_t)nblk * sizeof(double));
+    if (e == hipSuccess) e = device_malloc(&a->bspec, cap * sb);
+    if (e == hipSuccess) e = device_malloc(&a->bpart, cap * (size_t)nblk * sizeof(double));
     a->batch_cap = (int)cap;
     a->batch = (int)std::min(cap, std::max<size_t>(1, (128ull << 20) / sb));
   }
-  if (e == hipSuccess) e = hipMalloc(&a->mean, N * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc((void **)&a->idef_tab, n_subjects * sizeof(float *));
-  if (e == hipSuccess) e = hipMalloc(&a->w_dev, n_subjects * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&a->src_tab, n_subjects * sizeof(AtlasSrc));
-  if (e == hipSuccess) e = hipMalloc(&a->esub, n_subjects * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&a->partials, (size_t)nblk * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&a->maxpart, (size_t)nblk * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&a->hist, kHistCap * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&a->cursor, sizeof(int));
+  if (e == hipSuccess) e = device_malloc(&a->mean, N * sizeof(float));
+  if (e == hipSuccess) e = device_malloc((void **)&a->idef_tab, n_subjects * sizeof(float *));
+  if (e == hipSuccess) e = device_malloc(&a->w_dev, n_subjects * sizeof(float));
+  if (e == hipSuccess) e = device_malloc(&a->src_tab, n_subjects * sizeof(AtlasSrc));
+  if (e == hipSuccess) e = device_malloc(&a->esub, n_subjects * sizeof(double));
+  if (e == hipSuccess) e = device_malloc(&a->partials, (size_t)nblk * sizeof(double));
+  if (e == hipSuccess) e = device_malloc(&a->maxpart, (size_t)nblk * sizeof(float));
+  if (e == hipSuccess) e = device_malloc(&a->hist, kHistCap * sizeof(double));
+  if (e == hipSuccess) e = device_malloc(&a->cursor, sizeof(int));
   if (e == hipSuccess) e = hipMemset(a->cursor, 0, sizeof(int));
-  if (e == hipSuccess) e = hipMalloc(&a->flags, sizeof(unsigned));
+  if (e == hipSuccess) e = device_malloc(&a->flags, sizeof(unsigned));
   if (e == hipSuccess) e = hipMemset(a->flags, 0, sizeof(unsigned));
-  if (e == hipSuccess) e = hipMalloc(&a->vbuf, 3 * N * sizeof(float));
+  if (e == hipSuccess) e = device_malloc(&a->vbuf, 3 * N * sizeof(float));
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&a->as, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&a->ev_in, hipEventDisableTiming);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&a->ev_out, hipEventDisableTiming);
@@ -517,10 +517,10 @@ awk_status awk_atlas_create(awk_atlas_t *out, int nx, int ny, int nz, float spx,
     L.k = a->k;  // shares the operator tables
     L.k.spec = nullptr;
     L.k.eig = nullptr;
-    e = hipMalloc(&L.k.spec, 3 * a->k.spec_plane() * sizeof(float2));
-    if (e == hipSuccess) e = hipMalloc(&L.partials, (size_t)nblk * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc(&L.maxpart, (size_t)nblk * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc(&L.vbuf, 3 * N * sizeof(float));
+    e = device_malloc(&L.k.spec, 3 * a->k.spec_plane() * sizeof(float2));
+    if (e == hipSuccess) e = device_malloc(&L.partials, (size_t)nblk * sizeof(double));
+    if (e == hipSuccess) e = device_malloc(&L.maxpart, (size_t)nblk * sizeof(float));
+    if (e == hipSuccess) e = device_malloc(&L.vbuf, 3 * N * sizeof(float));
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&L.st, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&L.join, hipEventDisableTiming);
   }
@@ -595,7 +595,7 @@ awk_status awk_atlas_set_subject_inverse(awk_atlas_t a, int s, const float *cons
     return fail(AWK_ERR_INVALID, "awk_atlas_set_subject_inverse: the subject's image must be on the template grid");
   const size_t N = (size_t)a->nx * a->ny * a->nz;
   for (int b = 0; b < 2; ++b)
-    if (!sb.hinv[b]) AWK_HIP(hipMalloc(&sb.hinv[b], 3 * N * sizeof(float)));
+    if (!sb.hinv[b]) AWK_HIP(device_malloc(&sb.hinv[b], 3 * N * sizeof(float)));
   hipStream_t cs = as_stream(stream);
   for (int c = 0; c < 3; ++c)
     AWK_HIP(hipMemcpyAsync(sb.hinv[a->cur] + c * N, hinv0[c], N * sizeof(float), hipMemcpyDeviceToDevice, cs));

@@ -87,8 +87,14 @@ inline hipError_t load_scalar_sync(T *host, const T *dev, hipStream_t s) {
   return e;
 }
 
-// Device memory kept between handles, and stream-ordered scratch of one call
-// (awk_mem.hip).  dev_free waits for the device and takes null pointers.
+// Device memory (awk_mem.hip): plain (device_malloc, released by hipFree), kept between
+// handles (dev_alloc, released by dev_free, which waits for the device and takes null
+// pointers), and stream-ordered scratch of one call.
+hipError_t device_malloc_bytes(void **p, size_t bytes);
+template <class T>
+inline hipError_t device_malloc(T **p, size_t bytes) {
+  return device_malloc_bytes(reinterpret_cast<void **>(p), bytes);
+}
 hipError_t dev_alloc_bytes(void **p, size_t bytes);
 template <class T>
 inline hipError_t dev_alloc(T **p, size_t bytes) {

@@ -206,20 +206,20 @@ awk_status awk_ldmm_atlas_create(awk_ldmm_atlas_t *out, int nx, int ny, int nz, 
   a->w_host.assign(S, 0.f);
   hipError_t e = hipSuccess;
   if (!st) {
-    e = hipMalloc(&a->mean, N * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc(&a->w, S * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc(&a->jt0, S * sizeof(float *));
-    if (e == hipSuccess) e = hipMalloc(&a->jd0, S * sizeof(float *));
-    if (e == hipSuccess) e = hipMalloc(&a->esub, 3 * (size_t)S * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc(&a->energy, 3 * sizeof(double));
+    e = device_malloc(&a->mean, N * sizeof(float));
+    if (e == hipSuccess) e = device_malloc(&a->w, S * sizeof(float));
+    if (e == hipSuccess) e = device_malloc(&a->jt0, S * sizeof(float *));
+    if (e == hipSuccess) e = device_malloc(&a->jd0, S * sizeof(float *));
+    if (e == hipSuccess) e = device_malloc(&a->esub, 3 * (size_t)S * sizeof(double));
+    if (e == hipSuccess) e = device_malloc(&a->energy, 3 * sizeof(double));
     std::vector<const float *> p0(S), p1(S);
     for (int k = 0; k < S && e == hipSuccess; ++k) {
       LaSubject &sb = a->subs[k];
       sb.v.assign(3 * (size_t)n_time_steps, nullptr);
-      e = hipMalloc(&sb.I, N * sizeof(float));
-      if (e == hipSuccess) e = hipMalloc(&sb.jt, (size_t)n_time_steps * N * sizeof(float));
-      if (e == hipSuccess) e = hipMalloc(&sb.jd, (size_t)n_time_steps * N * sizeof(float));
-      if (e == hipSuccess) e = hipMalloc(&sb.step, sizeof(float));
+      e = device_malloc(&sb.I, N * sizeof(float));
+      if (e == hipSuccess) e = device_malloc(&sb.jt, (size_t)n_time_steps * N * sizeof(float));
+      if (e == hipSuccess) e = device_malloc(&sb.jd, (size_t)n_time_steps * N * sizeof(float));
+      if (e == hipSuccess) e = device_malloc(&sb.step, sizeof(float));
       if (e == hipSuccess) e = hipMemset(sb.step, 0, sizeof(float));
       p0[k] = sb.jt;  // t = 0 slots
       p1[k] = sb.jd;

@@ -1,18 +1,22 @@
 // awk_mem.hip -- device memory that outlives a handle or a call.
 //
-// dev_alloc / dev_free: the buffers of operators, iterators and atlases.  A handle's
+// dev_alloc / dev_free: the buffers of operators and of greedy and LDMM iterators (an
+// atlas's own slabs, the network's and the trainer's are plain allocations).  A handle's
 // allocation and release map and unmap its pages (160 x 192 x 144 greedy iterator: 1.1
 // ms to create, 1.0 to destroy, against 0.19 ms per iteration), and a multiscale run
-// makes one per level.  Released blocks are kept for the next handle of about the
-// size: at most 1 GiB per device in blocks of up to 512 MiB, the oldest given back
-// first, all of them when an allocation fails.  A block is put away only once the
-// device is idle (hipFree waits in the same way), so whoever takes it next, on any
-// thread or stream, finds no work on it.
+// makes one per level.  Released blocks are kept for the next handle that wants the
+// same sizes: at most 1 GiB per device in blocks of up to 512 MiB, the oldest given back
+// first.  A block is put away only once the device is idle (hipFree waits in the same
+// way), so whoever takes it next, on any thread or stream, finds no work on it.
 //
 // scratch_alloc / scratch_free: stream-ordered scratch of one call, from a pool that
 // keeps up to 512 MiB between calls; the runtime's default pool gives everything back
 // at each synchronisation and the next call pays for the mapping (a 256^3 splat that
 // is waited for: 650 us with it, 260 from the pool).
+//
+// What is kept is given back, and the allocation tried once more, when any of this
+// library's allocations (device_malloc among them) finds the device full.  Other
+// allocators in the process cannot ask for it: awk_release_memory does.
 #include <mutex>
 #include <unordered_map>
 #include <vector>
@@ -42,52 +46,65 @@ Cache &cache() {  // never destroyed: handles may be released at the process's e
   static Cache *c = new Cache();
   return *c;
 }
+// Everything kept on device dev goes back to the runtime (the lock is held).
+void release_kept(Cache &c, int dev) {
+  (void)hipDeviceSynchronize();  // scratch that is free in stream order only is free now
+  for (size_t i = 0; i < c.idle.size();)
+    if (c.idle[i].dev == dev) {
+      (void)hipFree(c.idle[i].p);
+      c.held[dev] -= c.idle[i].size;
+      c.idle.erase(c.idle.begin() + i);
+    } else {
+      ++i;
+    }
+  if (c.pool[dev]) (void)hipMemPoolTrimTo(c.pool[dev], 0);
+}
+// alloc() once more with nothing kept if the device was full.
+template <class F>
+hipError_t or_release(F alloc, int dev) {
+  hipError_t e = alloc();
+  if (e != hipErrorOutOfMemory || dev < 0 || dev >= kMaxDev) return e;
+  Cache &c = cache();
+  std::lock_guard<std::mutex> lock(c.mu);
+  (void)hipGetLastError();
+  release_kept(c, dev);
+  return alloc();
+}
 size_t block_size(size_t bytes) {
   const size_t unit = bytes < (1u << 20) ? 4096 : 65536;
   return (bytes + unit - 1) / unit * unit;
 }
 }  // namespace
 
-hipError_t dev_alloc_bytes(void **p, size_t bytes) {
+hipError_t device_malloc_bytes(void **p, size_t bytes) {
   *p = nullptr;
-  if (!bytes) return hipMalloc(p, bytes);
   int dev = -1;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
+  if (hipError_t e = hipGetDevice(&dev)) return e;
+  return or_release([&] { return hipMalloc(p, bytes); }, dev);
+}
+
+hipError_t dev_alloc_bytes(void **p, size_t bytes) {
+  if (!bytes) return device_malloc_bytes(p, bytes);
+  *p = nullptr;
+  int dev = -1;
+  if (hipError_t e = hipGetDevice(&dev)) return e;
   const size_t want = block_size(bytes);
   Cache &c = cache();
+  {
+    // the same size only: a larger block would hold more than the handle needs
+    std::lock_guard<std::mutex> lock(c.mu);
+    for (size_t i = 0; i < c.idle.size(); ++i) {
+      const Block b = c.idle[i];
+      if (b.dev != dev || b.size != want) continue;
+      c.live[b.p] = b;
+      c.idle.erase(c.idle.begin() + i);
+      c.held[dev] -= b.size;
+      *p = b.p;
+      return hipSuccess;
+    }
+  }
+  if (hipError_t e = or_release([&] { return hipMalloc(p, want); }, dev)) return e;
   std::lock_guard<std::mutex> lock(c.mu);
-  int best = -1;
-  for (int i = 0; i < (int)c.idle.size(); ++i) {
-    const Block &b = c.idle[i];
-    if (b.dev == dev && b.size >= want && b.size <= want + want / 4 && (best < 0 || b.size < c.idle[best].size)) best = i;
-  }
-  if (best >= 0) {
-    const Block b = c.idle[best];
-    c.idle.erase(c.idle.begin() + best);
-    c.held[dev] -= b.size;
-    c.live[b.p] = b;
-    *p = b.p;
-    return hipSuccess;
-  }
-  e = hipMalloc(p, want);
-  if (e != hipSuccess) {
-    // give back what is kept here and try once more
-    bool any = false;
-    for (size_t i = 0; i < c.idle.size();)
-      if (c.idle[i].dev == dev) {
-        (void)hipFree(c.idle[i].p);
-        c.held[dev] -= c.idle[i].size;
-        c.idle.erase(c.idle.begin() + i);
-        any = true;
-      } else {
-        ++i;
-      }
-    if (!any) return e;
-    (void)hipGetLastError();
-    e = hipMalloc(p, want);
-    if (e != hipSuccess) return e;
-  }
   c.live[*p] = Block{*p, want, dev};
   return hipSuccess;
 }
@@ -151,10 +168,24 @@ hipError_t scratch_alloc_bytes(void **p, size_t bytes, hipStream_t s) {
     }
     pool = c.pool[dev];
   }
-  if (pool) return hipMallocFromPoolAsync(p, bytes, pool, s);
-  return hipMallocAsync(p, bytes, s);
+  if (capturing) return hipMallocAsync(p, bytes, s);
+  if (!pool) return or_release([&] { return hipMallocAsync(p, bytes, s); }, dev);
+  return or_release([&] { return hipMallocFromPoolAsync(p, bytes, pool, s); }, dev);
 }
 
 hipError_t scratch_free(void *p, hipStream_t s) { return hipFreeAsync(p, s); }
 
 }  // namespace awk
+
+using namespace awk;
+
+extern "C" awk_status awk_release_memory(void) {
+  int dev = -1;
+  AWK_HIP(hipGetDevice(&dev));
+  if (dev < 0 || dev >= kMaxDev) return AWK_OK;  // (none is kept there)
+  AWK_HIP(hipDeviceSynchronize());
+  Cache &c = cache();
+  std::lock_guard<std::mutex> lock(c.mu);
+  release_kept(c, dev);
+  return AWK_OK;
+}

@@ -719,15 +719,15 @@ awk_status awk_unet_create_batch(awk_unet_t *out, int nx, int ny, int nz, int ma
     u->kpad[l] = (27 * L.cin + 31) / 32 * 32;
     const std::vector<bf16> wt = pack_weights(weights + off, L.cout, L.cin, bc, u->kpad[l]);
     off += (size_t)L.cout * bc * 27;
-    if (e == hipSuccess) e = hipMalloc(&u->w[l], wt.size() * sizeof(bf16));
+    if (e == hipSuccess) e = device_malloc(&u->w[l], wt.size() * sizeof(bf16));
     if (e == hipSuccess) e = hipMemcpy(u->w[l], wt.data(), wt.size() * sizeof(bf16), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMalloc(&u->bias[l], L.cout * sizeof(float));
+    if (e == hipSuccess) e = device_malloc(&u->bias[l], L.cout * sizeof(float));
     if (e == hipSuccess) e = hipMemcpy(u->bias[l], weights + off, L.cout * sizeof(float), hipMemcpyHostToDevice);
     off += L.cout;
   }
-  if (e == hipSuccess) e = hipMalloc(&u->head_w, 48 * sizeof(float));
+  if (e == hipSuccess) e = device_malloc(&u->head_w, 48 * sizeof(float));
   if (e == hipSuccess) e = hipMemcpy(u->head_w, weights + off, 48 * sizeof(float), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMalloc(&u->head_b, 3 * sizeof(float));
+  if (e == hipSuccess) e = device_malloc(&u->head_b, 3 * sizeof(float));
   if (e == hipSuccess) e = hipMemcpy(u->head_b, weights + off + 48, 3 * sizeof(float), hipMemcpyHostToDevice);
   const size_t N0 = (size_t)nx * ny * nz * max_batch, N1 = N0 / 8, N2 = N1 / 8, N3 = N2 / 8;
   struct {
@@ -740,7 +740,7 @@ awk_status awk_unet_create_batch(awk_unet_t *out, int nx, int ny, int nz, int ma
               {&u->d1a, N1 * 32}, {&u->d1, N1 * 32},  {&u->c0, N0 * 48},  {&u->d0a, N0 * 16},
               {&u->d0, N0 * 16}};
   for (auto &b : bufs)
-    if (e == hipSuccess) e = hipMalloc((void **)b.p, b.n * sizeof(bf16));
+    if (e == hipSuccess) e = device_malloc((void **)b.p, b.n * sizeof(bf16));
   if (e != hipSuccess) {
     awk_status st = hip_check(e, "awk_unet_create: allocation");
     unet_free(u);

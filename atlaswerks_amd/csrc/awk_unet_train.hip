@@ -661,7 +661,7 @@ awk_status awk_unet_trainer_create(awk_unet_trainer_t *out, awk_unet_t net, cons
   const size_t wb = n_weights * sizeof(float);
   float **fb[] = {&t->w, &t->g, &t->m, &t->v};
   for (float **p : fb) {
-    if (e == hipSuccess) e = hipMalloc((void **)p, wb);
+    if (e == hipSuccess) e = device_malloc((void **)p, wb);
     if (e == hipSuccess) e = hipMemset(*p, 0, wb);
   }
   if (e == hipSuccess) e = hipMemcpy(t->w, weights, wb, hipMemcpyHostToDevice);
@@ -669,7 +669,7 @@ awk_status awk_unet_trainer_create(awk_unet_trainer_t *out, awk_unet_t net, cons
     const LayerSpec &L = kUnetLayers[l];
     t->kpad_d[l] = (27 * L.cout + 31) / 32 * 32;
     const size_t n = (size_t)L.cin * t->kpad_d[l];
-    e = hipMalloc(&t->wd[l], n * sizeof(bf16));
+    e = device_malloc(&t->wd[l], n * sizeof(bf16));
     if (e == hipSuccess) e = hipMemset(t->wd[l], 0, n * sizeof(bf16));
   }
   struct {
@@ -681,10 +681,10 @@ awk_status awk_unet_trainer_create(awk_unet_trainer_t *out, awk_unet_t net, cons
               {&t->dz5, N2 * 64},  {&t->dz4, N2 * 64},  {&t->dp1, N2 * 32},  {&t->dz3, N1 * 32},
               {&t->dz2, N1 * 32},  {&t->dp0, N1 * 16},  {&t->dz1, N0 * 16},  {&t->dz0, N0 * 16}};
   for (auto &b : bufs)
-    if (e == hipSuccess) e = hipMalloc((void **)b.p, b.n * sizeof(bf16));
-  if (e == hipSuccess) e = hipMalloc(&t->u, 3 * N0 * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&t->hpart, (N0 + 255) / 256 * 52 * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&t->ws, (kWgWsFloats + (size_t)kWgMaxBlocks * 128) * sizeof(float));
+    if (e == hipSuccess) e = device_malloc((void **)b.p, b.n * sizeof(bf16));
+  if (e == hipSuccess) e = device_malloc(&t->u, 3 * N0 * sizeof(float));
+  if (e == hipSuccess) e = device_malloc(&t->hpart, (N0 + 255) / 256 * 52 * sizeof(float));
+  if (e == hipSuccess) e = device_malloc(&t->ws, (kWgWsFloats + (size_t)kWgMaxBlocks * 128) * sizeof(float));
   // rows = ceil(nb / kWgSumRows) <= nb / kWgSumRows + 1, so rows * ne <= ws / kWgSumRows + ne
   size_t max_ne = 0;
   for (int l = 0; l < 14; ++l) {
@@ -692,7 +692,7 @@ awk_status awk_unet_trainer_create(awk_unet_trainer_t *out, awk_unet_t net, cons
     if (ne > max_ne) max_ne = ne;
   }
   if (e == hipSuccess)
-    e = hipMalloc(&t->ws2, (kWgWsFloats / kWgSumRows + max_ne + (size_t)kWgMaxBlocks * 128) * sizeof(float));
+    e = device_malloc(&t->ws2, (kWgWsFloats / kWgSumRows + max_ne + (size_t)kWgMaxBlocks * 128) * sizeof(float));
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&t->side, hipStreamNonBlocking);
   for (hipEvent_t &ev : t->fork)
     if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
@@ -751,7 +751,7 @@ awk_status awk_unet_trainer_gradients(awk_unet_trainer_t t, const float *templ, 
       !loss_host)
     return fail(AWK_ERR_INVALID, "awk_unet_trainer_gradients: null argument");
   double *ld = nullptr;
-  AWK_HIP(hipMalloc(&ld, sizeof(double)));
+  AWK_HIP(device_malloc(&ld, sizeof(double)));
   awk_status st = AWK_OK;
   hipError_t e = hipMemset(ld, 0, sizeof(double));
   if (e == hipSuccess) e = hipMemset(t->g, 0, t->nw * sizeof(float));

@@ -8,6 +8,14 @@ import ctypes
 
 import torch
 
+from . import _lib
+
+
+def release_memory():
+    """Give back the device memory the library keeps between handles and calls (at most
+    1.5 GiB): before another allocator, torch's among them, needs all of the device."""
+    _lib.call("awk_release_memory")
+
 
 def stream_handle(stream=None):
     s = stream if stream is not None else torch.cuda.current_stream()

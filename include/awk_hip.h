@@ -82,6 +82,13 @@ enum {
 awk_status awk_tune_set(const char *name, int value);
 awk_status awk_tune_get(const char *name, int *value);
 
+/* Device memory that the library keeps on the current device between handles (blocks of
+ * destroyed operators and iterators, at most 1 GiB) and calls (scratch, at most 512 MiB)
+ * goes back to the runtime.  The library does this by itself when one of its own
+ * allocations finds the device full; this is for other allocators in the process.
+ * Waits for the device.  No counterpart in the reference. */
+awk_status awk_release_memory(void);
+
 /* Last error message of the calling host thread ("" if none). */
 const char *awk_last_error(void);
 /* Library version, major*10000 + minor*100 + patch. */

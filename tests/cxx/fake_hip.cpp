@@ -53,7 +53,7 @@ hipError_t take(void **p, size_t n, Pool *pool) {
       return hipSuccess;
     }
   }
-  if (n > g_budget - g_used) return ret(hipErrorOutOfMemory);
+  if (n > g_budget || g_used > g_budget - n) return ret(hipErrorOutOfMemory);
   g_used += n;
   *p = reinterpret_cast<void *>(g_next);
   g_live[g_next] = Block{n, pool};

@@ -43,3 +43,44 @@ rc = lib.awk_splat_sorted(p, p, p, p, p, *%r, 1, None, None, None)
 assert rc == 0, lib.awk_last_error()
 assert any("k_base_sum" in r[1] for r in log("launch"))
 """ % (size,))
+
+
+# what a handle or call takes, in every way the library allocates
+_TAKERS = {
+    "gaussian_filter": "assert lib.awk_gaussian_filter(p, q, 96, 96, 96, 1.0, 1.0, 1.0, 2, 2, 2, None) == 0, lib.awk_last_error()",
+    "splat": "assert lib.awk_splat(p, q, q, q, q, 96, 96, 96, 0, None) == 0, lib.awk_last_error()",
+    "greedy": "assert lib.awk_greedy_create(ctypes.byref(h), 80, 80, 80, *([1.0] * 3), .01, .01, .001, .1) == 0, lib.awk_last_error()",
+    "atlas": "assert lib.awk_atlas_create(ctypes.byref(h), 48, 48, 48, *([1.0] * 3), .01, .01, .001, .1, 3) == 0, lib.awk_last_error()",
+    "ldmm_atlas": "assert lib.awk_ldmm_atlas_create(ctypes.byref(h), 40, 40, 40, *([1.0] * 3), .01, .01, .001, 3, 1.0, .1, 2, 0) == 0, lib.awk_last_error()",
+    "unet": "w = (ctypes.c_float * lib.awk_unet_weight_count())(); assert lib.awk_unet_create(ctypes.byref(h), 64, 64, 64, w, len(w)) == 0, lib.awk_last_error()",
+    "unet_trainer": "t = P(); w = (ctypes.c_float * lib.awk_unet_weight_count())(); assert lib.awk_unet_create(ctypes.byref(h), 32, 32, 32, w, len(w)) == 0 and "
+                    "lib.awk_unet_trainer_create(ctypes.byref(t), h, w, len(w)) == 0, lib.awk_last_error()",
+}
+
+
+@pytest.mark.parametrize("kept", ["blocks", "scratch"])
+@pytest.mark.parametrize("taker", sorted(_TAKERS))
+def test_kept_memory_is_given_back(fake, taker, kept):
+    """An allocation that fits the device once nothing is kept succeeds while blocks or
+    scratch are: what the taker needs is measured in a fresh process, then it runs on a
+    device with exactly that much beside what the program itself holds."""
+    head = "h, p, q = P(), P(0x4000), P(0x8000)\n"
+    need = int(fake_hip.run(fake, head + _TAKERS[taker] + "\nprint(fake.fake_used())"))
+    keep = {"blocks": "g = P(); assert lib.awk_greedy_create(ctypes.byref(g), 64, 72, 60, *([1.0] * 3), .01, .01, .001, .1) == 0 and lib.awk_greedy_destroy(g) == 0",
+            "scratch": "assert lib.awk_splat(p, q, q, q, q, 64, 72, 60, 0, None) == 0"}[kept]
+    fake_hip.run(fake, head + keep + """
+assert fake.fake_used() > 1 << 20  # kept
+fake.fake_budget(max(%d, fake.fake_used()))
+""" % need + _TAKERS[taker])
+
+
+def test_release_memory(fake):
+    fake_hip.run(fake, """
+g, p, q = P(), P(0x4000), P(0x8000)
+assert lib.awk_greedy_create(ctypes.byref(g), 64, 72, 60, *([1.0] * 3), .01, .01, .001, .1) == 0
+live = fake.fake_used()
+assert lib.awk_splat(p, q, q, q, q, 64, 72, 60, 0, None) == 0
+assert lib.awk_release_memory() == 0 and fake.fake_used() == live
+assert lib.awk_greedy_destroy(g) == 0 and fake.fake_used() == live  # kept
+assert lib.awk_release_memory() == 0 and fake.fake_used() == 0
+""")
