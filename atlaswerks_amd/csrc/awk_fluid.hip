@@ -524,6 +524,13 @@ awk_status fk_prepare_eigen(FluidKernel &k, int dir, hipStream_t s) {
   if (k.eig && k.eig_dir == dir) return AWK_OK;
   const size_t nf = (size_t)k.nxh * k.ny * k.nz;
   if (!k.eig) {
+    // Under capture the table would be recorded and not made, and calls outside the graph
+    // would read it: refused whether or not a kept block spares the allocation (which a
+    // capture does not take).
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    AWK_HIP(hipStreamIsCapturing(s, &cap));
+    if (cap != hipStreamCaptureStatusNone)
+      return fail(AWK_ERR_HIP, "fluid kernel: the first application with an eigen table cannot be captured");
     AWK_HIP(dev_alloc(&k.eig, nf * 6 * sizeof(float)));
     k.scratch_bytes += nf * 6 * sizeof(float);
   }
