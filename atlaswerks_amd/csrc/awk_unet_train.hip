@@ -543,6 +543,22 @@ static awk_status wgrad(awk_unet_trainer *t, int l, const bf16 *dz, const bf16 *
 
 // Forward and backward of one pair: the gradient is added to t->g, the loss to
 // *loss_dev.
+// The weight gradients' stream joined into the caller's, also where a call ends early: what
+// is still queued there reads activations that the next call overwrites.
+struct SideJoin {
+  awk_unet_trainer *t;
+  hipStream_t s;
+  bool open = false;  // something was put on the side stream
+  hipError_t close() {
+    open = false;
+    const hipError_t e = hipEventRecord(t->join, t->side);
+    return e == hipSuccess ? hipStreamWaitEvent(s, t->join, 0) : e;
+  }
+  ~SideJoin() {
+    if (open) (void)close();
+  }
+};
+
 static awk_status train_backward(awk_unet_trainer *t, const float *templ, const float *subject,
                                  const float *const target[3], double *loss_dev, hipStream_t s) {
   awk_unet *u = t->net;
@@ -567,10 +583,12 @@ static awk_status train_backward(awk_unet_trainer *t, const float *templ, const 
   // (64^3: most launches of either are fewer blocks than the chip holds).  They share
   // the workspace, so they stay in order among themselves.
   int forks = 0;
+  SideJoin side{t, s};
   auto fork = [&]() -> awk_status {
     hipEvent_t e = t->fork[forks++];
     AWK_HIP(hipEventRecord(e, s));
     AWK_HIP(hipStreamWaitEvent(t->side, e, 0));
+    side.open = true;
     return AWK_OK;
   };
   struct Wg {
@@ -624,8 +642,7 @@ static awk_status train_backward(awk_unet_trainer *t, const float *templ, const 
   if ((st = wgrads({{1, t->dz1, u->t0, nx, ny, nz}}))) return st;
   if ((st = dgrad(t, 1, t->dz1, u->t0, t->dz0, nx, ny, nz, s))) return st;
   if ((st = wgrads({{0, t->dz0, u->x0, nx, ny, nz}}))) return st;
-  AWK_HIP(hipEventRecord(t->join, t->side));
-  AWK_HIP(hipStreamWaitEvent(s, t->join, 0));
+  AWK_HIP(side.close());
   AWK_LAUNCH_CHECK("backward");
   return AWK_OK;
 }

@@ -109,3 +109,42 @@ assert any("k_eigen_table" in r[1] for r in log("launch"))
 fake.fake_capture(1)
 assert lib.awk_fluid_kernel_apply(b, p, p, p, 1, None) == 0  # with its table it may be captured
 """)
+
+
+def test_weight_gradient_stream_is_joined_on_every_exit(fake):
+    """Whichever launch of a training step fails, the caller's stream waits for what was
+    put on the weight gradients' stream: the next call may overwrite what they read."""
+    out = fake_hip.run(fake, """
+w = (ctypes.c_float * lib.awk_unet_weight_count())()
+net, t = P(), P()
+assert lib.awk_unet_create(ctypes.byref(net), 16, 16, 16, w, len(w)) == 0
+assert lib.awk_unet_trainer_create(ctypes.byref(t), net, w, len(w)) == 0
+p, s = P(0x4000), 0x77770
+u = (P * 3)(0x4000, 0x8000, 0xc000)
+def step():
+    fake.fake_clear()
+    rc = lib.awk_unet_trainer_step(t, p, p, u, 1e-3, p, P(s))
+    rows = log()
+    side = [i for i, r in enumerate(rows) if r[0] == "launch" and r[5] != str(s)]
+    if not side:
+        return rc, len([r for r in rows if r[0] == "launch"]), True
+    st = rows[side[-1]][5]
+    after = rows[side[-1] + 1:]
+    rec = [i for i, r in enumerate(after) if r[0] == "record" and r[2] == st]
+    joined = any(r[0] == "wait" and r[1] == str(s) and r[2] == after[i][1] for i in rec for r in after[i:])
+    return rc, len([r for r in rows if r[0] == "launch"]), joined
+rc, n, joined = step()
+assert rc == 0 and joined, (rc, joined)
+bad = []
+for k in range(n):
+    fake.fake_fail(b"k_", k)
+    rc, _, joined = step()
+    assert rc != 0, k
+    if not joined:
+        bad.append(k)
+fake.fake_fail(b"", 0)
+assert step()[0] == 0
+print(n, len(bad))
+""")
+    n, bad = map(int, out.split())
+    assert n > 50 and bad == 0, (n, bad)
