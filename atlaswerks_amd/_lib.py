@@ -25,6 +25,7 @@ SIGNATURES = {
     "awk_version": [],
     "awk_tune_set": [ctypes.c_char_p, _I],
     "awk_tune_get": [ctypes.c_char_p, ctypes.POINTER(_I)],
+    "awk_fft_axis_staged": [_I, _I],
     "awk_release_memory": [],
     "awk_fluid_kernel_create": [ctypes.POINTER(_P), _I, _I, _I, _F, _F, _F, _F, _F, _F, _F, _I],
     "awk_fluid_kernel_set_params": [_P, _F, _F, _F, _F, _I],

@@ -190,22 +190,41 @@ PLAN_KNOBS = {
 }
 
 
+def _plan_knobs(size):
+    """The plan knobs that an operator of grid (nx, ny, nz) reads: those of its axes whose
+    passes run the LDS stages."""
+    staged = [bool(_lib.load().awk_fft_axis_staged(a, n)) for a, n in enumerate(size)]
+    names = {k for k, s in zip(("x_rt", "y_tx", "z_tx"), staged) if s}
+    if any(s and n > 1 for s, n in zip(staged, size)):
+        names.add("fft_order")
+    return names
+
+
 def tune_fft(size, reps=10, device="cuda", verbose=False):
-    """FFT plan for one grid (nx, ny, nz): the radix order of the generic LDS
-    stages and the x / y / z pass tiles, chosen one knob after the other by timing
-    the operator L^-1 (DiffOperGPU::ApplyInverseOperator) through graph replays.
-    Plans are read when an operator is created, so the chosen knobs stay set for
-    the operators made afterwards.  They change results only at FP32 rounding
-    level (another butterfly order or kernel).  Returns (chosen, timings)."""
+    """FFT plan for one grid (nx, ny, nz): the radix order of the LDS stages and their x /
+    y / z pass tiles, chosen one knob after the other by timing the operator L^-1
+    (DiffOperGPU::ApplyInverseOperator) through graph replays.  Lengths with a kernel of
+    their own, two radices or a dense product have one plan: a knob that no axis of the
+    grid reads is not timed and set to its default.  Plans are read when an operator is
+    created, so the chosen knobs stay set for the operators made afterwards.  They change
+    results only at FP32 rounding level (another butterfly order or kernel).  Returns
+    (chosen, timings)."""
     from .fluid import DiffOperGPU
     nx, ny, nz = size
-    f = torch.randn((3, nz, ny, nx), device=device)
+    read = _plan_knobs(size)
     chosen, timings = {}, {}
-    op = DiffOperGPU((nx, ny, nz))  # warm-up: the first operator's first-use costs
-    _time(lambda: op.ApplyInverseOperator(f), reps)
-    del op
+    f = None
     for name, values in PLAN_KNOBS.items():
         timings[name] = {}
+        if name not in read:
+            set_knob(name, values[0])
+            chosen[name] = values[0]
+            continue
+        if f is None:
+            f = torch.randn((3, nz, ny, nx), device=device)
+            op = DiffOperGPU((nx, ny, nz))  # warm-up: the first operator's first-use costs
+            _time(lambda: op.ApplyInverseOperator(f), reps)
+            del op
         best = None
         for v in values:
             set_knob(name, v)

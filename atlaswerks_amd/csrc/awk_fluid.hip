@@ -726,6 +726,10 @@ using namespace awk;
 
 extern "C" {
 
+int awk_fft_axis_staged(int axis, int n) {
+  return axis >= 0 && axis < 3 && n >= 1 && !use_radix(axis, n) && !use_dense(n, factor(n));
+}
+
 awk_status awk_fluid_kernel_create(awk_fk_t *out, int nx, int ny, int nz, float spx, float spy,
                                    float spz, float alpha, float beta, float gamma, float lpow,
                                    int flags) {

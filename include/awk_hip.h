@@ -78,9 +78,14 @@ enum {
  * subjects per group of one fused launch; read when an atlas iteration is
  * launched or captured); results do not depend on them.  FFT plan knobs read when an operator is created:
  * "fft_order", "x_rt", "y_tx", "z_tx" (another butterfly order or tile, results
- * within FP32 rounding; for lengths that neither a two-radix nor a dense plan takes).  Process-wide.  No counterpart in the reference. */
+ * within FP32 rounding; for axes that run the LDS stages, see awk_fft_axis_staged).
+ * Process-wide.  No counterpart in the reference. */
 awk_status awk_tune_set(const char *name, int value);
 awk_status awk_tune_get(const char *name, int *value);
+/* 1 where an operator's axis (0 x, 1 y, 2 z) of n voxels runs the LDS stages, which alone
+ * the plan knobs change: lengths that neither two radices up to 32 nor a dense product
+ * take.  0 otherwise.  No device call. */
+int awk_fft_axis_staged(int axis, int n);
 
 /* Device memory that the library keeps on the current device between handles (blocks of
  * destroyed operators and iterators, at most 1 GiB) and calls (scratch, at most 512 MiB)
