@@ -15,12 +15,12 @@ TOL = 1e-5
 SIZES = [(8, 8, 8), (6, 10, 12), (24, 40, 36), (32, 31, 36), (64, 64, 64), (17, 9, 5),
          (96, 48, 40), (1, 16, 16), (128, 128, 128), (32, 64, 256), (256, 256, 16),
          (128, 32, 64)]
-# axes with a prime factor above 64 (Bluestein's transform): 67, 71, 127, 181 on each
-# axis; 217 = 7 * 31 and 61 take direct prime stages
+# axes with a prime factor above 13 (dense products): 67, 71, 127, 181 on each axis, 217 =
+# 7 * 31 and 61
 PRIME_SIZES = [(12, 20, 67), (16, 127, 10), (181, 12, 14), (61, 67, 71), (36, 217, 181),
                (1, 1, 181)]
 # axes whose pass blocks stage more than 64 KiB of LDS (up to 159 KiB): 2500 along x,
-# Bluestein primes 1021 along x and 3001 along y, 1499 along z
+# the primes 1021 along x, 3001 along y and 1499 along z (chirp-z transforms)
 LONG_SIZES = [(3, 4, 2500), (4, 5, 1021), (2, 3001, 3), (1499, 3, 2)]
 
 
@@ -89,8 +89,9 @@ def test_round_trip_identity():
                                    {"fft_order": 1, "x_rt": 6, "y_tx": 4, "z_tx": 2}])
 @pytest.mark.parametrize("shape", [(24, 40, 36), (36, 48, 60), (12, 20, 67), (128, 128, 128)])
 def test_tuned_fft_plans_match_oracle(shape, knobs):
-    """The plans the autotuner chooses between (radix order of the generic stages,
-    x / y / z pass tiles): L^-1 within the same 1e-5 of the FP64 oracle."""
+    """Axes with two radices, a dense product or a kernel of their own under plan knobs
+    (which only other lengths read, see the staged axes below): L^-1 within the same 1e-5
+    of the FP64 oracle."""
     from atlaswerks_amd import autotune
     from atlaswerks_amd.fluid import DiffOperGPU, DiffOperParam
     from gpu_util import aos, host, rel_l2, soa, to_dev
@@ -196,6 +197,62 @@ def test_force_columns_match_oracle(shape):
     from atlaswerks_amd.greedy import GreedyWarp
     from gpu_util import host, rel_l2, soa
     print("greedy columns", shape, flush=True)
+    t, h, _ = synth.pair(shape, seed=4, max_disp=1.0)
+    target = oracle.apply(t, np.moveaxis(h, 0, -1), dtype=np.float32)
+    sp = (1.2, 0.9, 1.0)
+    hd, _, _, ed, _ = oracle.greedy_run(t, target, 4, sp=sp)
+    data = GreedyWarp(torch.from_numpy(t).cuda(), torch.from_numpy(target).cuda(), 4, spacing=sp).RunWarp()
+    assert np.max(np.abs(data.energies() - ed) / ed) < 1e-3
+    assert rel_l2(host(data.Def1To0), soa(hd)) <= 1e-5
+
+
+# Axes that run the LDS stages: small primes without two radices up to 32 (343 = 7^3, 245,
+# 429), chirp-z past the dense lengths (514 = 2 * 257), and a single voxel; rows past the
+# two-radix lengths (1100); row groups over a plane's end and past the volume's
+STAGED_SHAPES = [(3, 7, 343), (2, 5, 514), (3, 11, 1), (2, 3, 1100), (3, 343, 6), (2, 514, 5), (245, 4, 6),
+                 (514, 3, 5), (7, 5, 429)]
+
+
+def _axis_staged(shape):
+    from atlaswerks_amd import _lib
+    return [bool(_lib.load().awk_fft_axis_staged(a, n)) for a, n in enumerate(shape[::-1])]
+
+
+@pytest.mark.parametrize("knobs", [{}, {"fft_order": 1}, {"x_rt": 2}, {"x_rt": 4, "y_tx": 2, "z_tx": 1},
+                                   {"fft_order": 1, "x_rt": 6, "y_tx": 4, "z_tx": 2}])
+@pytest.mark.parametrize("shape", STAGED_SHAPES)
+def test_staged_axis_plans_match_oracle(shape, knobs):
+    """L^-1 with an axis that reads the plan knobs, under each of the plans the autotuner
+    chooses between.  Bar: the operator tests' 1e-5."""
+    from atlaswerks_amd import autotune
+    from atlaswerks_amd.fluid import DiffOperGPU, DiffOperParam
+    from gpu_util import aos, host, rel_l2, soa, to_dev
+    nz, ny, nx = shape
+    print("fluid staged", shape, knobs, flush=True)
+    assert any(_axis_staged(shape))
+    f = _field(shape, seed=13)
+    sp = (1.0, 1.25, 0.8)
+    try:
+        for k, v in knobs.items():
+            autotune.set_knob(k, v)
+        op = DiffOperGPU((nx, ny, nz), sp, DiffOperParam(alpha=0.01, beta=0.01, gamma=0.001))
+    finally:
+        for k in autotune.PLAN_KNOBS:
+            autotune.set_knob(k, 0)
+    d = to_dev(f)
+    op.ApplyInverseOperator(d)
+    ref = oracle.diffoper(aos(f), sp=sp, alpha=0.01, beta=0.01, gamma=0.001, inverse=True)
+    assert rel_l2(host(d), soa(ref)) <= TOL
+
+
+@pytest.mark.parametrize("shape", STAGED_SHAPES)
+def test_staged_axes_greedy_matches_oracle(shape):
+    """The force, energy, composition and next deformed image around the LDS stages: the
+    greedy parity tests' bars."""
+    import torch
+    from atlaswerks_amd.greedy import GreedyWarp
+    from gpu_util import host, rel_l2, soa
+    print("greedy staged", shape, flush=True)
     t, h, _ = synth.pair(shape, seed=4, max_disp=1.0)
     target = oracle.apply(t, np.moveaxis(h, 0, -1), dtype=np.float32)
     sp = (1.2, 0.9, 1.0)

@@ -156,3 +156,29 @@ def test_ldmm_vector_energy_rows(shape, orig):
     torch.cuda.synchronize()
     np.testing.assert_allclose(e.energies()[:, 1], ev, rtol=1e-5)
     np.testing.assert_allclose(e.energies()[:, 0], ei, rtol=1e-5)
+
+
+STAGED_SHAPES = [(3, 7, 343), (2, 5, 514), (3, 343, 6), (245, 4, 6)]
+
+
+# rows of one voxel: IterateNew only (IterateOrig's Jacobian determinant is zero there)
+@pytest.mark.parametrize("shape,orig,splat", [(s, o, k) for s in STAGED_SHAPES for o, k in MODES] +
+                         [((3, 11, 1), False, "fixed"), ((3, 11, 1), False, "sorted")])
+def test_ldmm_staged_axes_vs_oracle(shape, orig, splat):
+    """The velocity update, step size and vector energy around the LDS stages (lengths
+    without two radices or a dense product), row groups over a plane's end and past the
+    volume's.  The bars above."""
+    import torch
+    from atlaswerks_amd import ldmm
+    from gpu_util import rel_l2, to_dev
+    print("ldmm staged", shape, orig, splat, flush=True)
+    I0, I1 = _pair(shape, seed=9, disp=0.8)
+    v_ref, ei, ev, st = _oracle_run(orig)(I0, I1, 2, 2, sigma=0.1, max_pert=0.1)
+    prm = ldmm.LDMMIteratorParam(sigma=0.1, max_pert=0.1, use_orig_gradient=orig, splat=splat)
+    w = ldmm.LDMMWarp(to_dev(I0), to_dev(I1), n_time_steps=2, n_iter=2, param=prm)
+    e = w.RunWarp(vec_energy=True)
+    torch.cuda.synchronize()
+    assert abs(w.iterator.StepSize() / st - 1) < 1e-5
+    assert rel_l2(e.v.cpu().numpy(), _soa_v(v_ref)) <= 1e-4
+    np.testing.assert_allclose(e.energies()[:, 1], ev, rtol=1e-5)
+    np.testing.assert_allclose(e.energies()[:, 0], ei, rtol=1e-5)
