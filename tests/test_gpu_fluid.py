@@ -260,3 +260,29 @@ def test_staged_axes_greedy_matches_oracle(shape):
     data = GreedyWarp(torch.from_numpy(t).cuda(), torch.from_numpy(target).cuda(), 4, spacing=sp).RunWarp()
     assert np.max(np.abs(data.energies() - ed) / ed) < 1e-3
     assert rel_l2(host(data.Def1To0), soa(hd)) <= 1e-5
+
+
+# Mean relative error against 64 bits of L^-1 through the mixed-radix LDS stages that the
+# plans of these lengths took the place of (the seeds and spacing below)
+STAGES_ERROR = [((36, 36, 36), 4, 1.894e-7), ((42, 42, 42), 4, 1.941e-7), ((84, 84, 84), 4, 2.116e-7),
+                ((100, 100, 100), 2, 2.161e-7), ((30, 30, 30), 4, 1.566e-7), ((5, 200, 12), 2, 1.347e-7)]
+
+
+@pytest.mark.parametrize("shape,seeds,stages", STAGES_ERROR)
+def test_operator_error_is_no_larger_than_the_stages(shape, seeds, stages):
+    """A plan is no less precise than what it replaced: the mean error over the seeds within
+    2 % of the stages' (the spread of the ratio between such sets of seeds)."""
+    from atlaswerks_amd.fluid import DiffOperGPU, DiffOperParam
+    from gpu_util import aos, host, rel_l2, soa, to_dev
+    nz, ny, nx = shape
+    print("fluid error", shape, flush=True)
+    sp = (1.0, 1.25, 0.8)
+    op = DiffOperGPU((nx, ny, nz), sp, DiffOperParam(alpha=0.01, beta=0.01, gamma=0.001))
+    err = []
+    for seed in range(1, seeds + 1):
+        f = _field(shape, seed)
+        d = to_dev(f)
+        op.ApplyInverseOperator(d)
+        ref = oracle.diffoper(aos(f), sp=sp, alpha=0.01, beta=0.01, gamma=0.001, inverse=True)
+        err.append(rel_l2(host(d), soa(ref)))
+    assert np.mean(err) <= 1.02 * stages, np.mean(err) / stages
