@@ -14,10 +14,9 @@
 // otherwise idle, without stages, barriers or index arithmetic, and for any n.
 // It serves the lengths with no short radix plan.
 //
-// Rounding: sums run over at most 16 terms before they are folded into a second
-// accumulator, so the error grows with the number of folds (n / 32), not with n:
-// 0.7e-7 ... 1.2e-7 relative for n = 31 ... 251, against 1.4e-7 ... 1.7e-7 of the
-// chirp-z transforms it takes the place of.
+// Rounding: sums run over 8 or 16 terms before they are folded into a second accumulator,
+// so the error grows with the run and the number of folds, not with n.  Runs of 8 where
+// the LDS stages round as little as runs of 16 (dense_short_runs).
 #pragma once
 
 #include "awk_fft.h"
@@ -36,7 +35,17 @@ constexpr int kDenseMin = 7, kDenseMax = 511;
 struct DenseAxis {
   const float2 *tab;
   int n, H, tiles, ks;  // ks: steps of 2 j, a multiple of 4
+  int short_runs;       // sums in runs of 8 terms (else 16)
 };
+
+// Which lengths take runs of 8 terms, whose folds cost 1 to 2 % of an operator's time at
+// 68^3 ... 136^3 and 3 % at 181 x 217 x 181.  The error of L^-1 against the LDS stages' (means
+// over seeds, each axis): with 16 terms 1.00 ... 1.05 at 34 ... 136 and, of the longer
+// lengths, at those of primes up to 19 (170, 190, 204, 238, 255: 1.01 ... 1.06), with 8
+// terms 0.88 ... 1.02 and 0.98 ... 1.04.  Lengths of larger primes from 144 on (181, 217,
+// 251: 0.73 ... 0.95 with 16 terms) have no need of them, and past 255 the folds of runs
+// of 8 round more than they save.
+inline bool dense_short_runs(int n, int largest_prime) { return n <= 143 || (n <= 255 && largest_prime <= 19); }
 
 __device__ __forceinline__ v16f mfma32(float a, float b, v16f c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
@@ -48,25 +57,21 @@ __device__ __forceinline__ int dense_row(int i, int lane) {
   return 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
 }
 
-// One tile: E and O summed over all j.  p / q: this lane's first values (rows j =
-// lane / 32 and n - j of the staged lines, or of the two staged parts), advanced
-// by dp / dq floats per step; tab: this lane's entry of the tile's first step.
-// DATA_A: the lines are the rows of the result and k its columns (else the lines
-// are the columns).  FOLD: form e and o from the two rows (else they are given).
-template <bool DATA_A, bool FOLD>
-__device__ __forceinline__ void dense_tile(const float *p, const float *q, int dp, int dq,
+// dense_tile's sums in runs of 8 G terms.
+template <bool DATA_A, bool FOLD, int G>
+__device__ __forceinline__ void dense_runs(const float *p, const float *q, int dp, int dq,
                                            const float2 *__restrict__ tab, int ks, v16f &E, v16f &O) {
 #pragma unroll
   for (int i = 0; i < 16; ++i) E[i] = O[i] = 0.f;
   float2 t[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) t[i] = tab[i * 64];
-  for (int s = 0; s < ks; s += 8) {
+  for (int s = 0; s < ks; s += 4 * G) {
     v16f ae, ao;
 #pragma unroll
     for (int i = 0; i < 16; ++i) ae[i] = ao[i] = 0.f;
 #pragma unroll
-    for (int g = 0; g < 2; ++g) {
+    for (int g = 0; g < G; ++g) {
       if (s + 4 * g < ks) {
         float2 u[4];
         const bool more = s + 4 * g + 4 < ks;
@@ -99,6 +104,19 @@ __device__ __forceinline__ void dense_tile(const float *p, const float *q, int d
   }
 }
 
+// One tile: E and O summed over all j.  p / q: this lane's first values (rows j =
+// lane / 32 and n - j of the staged lines, or of the two staged parts), advanced
+// by dp / dq floats per step.
+// DATA_A: the lines are the rows of the result and k its columns (else the lines
+// are the columns).  FOLD: form e and o from the two rows (else they are given).
+template <bool DATA_A, bool FOLD>
+__device__ __forceinline__ void dense_tile(const float *p, const float *q, int dp, int dq,
+                                           const DenseAxis &ax, int tile, int lane, v16f &E, v16f &O) {
+  const float2 *tab = ax.tab + (size_t)tile * ax.ks * 64 + lane;
+  if (ax.short_runs) dense_runs<DATA_A, FOLD, 1>(p, q, dp, dq, tab, ax.ks, E, O);
+  else dense_runs<DATA_A, FOLD, 2>(p, q, dp, dq, tab, ax.ks, E, O);
+}
+
 // The value of the lane's neighbour (lane ^ 1): the other part of a complex column.
 __device__ __forceinline__ float dense_swap(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, true));
@@ -112,7 +130,7 @@ __device__ __forceinline__ void dense_lines(const float *sm, const DenseAxis &ax
   const int hi = lane >> 5, col = lane & 31;
   v16f E, O;
   dense_tile<false, true>(sm + hi * 32 + col, sm + (ax.n - hi) * 32 + col, 64, -64,
-                          ax.tab + (size_t)tile * ax.ks * 64 + lane, ax.ks, E, O);
+                          ax, tile, lane, E, O);
   // forward: X = E - i O: the real part takes + Im O, the imaginary part - Re O
   const float sg = ((lane & 1) != 0) != inv ? -1.f : 1.f;
 #pragma unroll

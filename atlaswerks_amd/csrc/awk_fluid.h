@@ -22,7 +22,7 @@ struct AxisPlan {
   std::vector<int> mrad;
   const float2 *chirp = nullptr, *bhat = nullptr, *mtw = nullptr;
   // Dense transform on the matrix cores (0 tiles: not used)
-  DenseAxis dense{nullptr, 0, 0, 0, 0};
+  DenseAxis dense{nullptr, 0, 0, 0, 0, 0};
   // Two radices in registers (ra 0: not used)
   RadixAxis radix{nullptr, 0, 0, 0};
   // the line length the LDS stages hold (the work area of m when used)

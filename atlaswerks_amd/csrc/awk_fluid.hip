@@ -414,13 +414,15 @@ awk_status fk_init(FluidKernel &k, int nx, int ny, int nz, const float sp[3]) {
     k.ax[i].rad = factor(ns[i]);
     k.ax[i].m = 0;
     k.ax[i].mrad.clear();
-    k.ax[i].dense = DenseAxis{nullptr, 0, 0, 0, 0};
+    k.ax[i].dense = DenseAxis{nullptr, 0, 0, 0, 0, 0};
     k.ax[i].radix = RadixAxis{nullptr, ns[i], 0, 0};
     if (use_radix(i, ns[i])) radix_plan(ns[i], k.ax[i].radix.ra, k.ax[i].radix.rb);
     bool big = false;
     for (int r : k.ax[i].rad) big = big || r > 64;
     if (use_dense(ns[i], k.ax[i].rad)) {
       dense[i] = dense_table(ns[i], k.ax[i].dense);
+      // (factor() gives primes but for powers of two)
+      k.ax[i].dense.short_runs = dense_short_runs(ns[i], *std::max_element(k.ax[i].rad.begin(), k.ax[i].rad.end()));
     } else if (big) {
       // Bluestein: a power-of-two convolution of length m >= 2n - 1
       int m = 1;

@@ -316,7 +316,7 @@ k_xfwd(XFwdArgs a, Axis ax, XPlan xp, int nx_rt, int ny, int nz, int nxh_rt, int
     if (tile < xp.dense.tiles) {
       v16f E, O;
       dense_tile<true, true>(smf + hi * kDenseLS + col, smf + (nx - hi) * kDenseLS + col, 2 * kDenseLS,
-                             -2 * kDenseLS, xp.dense.tab + (size_t)tile * xp.dense.ks * 64 + lane, xp.dense.ks, E, O);
+                             -2 * kDenseLS, xp.dense, tile, lane, E, O);
       const int k = 32 * tile + col;
       if (k < nxh) {
 #pragma unroll
@@ -424,7 +424,7 @@ k_xinv(XInvArgs a, Axis ax, XPlan xp, int nx_rt, int ny, int nz, int nxh_rt, int
     v16f P, Q;
     if (wave < xp.dense.tiles)
       dense_tile<true, false>(smf + hi * kDenseLS + col, im + hi * kDenseLS + col, 2 * kDenseLS,
-                              2 * kDenseLS, xp.dense.tab + (size_t)wave * xp.dense.ks * 64 + lane, xp.dense.ks, P, Q);
+                              2 * kDenseLS, xp.dense, wave, lane, P, Q);
     __syncthreads();  // the staged frequencies are read: the lines take their place
     const int j = 32 * wave + col;
     if (wave < xp.dense.tiles && j < xp.dense.H) {

@@ -265,7 +265,9 @@ def test_staged_axes_greedy_matches_oracle(shape):
 # Mean relative error against 64 bits of L^-1 through the mixed-radix LDS stages that the
 # plans of these lengths took the place of (the seeds and spacing below)
 STAGES_ERROR = [((36, 36, 36), 4, 1.894e-7), ((42, 42, 42), 4, 1.941e-7), ((84, 84, 84), 4, 2.116e-7),
-                ((100, 100, 100), 2, 2.161e-7), ((30, 30, 30), 4, 1.566e-7), ((5, 200, 12), 2, 1.347e-7)]
+                ((100, 100, 100), 2, 2.161e-7), ((30, 30, 30), 4, 1.566e-7), ((5, 200, 12), 2, 1.347e-7),
+                ((34, 34, 34), 4, 2.087e-7), ((51, 51, 51), 4, 2.126e-7), ((68, 68, 68), 4, 2.094e-7),
+                ((85, 85, 85), 4, 2.146e-7)]
 
 
 @pytest.mark.parametrize("shape,seeds,stages", STAGES_ERROR)
