@@ -524,6 +524,7 @@ awk_status awk_atlas_create(awk_atlas_t *out, int nx, int ny, int nz, float spx,
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&L.st, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&L.join, hipEventDisableTiming);
   }
+  if (e == hipSuccess) e = creation_done();
   if (e != hipSuccess) {
     st = hip_check(e, "awk_atlas_create: allocation");
     atlas_free(a);

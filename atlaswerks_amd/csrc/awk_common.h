@@ -87,6 +87,11 @@ inline hipError_t load_scalar_sync(T *host, const T *dev, hipStream_t s) {
   return e;
 }
 
+// Waits for what a creation (or a call that hands a handle back cleared) put on the null stream (hipMemset returns before it has run):
+// the caller's streams need not wait for that stream, and a step size cleared after the
+// first iteration had set it stayed zero.
+inline hipError_t creation_done() { return hipStreamSynchronize(nullptr); }
+
 // Device memory (awk_mem.hip): plain (device_malloc, released by hipFree), kept between
 // handles (dev_alloc, released by dev_free, which waits for the device and takes null
 // pointers), and stream-ordered scratch of one call.

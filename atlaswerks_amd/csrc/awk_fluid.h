@@ -120,6 +120,8 @@ struct Batch {
   int scalar = 0;        // step, energy, prev, have_prev: one per subject (stride 1)
 };
 
+constexpr size_t kScalarBytes = 64;
+
 struct FluidKernel {
   int nx = 0, ny = 0, nz = 0;
   int nxh = 0, nxh_pad = 0;
@@ -140,6 +142,8 @@ struct FluidKernel {
   // device buffers
   float2 *spec = nullptr;  // 3 planes of nz*ny*nxh_pad complex
   float *lut = nullptr;    // cwx[nxh] swx[nxh] cwy[ny] swy[ny] cwz[nz] swz[nz]
+  void *scalars = nullptr; // kScalarBytes behind the tables for an iterator's device scalars,
+                           // cleared by the tables' upload, which is done when it returns
   float *eig = nullptr;    // 6 floats per frequency: symmetric L^p (eigen path)
   int eig_dir = 0;         // which power eig holds: +1 (L^lpow) or -1 (L^-lpow), 0 none
   size_t spec_plane() const { return (size_t)nz * ny * nxh_pad; }

@@ -476,7 +476,8 @@ awk_status fk_init(FluidKernel &k, int nx, int ny, int nz, const float sp[3]) {
   }
   const size_t ntw = tw.size();
   const size_t nlut = 2 * (size_t)k.nxh + 2 * (size_t)ny + 2 * (size_t)nz;
-  std::vector<float> lut(nlut);
+  const size_t scalars = (nlut + 3) / 4 * 4;
+  std::vector<float> lut(scalars + kScalarBytes / sizeof(float), 0.f);
   {
     // DiffOper.cxx:602-625: cosW = (2cos(2 pi k/n) - 2)/sp^2, sinW = sin(2 pi k/n)/sp
     float *p = lut.data();
@@ -507,8 +508,9 @@ awk_status fk_init(FluidKernel &k, int nx, int ny, int nz, const float sp[3]) {
     }
   for (int i = 0; i < 3; ++i)
     if (k.ax[i].dense.tiles) k.ax[i].dense.tab = twd + doff[i];
-  AWK_HIP(dev_alloc(&k.lut, nlut * sizeof(float)));
-  AWK_HIP(hipMemcpy(k.lut, lut.data(), nlut * sizeof(float), hipMemcpyHostToDevice));
+  AWK_HIP(dev_alloc(&k.lut, lut.size() * sizeof(float)));
+  AWK_HIP(hipMemcpy(k.lut, lut.data(), lut.size() * sizeof(float), hipMemcpyHostToDevice));
+  k.scalars = k.lut + scalars;
   k.scratch_bytes = spec_bytes + ntw * sizeof(float2) + nlut * sizeof(float);
   return AWK_OK;
 }
@@ -519,6 +521,7 @@ void fk_release(FluidKernel &k) {
   k.spec = nullptr;
   k.ax[0].tw = k.ax[1].tw = k.ax[2].tw = nullptr;
   k.lut = nullptr;
+  k.scalars = nullptr;
   k.eig = nullptr;
 }
 

@@ -55,6 +55,13 @@ awk_status launch_step_from_max(const float *maxpart, int n, float max_pert, flo
 
 }  // namespace awk
 
+struct GreedyScalars {  // the iterator's device scalars
+  double prev;
+  float step;
+  int have_prev;
+  unsigned flags;
+};
+
 struct awk_greedy {
   awk::FluidKernel k;
   int nx = 0, ny = 0, nz = 0;
@@ -97,8 +104,8 @@ static void greedy_free(awk_greedy *g) {
   g->ev.clear();
   g->ev_mask.clear();
   fk_release(g->k);
-  void *const blocks[] = {g->idef, g->v, g->hbuf, g->partials, g->maxpart, g->step, g->prev, g->have_prev, g->flags};
-  dev_free(blocks, 9);
+  void *const blocks[] = {g->idef, g->v, g->hbuf, g->partials, g->maxpart};
+  dev_free(blocks, 5);
 }
 
 extern "C" {
@@ -136,14 +143,14 @@ awk_status awk_greedy_create(awk_greedy_t *out, int nx, int ny, int nz, float sp
   if (e == hipSuccess) e = dev_alloc(&g->hbuf, 3 * N * sizeof(float));
   if (e == hipSuccess) e = dev_alloc(&g->partials, (size_t)g->nblk * sizeof(double));
   if (e == hipSuccess) e = dev_alloc(&g->maxpart, (size_t)g->nblk * sizeof(float));
-  if (e == hipSuccess) e = dev_alloc(&g->step, sizeof(float));
-  if (e == hipSuccess) e = dev_alloc(&g->prev, sizeof(double));
-  if (e == hipSuccess) e = dev_alloc(&g->have_prev, sizeof(int));
-  if (e == hipSuccess) e = dev_alloc(&g->flags, sizeof(unsigned));
-  if (e == hipSuccess) e = hipMemset(g->flags, 0, sizeof(unsigned));
-  if (e == hipSuccess) e = hipMemset(g->step, 0, sizeof(float));
-  if (e == hipSuccess) e = hipMemset(g->prev, 0, sizeof(double));
-  if (e == hipSuccess) e = hipMemset(g->have_prev, 0, sizeof(int));
+  // cleared before any stream comes here (a memset would not have run yet: with the step
+  // cleared after the first iteration had set it, a level ended where it began)
+  static_assert(sizeof(GreedyScalars) <= kScalarBytes, "the operator's scalars");
+  GreedyScalars *sc = static_cast<GreedyScalars *>(g->k.scalars);
+  g->step = &sc->step;
+  g->prev = &sc->prev;
+  g->have_prev = &sc->have_prev;
+  g->flags = &sc->flags;
   if (e != hipSuccess) {
     st = hip_check(e, "awk_greedy_create: allocation");
     greedy_free(g);

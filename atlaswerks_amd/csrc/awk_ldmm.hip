@@ -371,6 +371,7 @@ awk_status awk::ldmm_init(awk_ldmm *l, int nx, int ny, int nz, const float sp[3]
   if (e == hipSuccess) e = hipMemset(l->step, 0, sizeof(float));
   if (e == hipSuccess) e = dev_alloc(&l->flags, sizeof(unsigned));
   if (e == hipSuccess) e = hipMemset(l->flags, 0, sizeof(unsigned));
+  if (e == hipSuccess) e = creation_done();
   return e == hipSuccess ? AWK_OK : hip_check(e, "LDMM iterator allocation");
 }
 

@@ -227,6 +227,7 @@ awk_status awk_ldmm_atlas_create(awk_ldmm_atlas_t *out, int nx, int ny, int nz, 
     if (e == hipSuccess) e = hipMemcpy(a->jt0, p0.data(), S * sizeof(float *), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(a->jd0, p1.data(), S * sizeof(float *), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemset(a->esub, 0, 3 * (size_t)S * sizeof(double));
+    if (e == hipSuccess) e = creation_done();
     if (e != hipSuccess) st = hip_check(e, "awk_ldmm_atlas_create: allocation");
   }
   if (st) {

@@ -779,6 +779,7 @@ awk_status awk_unet_trainer_gradients(awk_unet_trainer_t t, const float *templ, 
     if (e == hipSuccess) e = hipMemcpy(grad_host, t->g, t->nw * sizeof(float), hipMemcpyDeviceToHost);
     if (e == hipSuccess) e = hipMemcpy(loss_host, ld, sizeof(double), hipMemcpyDeviceToHost);
     if (e == hipSuccess) e = hipMemset(t->g, 0, t->nw * sizeof(float));
+    if (e == hipSuccess) e = creation_done();
     if (e != hipSuccess) st = hip_check(e, "awk_unet_trainer_gradients");
   }
   (void)hipFree(ld);

@@ -167,13 +167,17 @@ hipError_t hipMemPoolTrimTo(hipMemPool_t pool, size_t) {  // (to zero: all that 
 }
 hipError_t hipMemcpy(void *dst, const void *, size_t n, hipMemcpyKind k) {
   if (k == hipMemcpyDeviceToHost) std::memset(dst, 0, n);
+  note("sync");
   return g_capturing ? ret(hipErrorStreamCaptureUnsupported) : hipSuccess;
 }
 hipError_t hipMemcpyAsync(void *dst, const void *, size_t n, hipMemcpyKind k, hipStream_t) {
   if (k == hipMemcpyDeviceToHost) std::memset(dst, 0, n);
   return hipSuccess;
 }
-hipError_t hipMemset(void *, int, size_t) { return g_capturing ? ret(hipErrorStreamCaptureUnsupported) : hipSuccess; }
+hipError_t hipMemset(void *, int, size_t) {  // returns before it is done, unlike hipMemcpy
+  note("memset");
+  return g_capturing ? ret(hipErrorStreamCaptureUnsupported) : hipSuccess;
+}
 hipError_t hipMemsetAsync(void *, int, size_t, hipStream_t) { return hipSuccess; }
 hipError_t hipGetSymbolAddress(void **p, const void *) {
   *p = reinterpret_cast<void *>(uintptr_t{0x10000});
@@ -184,7 +188,10 @@ hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) {
   return hipSuccess;
 }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t s) {
+  if (!s) note("sync");
+  return hipSuccess;
+}
 hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *c) {
   *c = g_capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
   return hipSuccess;

@@ -148,3 +148,20 @@ print(n, len(bad))
 """)
     n, bad = map(int, out.split())
     assert n > 50 and bad == 0, (n, bad)
+
+
+_MAKERS = dict({k: v for k, v in _TAKERS.items() if k not in ("splat", "gaussian_filter")},
+               fluid="assert lib.awk_fluid_kernel_create(ctypes.byref(h), 24, 24, 24, 1.0, 1.0, 1.0, .02, .01, .01, 1.0, 0) == 0",
+               ldmm="assert lib.awk_ldmm_create(ctypes.byref(h), 16, 16, 16, 1.0, 1.0, 1.0, .01, .01, .001, 2, 1.0, .1) == 0",
+               gradients=_TAKERS["unet_trainer"] + "\nu = (P * 3)(1 << 16, 2 << 16, 3 << 16); l = ctypes.c_double()\n"
+                         "assert lib.awk_unet_trainer_gradients(t, p, q, u, w, ctypes.byref(l)) == 0")
+
+
+@pytest.mark.parametrize("maker", sorted(_MAKERS))
+def test_handles_are_ready_for_any_stream(fake, maker):
+    """A handle is made on the null stream and used on the caller's, which need not wait for
+    it: what the creation clears has been waited for when it returns."""
+    fake_hip.run(fake, "h, p, q = P(), P(0x4000), P(0x8000)\n" + _MAKERS[maker] + """
+kinds = [r[0] for r in log() if r[0] in ("memset", "sync")]
+assert "memset" not in kinds or kinds[-1] == "sync", kinds[-6:]
+""")
