@@ -449,6 +449,95 @@ k_base_runs(const unsigned *__restrict__ keys, const unsigned *__restrict__ ids,
   pos[e] = make_float4(1.f - (p.x - xi), 1.f - (p.y - yi), 1.f - (p.z - zi), p.w);
 }
 
+// A voxel's contribution, as corner c (of half: one plane below), to a cell.
+__device__ __forceinline__ float corner_weight(float4 p, int c, int half) {
+#pragma clang fp contract(off)
+  const float wx = (c & 1) ? 1.f - p.x : p.x, wy = (c >> 1) ? 1.f - p.y : p.y, wz = half ? 1.f - p.z : p.z;
+  return p.w * wx * wy * wz;
+}
+
+// A cell with a pile of voxels, by a wave: the next 64 voxels of each of the four runs in
+// LDS, each lane placing its four (up to the first window's end) by their ranks among
+// the other windows, and the contributions added one by one in that order.  Bound by the
+// windows' chain of loads, search and sum, about 30 to 110 cycles a contribution where a
+// lane that merges alone waits 450.  Fields contracted to a tenth, 128^3: 3458 us without,
+// 1123 with, 2353 through the pairs; to a fiftieth 259, 34 and 118 ms.  Where piles of
+// hundreds of voxels fill whole rows neither is as fast as the pairs (1000 x 40 x 40 to a
+// tenth: 2.6 against 1.8 ms); up to a contraction to a fifth this route is the faster.
+constexpr unsigned kPile = 128;     // voxels from which a cell is a pile
+constexpr unsigned kPileRate = 16;  // of a wave's voxels in the time of one of a lane's
+constexpr unsigned kPileStart = 10; // a pile's start in that unit
+constexpr int kPileFloats = 256 + 16 + 256;
+__device__ __forceinline__ float pile_sum(float acc, uint2 (&q)[4], const unsigned *__restrict__ ids,
+                                          const float4 *__restrict__ pos, int half, int lane, float *mine) {
+#pragma clang fp contract(off)
+  constexpr unsigned kNone = 0xffffffffu;
+  unsigned *win = reinterpret_cast<unsigned *>(mine + 272);
+  while (q[0].x < q[0].y || q[1].x < q[1].y || q[2].x < q[2].y || q[3].x < q[3].y) {
+    unsigned id[4], last = kNone;
+    float4 p[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const unsigned i = q[c].x + lane;
+      const bool in = i < q[c].y;
+      id[c] = in ? ids[i] : kNone;
+      p[c] = in ? pos[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      win[64 * c + lane] = id[c];
+      last = min(last, (unsigned)__builtin_amdgcn_readlane(id[c], 63));
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    // voxels of window k before this lane's of window c: at most 63, as the window's last
+    // is not before any that is taken
+    int lower[4][4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) lower[c][k] = 0;
+#pragma unroll
+    for (int step = 32; step > 0; step >>= 1) {
+      unsigned at[4][4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (k != c) at[c][k] = win[64 * k + lower[c][k] + step - 1];
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (k != c) lower[c][k] += at[c][k] < id[c] ? step : 0;
+    }
+    int n = 0;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const bool take = id[c] != kNone && id[c] <= last;
+      if (take) mine[lane + lower[c][0] + lower[c][1] + lower[c][2] + lower[c][3]] = corner_weight(p[c], c, half);
+      const int taken = __popcll(__ballot(take));
+      n += taken;
+      q[c].x += taken;
+    }
+    if (lane < 16) mine[n + lane] = 0.f;  // (the sum is never -0: adding 0 leaves it)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    for (int j = 0; j < n; j += 16) {
+      float4 v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = *reinterpret_cast<const float4 *>(mine + j + 4 * k);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        acc += v[k].x;
+        acc += v[k].y;
+        acc += v[k].z;
+        acc += v[k].w;
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
+  return acc;
+}
+
 // One block per 128 consecutive cells (of one row, or of several short ones).  The runs
 // of their base cells are four stretches of the sorted voxels that ascend with the cell
 // (its own base row and the three before it in y and z), staged in LDS with coalesced
@@ -460,6 +549,7 @@ k_base_sum(float *__restrict__ dst, const unsigned *__restrict__ ids, const floa
            const uint2 *__restrict__ ranges, int w, int h, int l) {
 #pragma clang fp contract(off)  // each contribution is rounded before it is added, as a stored pair is
   constexpr unsigned kNone = 0xffffffffu;
+  static_assert(kSumBlock / 64 * kPileFloats * sizeof(float) <= kSumCap * sizeof(float4), "piles use the stage");
   __shared__ unsigned lo[4], hi[4], sid[kSumCap];
   __shared__ float4 spos[kSumCap];
   const int N = w * h * l, i0 = (int)xcd_block() * kSumBlock, lane = threadIdx.x & 63;
@@ -527,7 +617,6 @@ k_base_sum(float *__restrict__ dst, const unsigned *__restrict__ ids, const floa
       }
     __syncthreads();
   }
-  if (!live) return;
   auto merge = [&](const unsigned *id, const float4 *at, bool moved) {
     float acc = 0.f;
 #pragma unroll
@@ -564,13 +653,47 @@ k_base_sum(float *__restrict__ dst, const unsigned *__restrict__ ids, const floa
           q[k].x = c == k ? i : q[k].x;
           next[k] = c == k ? after : next[k];
         }
-        const float wx = (c & 1) ? 1.f - p.x : p.x, wy = (c >> 1) ? 1.f - p.y : p.y, wz = half ? 1.f - p.z : p.z;
-        acc += p.w * wx * wy * wz;
+        acc += corner_weight(p, c, half);
       }
     }
     return acc;
   };
-  dst[i0 + threadIdx.x] = staged ? merge(sid, spos, true) : merge(ids, pos, false);
+  if (staged) {
+    if (live) dst[i0 + threadIdx.x] = merge(sid, spos, true);
+    return;
+  }
+  // Cells on which many voxels pile up, one after the other by the whole wave where that
+  // is less than the longest takes its lane, which waits for memory at each voxel
+  unsigned voxels = 0;
+#pragma unroll
+  for (int c = 0; c < 8; ++c) voxels += run[c].y - run[c].x;
+  unsigned long long piles = __ballot(voxels >= kPile);
+  unsigned most = voxels >= kPile ? voxels : 0u, all = most;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    most = max(most, (unsigned)__shfl_xor((int)most, off, 64));
+    all += (unsigned)__shfl_xor((int)all, off, 64);
+  }
+  if (all / kPileRate + kPileStart * __popcll(piles) > most) piles = 0ull;
+  float acc = 0.f;
+  if (!(piles >> lane & 1)) acc = merge(ids, pos, false);
+  float *mine = reinterpret_cast<float *>(spos) + (threadIdx.x >> 6) * kPileFloats;
+  for (; piles; piles &= piles - 1) {
+    const int who = __builtin_ctzll(piles);
+    float sum = 0.f;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      uint2 q[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        q[c].x = __builtin_amdgcn_readlane(run[4 * half + c].x, who);
+        q[c].y = __builtin_amdgcn_readlane(run[4 * half + c].y, who);
+      }
+      sum = pile_sum(sum, q, ids, pos, half, lane, mine);
+    }
+    acc = lane == who ? sum : acc;
+  }
+  if (live) dst[i0 + threadIdx.x] = acc;
 }
 
 // Scratch of a sort of M pairs: two key / value buffers, histogram, chunk sums, each at

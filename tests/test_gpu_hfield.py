@@ -279,3 +279,27 @@ def test_splat_sorted_row_lengths_bit_exact(shape, disp):
     hfield.splat_sorted(a, S, V, vals=vals)
     hfield.splat_sorted(b, S, V)
     np.testing.assert_array_equal(a.cpu().numpy(), b.cpu().numpy())
+
+
+# contraction per axis (x, y, z) towards the middle: cells of many voxels, few of a wave's
+# (summed by the whole wave, their runs interleaved) or most of them (by their lanes)
+@pytest.mark.parametrize("shape,by", [((40, 40, 40), (0.9, 0.9, 0.9)), ((30, 50, 70), (0.97, 0.97, 0.97)),
+                                      ((60, 60, 70), (0.0, 0.95, 0.95)), ((20, 30, 300), (0.9, 0.98, 0.9)),
+                                      ((33, 35, 37), (1.0, 1.0, 1.0))])
+def test_splat_sorted_piles_bit_exact(shape, by):
+    """The base-cell sums where voxels pile up against the sums over the sorted pairs, bit
+    for bit."""
+    import torch
+    from atlaswerks_amd import hfield
+    nz, ny, nx = shape
+    print("splat_sorted piles", shape, by, flush=True)
+    rng = np.random.default_rng(nx)
+    src = rng.standard_normal(shape).astype(np.float32)
+    mid = np.array([nx, ny, nz], np.float32)[:, None, None, None] / 2
+    v = rng.uniform(-0.3, 0.3, (3,) + shape) - np.array(by)[:, None, None, None] * (synth.identity(shape) - mid)
+    S, V = torch.from_numpy(src).cuda(), torch.from_numpy(np.ascontiguousarray(v.astype(np.float32))).cuda()
+    vals = torch.empty(8 * src.size, dtype=torch.float32, device="cuda")
+    a, b = torch.full_like(S, 7.0), torch.full_like(S, -3.0)
+    hfield.splat_sorted(a, S, V, vals=vals)
+    hfield.splat_sorted(b, S, V)
+    np.testing.assert_array_equal(a.cpu().numpy(), b.cpu().numpy())
