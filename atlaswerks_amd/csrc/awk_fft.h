@@ -1,4 +1,6 @@
-// awk_fft.h -- LDS-staged mixed-radix FFT engine for gfx950 (device code).
+// awk_fft.h -- LDS-staged mixed-radix FFT engine for gfx950 (device code).  Its register
+// butterflies serve every plan; its stages run the axes that have neither a kernel of
+// their own, nor two radices (awk_radix.h), nor a dense product (awk_dense.h).
 //
 // A batch of NL complex lines of length n lives in LDS in the interleaved layout
 // buf[i * LS + line] (LS >= NL) (element i of every line adjacent).  Stockham autosort

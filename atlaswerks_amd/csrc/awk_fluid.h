@@ -15,9 +15,9 @@ struct AxisPlan {
   std::vector<int> rad;
   Axis dev() const;
   float2 *tw = nullptr;  // device
-  // Bluestein's method (axes with a prime factor above 64): m = the power-of-two
-  // convolution length (0: not used), its radices, and device tables inside the
-  // operator's twiddle allocation
+  // Bluestein's method (LDS stages of an axis with a prime factor above 64, so past the
+  // dense lengths): m = the power-of-two convolution length (0: not used), its radices,
+  // and device tables inside the operator's twiddle allocation
   int m = 0;
   std::vector<int> mrad;
   const float2 *chirp = nullptr, *bhat = nullptr, *mtw = nullptr;

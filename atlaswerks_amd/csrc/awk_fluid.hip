@@ -330,10 +330,12 @@ constexpr size_t kPassLdsMax = 160 * 1024 - 1024;
 
 // Whether an axis is transformed as a dense product (awk_dense.h): a length with a
 // prime factor above 13, whose LDS stages would be a direct DFT of that prime or a
-// chirp-z transform.  L^-1 at 181 x 217 x 181 4347 -> 576 us, 251 x 241 x 239 7189 ->
-// 1085, 248 x 186 x 155 2611 -> 546, 62^3 184 -> 47, 32 x 31 x 36 63 -> 25, with a
-// smaller error against 64 bits each time.  Lengths of small primes are faster, and
-// round half as often, as radices: at 200^3 382 us (dense 664).
+// chirp-z transform.  L^-1 at 181 x 217 x 181 4347 -> 548 us, 251 x 241 x 239 7189 ->
+// 1085, 248 x 186 x 155 2611 -> 546, 62^3 184 -> 47, 32 x 31 x 36 63 -> 25.  Over 30 lengths
+// 17 ... 510 on each axis (the others 64 and 128): 1.3 ... 5 times as fast, small primes
+// times 17 included (408 along x / y / z 500 / 543 / 528 -> 215 / 250 / 328 us, 510 623 /
+// 646 / 644 -> 251 / 300 / 389).  Lengths of small primes are faster as radices: at 200^3
+// 382 us (dense 664).
 static bool use_dense(int n, const std::vector<int> &rad) {
   if (n < kDenseMin || n > kDenseMax) return false;
   for (int r : rad)
@@ -344,8 +346,10 @@ static bool use_dense(int n, const std::vector<int> &rad) {
 // Whether an axis is transformed by two radices in registers (awk_radix.h): every
 // length that has such a plan, up to 1024 (along z up to the 424 whose three
 // components fit a block's LDS).  L^-1 against the LDS stages: 160 x 192 x 144 312 ->
-// 171 us, 96^3 125 -> 62, 36^3 43 -> 27, 112^3 279 -> 78, 182^3 2199 -> 222, 240^3 931 ->
-// 527, 200^3 553 -> 382, 300 x 128 x 128 317 -> 173.
+// 160 us, 96^3 125 -> 59, 36^3 43 -> 26, 112^3 279 -> 78, 182^3 2199 -> 222, 240^3 931 ->
+// 490, 200^3 553 -> 374, 300 x 128 x 128 317 -> 172.  Over 40 lengths 2 ... 1024 on each
+// axis (the others 64 and 128): 1.02 ... 6.3 times as fast (1024 along x / y 322 / 323 ->
+// 292 / 264 us), 625 along x alone 3 % slower.
 static bool use_radix(int axis, int n) {
   int ra, rb;
   return n > 1 && radix_plan(n, ra, rb) && (axis < 2 || (size_t)n * 3 * 16 * sizeof(float2) <= kPassLdsMax);
@@ -571,9 +575,9 @@ awk_status fk_xfwd(FluidKernel &k, const XFwdArgs &a_in, hipStream_t s, int *nbl
                      k.nx, k.ny, k.nz, k.nxh, k.nxh_pad, k.rt, k.spec, k.spec_plane(), bt)
   // block size = row length selects column mode (128^3 LDMM: 17.2 -> 16.3 us
   // against the generic 256-thread form; the spectrum is the same bit for bit)
-  if (k.nx == 256 && k.rt == 8) AWK_XF(256, 8, 256);
-  else if (k.nx == 128 && k.rt == 8) AWK_XF(128, 8, 128);
-  else if (k.nx == 64 && k.rt == 8) AWK_XF(64, 8, 256);
+  if (k.nx == 256) AWK_XF(256, 8, 256);
+  else if (k.nx == 128) AWK_XF(128, 8, 128);
+  else if (k.nx == 64) AWK_XF(64, 8, 256);
   else any_xfwd(k, a, grid, s, bt);
 #undef AWK_XF
   AWK_LAUNCH_CHECK("k_xfwd");
@@ -682,7 +686,7 @@ awk_status fk_xinv(FluidKernel &k, const XInvArgs &a_in, hipStream_t s, int *nbl
   // through L2, with 4 blocks per CU; 0.30 ms with 512 threads of 4 points each,
   // whose FFT rounds differently), so by default rows up to 128 only.
   const int sk = tuning().xinv_stage;
-  const bool stg = a.mode == XSTORE_COMPOSE && (sk == 1 || (sk == 2 && k.nx <= 128)) && k.rt == 8 &&
+  const bool stg = a.mode == XSTORE_COMPOSE && (sk == 1 || (sk == 2 && k.nx <= 128)) &&
                    k.ny % 8 == 0 && (k.nx == 256 || k.nx == 128 || k.nx == 64);
   if (stg) {
     lds = std::max(lds, (size_t)3 * (k.rt + 2) * k.nx * sizeof(float));
@@ -695,7 +699,7 @@ awk_status fk_xinv(FluidKernel &k, const XInvArgs &a_in, hipStream_t s, int *nbl
     } else if (ap) AWK_XIS(64, 256, true);
     else AWK_XIS(64, 256, false);
   } else if (ap) {
-    if (k.nx == 256 && k.rt == 8) {
+    if (k.nx == 256) {
       if (pr) {
         if (xu == 4) AWK_XI3(256, 8, 256, 4, true, true);
         else if (xu == 2) AWK_XI3(256, 8, 256, 2, true, true);
@@ -703,10 +707,10 @@ awk_status fk_xinv(FluidKernel &k, const XInvArgs &a_in, hipStream_t s, int *nbl
       } else if (xu == 4) AWK_XI3(256, 8, 256, 4, false, true);
       else if (xu == 2) AWK_XI3(256, 8, 256, 2, false, true);
       else AWK_XI3(256, 8, 256, 1, false, true);
-    } else if (k.nx == 128 && k.rt == 8) AWK_XI3(128, 8, 256, 2, false, true);
-    else if (k.nx == 64 && k.rt == 8) AWK_XI3(64, 8, 256, 2, false, true);
+    } else if (k.nx == 128) AWK_XI3(128, 8, 256, 2, false, true);
+    else if (k.nx == 64) AWK_XI3(64, 8, 256, 2, false, true);
     else any_xinv(k, a, true, grid, s, bt);
-  } else if (k.nx == 256 && k.rt == 8) {
+  } else if (k.nx == 256) {
     if (pr) {
       if (xu == 4) AWK_XI3(256, 8, 256, 4, true, false);
       else if (xu == 2) AWK_XI3(256, 8, 256, 2, true, false);
@@ -714,8 +718,8 @@ awk_status fk_xinv(FluidKernel &k, const XInvArgs &a_in, hipStream_t s, int *nbl
     } else if (xu == 4) AWK_XI(256, 8, 256, 4);
     else if (xu == 2) AWK_XI(256, 8, 256, 2);
     else AWK_XI(256, 8, 256, 1);
-  } else if (k.nx == 128 && k.rt == 8) AWK_XI(128, 8, 256, 2);
-  else if (k.nx == 64 && k.rt == 8) AWK_XI(64, 8, 256, 2);
+  } else if (k.nx == 128) AWK_XI(128, 8, 256, 2);
+  else if (k.nx == 64) AWK_XI(64, 8, 256, 2);
   else any_xinv(k, a, false, grid, s, bt);
 #undef AWK_XI
 #undef AWK_XI3

@@ -1,7 +1,8 @@
-// awk_fluid_any.hip -- the passes of the FluidKernelFFT operator for any axis length:
-// LDS stages of mixed radices (chirp-z for large primes), or the dense product on the
-// matrix cores (awk_dense.h).  The powers of two from 32 to 256 have their own kernels
-// in awk_fluid.hip.
+// awk_fluid_any.hip -- the passes of the FluidKernelFFT operator for any axis length: two
+// radices in registers (awk_radix.h), the dense product on the matrix cores
+// (awk_dense.h), or LDS stages of mixed radices (chirp-z for large primes).  64, 128 and
+// 256 along x, 32 to 256 along y and 128 and 256 along z have kernels of their own in
+// awk_fluid.hip.
 #include "awk_fluid.h"
 #include "awk_radix.h"
 #include "awk_fluid_solve.h"
@@ -267,8 +268,8 @@ k_ypass_radix(RadixAxis ax, int nz, int nxh, int nxh_pad, float2 *__restrict__ s
 // ones, so stage A and its transpose are the only exchanges along z.  CG: component
 // groups of threads; 3 groups each take a component of every transform and a third of
 // the frequencies (three times the loads in flight and a third of the serial chain,
-// which is what small grids wait for), 1 group takes them in turn (radices up to 32,
-// whose three groups would not fit a block).  Measured against one group: 144 x 192 x 81
+// which is what small grids wait for), 1 group takes them in turn (radices above 16:
+// three groups fit a block up to radix 20, which is untried).  Measured against one group: 144 x 192 x 81
 // frequencies 54.6 -> 43.3 us (2.6 TB/s), 36 x 31 x 17 9.8 -> 6.7 us.
 template <int MAXR, int CG>
 __global__ void __launch_bounds__(16 * MAXR * CG)

@@ -463,7 +463,8 @@ __device__ __forceinline__ float corner_weight(float4 p, int c, int half) {
 // lane that merges alone waits 450.  Fields contracted to a tenth, 128^3: 3458 us without,
 // 1123 with, 2353 through the pairs; to a fiftieth 259, 34 and 118 ms.  Where piles of
 // hundreds of voxels fill whole rows neither is as fast as the pairs (1000 x 40 x 40 to a
-// tenth: 2.6 against 1.8 ms); up to a contraction to a fifth this route is the faster.
+// tenth: 2.6 against 1.8 ms); contracted to three tenths or less this route is the faster
+// on every grid tried, to a fifth about equal (0.90 ... 1.9 times).
 constexpr unsigned kPile = 128;     // voxels from which a cell is a pile
 constexpr unsigned kPileRate = 16;  // of a wave's voxels in the time of one of a lane's
 constexpr unsigned kPileStart = 10; // a pile's start in that unit
