@@ -23,6 +23,7 @@ awk_status fail(awk_status code, const std::string &msg) {
 
 awk_status hip_check(hipError_t e, const char *what) {
   g_err = std::string(what) + ": " + hipGetErrorString(e);
+  (void)hipGetLastError();  // reported here, so not by the next call's launch check as well
   return AWK_ERR_HIP;
 }
 

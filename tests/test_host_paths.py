@@ -165,3 +165,15 @@ def test_handles_are_ready_for_any_stream(fake, maker):
 kinds = [r[0] for r in log() if r[0] in ("memset", "sync")]
 assert "memset" not in kinds or kinds[-1] == "sync", kinds[-6:]
 """)
+
+
+def test_a_reported_error_is_not_reported_again(fake):
+    """A call that fails returns its error; the next one, which does not, returns none."""
+    fake_hip.run(fake, """
+h, p, q = P(), P(0x4000), P(0x8000)
+fake.fake_budget(1 << 20)
+assert lib.awk_splat(p, q, q, q, q, 96, 96, 96, 0, None) != 0
+assert lib.awk_splat(p, q, q, q, q, 16, 16, 16, 0, None) == 0, lib.awk_last_error()
+assert lib.awk_greedy_create(ctypes.byref(h), 80, 80, 80, *([1.0] * 3), .01, .01, .001, .1) != 0
+assert lib.awk_hfield_set_to_identity(p, p, p, 16, 16, 16, None) == 0, lib.awk_last_error()
+""")
