@@ -533,14 +533,8 @@ awk_status fk_prepare_eigen(FluidKernel &k, int dir, hipStream_t s) {
   if (k.eig && k.eig_dir == dir) return AWK_OK;
   const size_t nf = (size_t)k.nxh * k.ny * k.nz;
   if (!k.eig) {
-    // Under capture the table would be recorded and not made, and calls outside the graph
-    // would read it: refused whether or not a kept block spares the allocation (which a
-    // capture does not take).
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    AWK_HIP(hipStreamIsCapturing(s, &cap));
-    if (cap != hipStreamCaptureStatusNone)
-      return fail(AWK_ERR_HIP, "fluid kernel: the first application with an eigen table cannot be captured");
-    AWK_HIP(dev_alloc(&k.eig, nf * 6 * sizeof(float)));
+    // not a kept block, which would spare the allocation that a capture refuses
+    AWK_HIP(device_malloc(&k.eig, nf * 6 * sizeof(float)));
     k.scratch_bytes += nf * 6 * sizeof(float);
   }
   const double p = dir > 0 ? (double)k.lpow : -(double)k.lpow;
@@ -549,7 +543,11 @@ awk_status fk_prepare_eigen(FluidKernel &k, int dir, hipStream_t s) {
                      (double)k.sp[0], (double)k.sp[1], (double)k.sp[2], (double)k.alpha,
                      (double)k.beta, (double)k.gamma, p);
   AWK_LAUNCH_CHECK("k_eigen_table");
-  k.eig_dir = dir;
+  // under a capture (a relaxed one, which allows the allocation) the table is recorded and
+  // not made: the next call makes it
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  AWK_HIP(hipStreamIsCapturing(s, &cap));
+  k.eig_dir = cap == hipStreamCaptureStatusNone ? dir : 0;
   return AWK_OK;
 }
 

@@ -24,7 +24,7 @@ std::map<uintptr_t, Block> g_live;
 std::map<const void *, std::string> g_names;
 std::string g_log, g_fail_name;
 int g_fail_skip = 0;
-bool g_capturing = false;
+bool g_capturing = false, g_strict = false;  // strict: calls that no capture but a relaxed one allows fail
 hipError_t g_last = hipSuccess;
 std::vector<void *> g_call;
 dim3 g_grid, g_block;
@@ -93,7 +93,10 @@ void fake_fail(const char *name, int skip) {
   g_fail_name = name;
   g_fail_skip = skip;
 }
-void fake_capture(int on) { g_capturing = on != 0; }
+void fake_capture(int mode) {  // 0 none, 1 global, 2 relaxed
+  g_capturing = mode != 0;
+  g_strict = mode == 1;
+}
 const char *fake_log() { return g_log.c_str(); }
 void fake_clear() { g_log.clear(); }
 
@@ -142,10 +145,10 @@ hipError_t hipGetLastError() {
 const char *hipGetErrorString(hipError_t) { return "fake"; }
 hipError_t hipDeviceSynchronize() {
   note("sync");
-  return g_capturing ? ret(hipErrorStreamCaptureUnsupported) : hipSuccess;
+  return g_strict ? ret(hipErrorStreamCaptureUnsupported) : hipSuccess;
 }
 hipError_t hipMalloc(void **p, size_t n) {
-  if (g_capturing) return ret(hipErrorStreamCaptureUnsupported);
+  if (g_strict) return ret(hipErrorStreamCaptureUnsupported);
   return take(p, n, nullptr);
 }
 hipError_t hipFree(void *p) { return give(p); }
@@ -168,7 +171,7 @@ hipError_t hipMemPoolTrimTo(hipMemPool_t pool, size_t) {  // (to zero: all that 
 hipError_t hipMemcpy(void *dst, const void *, size_t n, hipMemcpyKind k) {
   if (k == hipMemcpyDeviceToHost) std::memset(dst, 0, n);
   note("sync");
-  return g_capturing ? ret(hipErrorStreamCaptureUnsupported) : hipSuccess;
+  return g_strict ? ret(hipErrorStreamCaptureUnsupported) : hipSuccess;
 }
 hipError_t hipMemcpyAsync(void *dst, const void *, size_t n, hipMemcpyKind k, hipStream_t) {
   if (k == hipMemcpyDeviceToHost) std::memset(dst, 0, n);
@@ -176,7 +179,7 @@ hipError_t hipMemcpyAsync(void *dst, const void *, size_t n, hipMemcpyKind k, hi
 }
 hipError_t hipMemset(void *, int, size_t) {  // returns before it is done, unlike hipMemcpy
   note("memset");
-  return g_capturing ? ret(hipErrorStreamCaptureUnsupported) : hipSuccess;
+  return g_strict ? ret(hipErrorStreamCaptureUnsupported) : hipSuccess;
 }
 hipError_t hipMemsetAsync(void *, int, size_t, hipStream_t) { return hipSuccess; }
 hipError_t hipGetSymbolAddress(void **p, const void *) {
