@@ -144,8 +144,8 @@ hipError_t hipGetLastError() {
 }
 const char *hipGetErrorString(hipError_t) { return "fake"; }
 hipError_t hipDeviceSynchronize() {
-  note("sync");
-  return g_strict ? ret(hipErrorStreamCaptureUnsupported) : hipSuccess;
+  note(g_capturing ? "invalidated" : "sync");  // whatever the capture's mode
+  return g_capturing ? ret(hipErrorStreamCaptureUnsupported) : hipSuccess;
 }
 hipError_t hipMalloc(void **p, size_t n) {
   if (g_strict) return ret(hipErrorStreamCaptureUnsupported);

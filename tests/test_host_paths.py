@@ -182,3 +182,18 @@ assert lib.awk_splat(p, q, q, q, q, 16, 16, 16, 0, None) == 0, lib.awk_last_erro
 assert lib.awk_greedy_create(ctypes.byref(h), 80, 80, 80, *([1.0] * 3), .01, .01, .001, .1) != 0
 assert lib.awk_hfield_set_to_identity(p, p, p, 16, 16, 16, None) == 0, lib.awk_last_error()
 """)
+
+
+_DESTROY = {"fluid": "awk_fluid_kernel_destroy", "greedy": "awk_greedy_destroy", "ldmm": "awk_ldmm_destroy"}
+
+
+@pytest.mark.parametrize("maker", sorted(_DESTROY))
+def test_destroying_leaves_a_relaxed_capture_valid(fake, maker):
+    """Freeing memory is allowed while a relaxed capture runs; waiting for the device is not."""
+    fake_hip.run(fake, "h, p, q = P(), P(0x4000), P(0x8000)\n" + _MAKERS[maker] + """
+fake.fake_clear()
+fake.fake_capture(2)
+assert lib.%s(h) == 0
+fake.fake_capture(0)
+assert not log("invalidated")
+""" % _DESTROY[maker])
