@@ -390,7 +390,7 @@ k_segment_sum(const unsigned *__restrict__ keys, const float *__restrict__ vals,
 // voxels are in that order already (the sort is stable), so a four-way merge adds
 // them one by one in exactly the sequence of the pairs.  The same bits.
 //
-// Bound by the passes over the voxels; 128^3: 479 -> 247 us.
+// Bound by the passes over the voxels; 128^3: 479 -> 239 us.
 
 // The base cell of a voxel at (x, y, z), as k_create_index forms it.
 __device__ __forceinline__ void base_corner(float x, float y, float z, int truncate, int &xi, int &yi, int &zi) {
