@@ -18,6 +18,7 @@
 // library's allocations (device_malloc among them) finds the device full.  Other
 // allocators in the process cannot ask for it: awk_release_memory does.
 #include <mutex>
+#include <new>
 #include <unordered_map>
 #include <vector>
 
@@ -79,6 +80,17 @@ hipError_t or_release(F alloc, int dev) {
   release_kept(c, dev);
   return alloc();
 }
+// A block handed out, with room to put it away later: dev_free allocates nothing, so it
+// throws nothing.  False when host memory has run out.
+bool hold(Cache &c, const Block &b) {
+  try {
+    if (c.idle.capacity() < c.idle.size() + c.live.size() + 1) c.idle.reserve(2 * (c.idle.size() + c.live.size() + 1));
+    c.live[b.p] = b;
+    return true;
+  } catch (const std::bad_alloc &) {
+    return false;
+  }
+}
 size_t block_size(size_t bytes) {
   const size_t unit = bytes < (1u << 20) ? 4096 : 65536;
   return (bytes + unit - 1) / unit * unit;
@@ -105,7 +117,7 @@ hipError_t dev_alloc_bytes(void **p, size_t bytes) {
     for (size_t i = 0; i < c.idle.size(); ++i) {
       const Block b = c.idle[i];
       if (b.dev != dev || b.size != want) continue;
-      c.live[b.p] = b;
+      if (!hold(c, b)) return hipErrorOutOfMemory;
       c.idle.erase(c.idle.begin() + i);
       c.held[dev] -= b.size;
       *p = b.p;
@@ -114,8 +126,10 @@ hipError_t dev_alloc_bytes(void **p, size_t bytes) {
   }
   if (hipError_t e = or_release([&] { return hipMalloc(p, want); }, dev)) return e;
   std::lock_guard<std::mutex> lock(c.mu);
-  c.live[*p] = Block{*p, want, dev};
-  return hipSuccess;
+  if (hold(c, Block{*p, want, dev})) return hipSuccess;
+  (void)hipFree(*p);
+  *p = nullptr;
+  return hipErrorOutOfMemory;
 }
 
 void dev_free(void *const *blocks, int n) {

@@ -5,7 +5,9 @@
 #include <hip/hip_runtime_api.h>
 
 #include <cstdint>
+#include <cstdlib>
 #include <cstring>
+#include <new>
 #include <map>
 #include <string>
 #include <vector>
@@ -17,6 +19,12 @@ struct Pool {
 struct Block {
   size_t size;
   Pool *pool;  // null: hipMalloc, or the runtime's own pool (which keeps nothing)
+};
+bool g_no_host_memory = false;
+struct Own {  // the books themselves do not run out
+  bool was = g_no_host_memory;
+  Own() { g_no_host_memory = false; }
+  ~Own() { g_no_host_memory = was; }
 };
 size_t g_budget = SIZE_MAX, g_used = 0;
 uintptr_t g_next = 0x100000000ull;
@@ -36,7 +44,10 @@ hipError_t ret(hipError_t e) {
   if (e != hipSuccess) g_last = e;
   return e;
 }
-void note(const std::string &s) { g_log += s + "\n"; }
+void note(const std::string &s) {
+  Own own;
+  g_log += s + "\n";
+}
 std::string num(uintptr_t v) { return std::to_string((unsigned long long)v); }
 template <class T>
 std::string num(T *p) {
@@ -44,6 +55,7 @@ std::string num(T *p) {
 }
 
 hipError_t take(void **p, size_t n, Pool *pool) {
+  Own own;
   if (pool) {
     auto it = pool->idle.lower_bound(n);
     if (it != pool->idle.end()) {
@@ -61,6 +73,7 @@ hipError_t take(void **p, size_t n, Pool *pool) {
   return hipSuccess;
 }
 hipError_t give(void *p) {
+  Own own;
   if (!p) return hipSuccess;
   auto it = g_live.find(reinterpret_cast<uintptr_t>(p));
   if (it == g_live.end()) return ret(hipErrorInvalidValue);
@@ -84,9 +97,19 @@ hipError_t launch(const void *f, dim3 g, dim3 b, void **args, hipStream_t s) {
 }
 }  // namespace
 
+// host memory that runs out on demand
+void *operator new(std::size_t n) {
+  void *p = g_no_host_memory ? nullptr : std::malloc(n ? n : 1);
+  if (!p) throw std::bad_alloc();
+  return p;
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, std::size_t) noexcept { std::free(p); }
+
 extern "C" {
 
 // ---- the test's side
+void fake_no_host_memory(int on) { g_no_host_memory = on != 0; }
 void fake_budget(unsigned long long bytes) { g_budget = bytes; }
 unsigned long long fake_used() { return g_used; }
 void fake_fail(const char *name, int skip) {

@@ -197,3 +197,22 @@ assert lib.%s(h) == 0
 fake.fake_capture(0)
 assert not log("invalidated")
 """ % _DESTROY[maker])
+
+
+@pytest.mark.parametrize("maker", sorted(_DESTROY))
+def test_destroying_needs_no_host_memory(fake, maker):
+    """A handle's blocks are put away without allocating: nothing is thrown through the C entry."""
+    fake_hip.run(fake, """
+h, p, q = P(), P(0x4000), P(0x8000)
+handles = []
+for i in range(5):
+    h = P()
+    %s
+    handles.append(h)
+for h in handles:
+    fake.fake_no_host_memory(1)
+    rc = lib.%s(h)
+    fake.fake_no_host_memory(0)
+    assert rc == 0
+assert lib.awk_release_memory() == 0 and fake.fake_used() == 0
+""" % (_MAKERS[maker], _DESTROY[maker]))
