@@ -199,6 +199,7 @@ static void atlas_drop_graphs(awk_atlas *a) {
 
 static void atlas_free(awk_atlas *a) {
   atlas_drop_graphs(a);
+  a->k.other_stream = true;  // the lanes' copies share its tables
   fk_release(a->k);
   for (Subject &s : a->subj) {
     void *b[] = {s.hinv[0], s.hinv[1]};

@@ -105,7 +105,8 @@ template <class T>
 inline hipError_t dev_alloc(T **p, size_t bytes) {
   return dev_alloc_bytes(reinterpret_cast<void **>(p), bytes);
 }
-void dev_free(void *const *blocks, int n);
+// null_only: the blocks were used on the null stream alone, which is then waited for.
+void dev_free(void *const *blocks, int n, bool null_only = false);
 hipError_t scratch_alloc_bytes(void **p, size_t bytes, hipStream_t s);
 template <class T>
 inline hipError_t scratch_alloc(T **p, size_t bytes, hipStream_t s) {

@@ -146,12 +146,19 @@ struct FluidKernel {
                            // cleared by the tables' upload, which is done when it returns
   float *eig = nullptr;    // 6 floats per frequency: symmetric L^p (eigen path)
   int eig_dir = 0;         // which power eig holds: +1 (L^lpow) or -1 (L^-lpow), 0 none
+  // a stream other than the null stream has worked on the operator's or its owner's buffers
+  bool other_stream = false;
+  void used_on(hipStream_t s) { other_stream = other_stream || s; }
   size_t spec_plane() const { return (size_t)nz * ny * nxh_pad; }
   size_t scratch_bytes = 0;
 };
 
 awk_status fk_init(FluidKernel &k, int nx, int ny, int nz, const float sp[3]);
 void fk_release(FluidKernel &k);
+// The operator's blocks, taken from it, for a handle that frees them with its own: one
+// wait for the device instead of two.
+constexpr int kFkBlocks = 4;
+void fk_take_blocks(FluidKernel &k, void *blocks[kFkBlocks]);
 awk_status fk_prepare_eigen(FluidKernel &k, int dir, hipStream_t s);
 // Pass launchers; b (may be null: one subject) batches subjects over blockIdx.y.
 awk_status fk_xfwd(FluidKernel &k, const XFwdArgs &a, hipStream_t s, int *nblocks,

@@ -519,14 +519,22 @@ awk_status fk_init(FluidKernel &k, int nx, int ny, int nz, const float sp[3]) {
   return AWK_OK;
 }
 
-void fk_release(FluidKernel &k) {
-  void *const blocks[] = {k.spec, const_cast<float2 *>(k.ax[0].tw), k.lut, k.eig};
-  dev_free(blocks, 4);
+void fk_take_blocks(FluidKernel &k, void *blocks[kFkBlocks]) {
+  blocks[0] = k.spec;
+  blocks[1] = const_cast<float2 *>(k.ax[0].tw);
+  blocks[2] = k.lut;
+  blocks[3] = k.eig;
   k.spec = nullptr;
   k.ax[0].tw = k.ax[1].tw = k.ax[2].tw = nullptr;
   k.lut = nullptr;
   k.scalars = nullptr;
   k.eig = nullptr;
+}
+
+void fk_release(FluidKernel &k) {
+  void *blocks[kFkBlocks];
+  fk_take_blocks(k, blocks);
+  dev_free(blocks, kFkBlocks, !k.other_stream);
 }
 
 awk_status fk_prepare_eigen(FluidKernel &k, int dir, hipStream_t s) {
@@ -556,6 +564,7 @@ int fk_xblocks(const FluidKernel &k) {
 }
 
 awk_status fk_xfwd(FluidKernel &k, const XFwdArgs &a_in, hipStream_t s, int *nblocks, const Batch *b) {
+  k.used_on(s);
   const Batch bt = b ? *b : Batch();
   const unsigned grid = grid_for((long long)k.ny * k.nz, k.rt);
   XFwdArgs a = a_in;
@@ -584,6 +593,7 @@ awk_status fk_xfwd(FluidKernel &k, const XFwdArgs &a_in, hipStream_t s, int *nbl
 }
 
 awk_status fk_ypass(FluidKernel &k, bool inv, hipStream_t s, const ReduceArgs *red, const Batch *b) {
+  k.used_on(s);
   const Batch bt = b ? *b : Batch();
   ReduceArgs ra;
   std::memset(&ra, 0, sizeof(ra));
@@ -606,6 +616,7 @@ awk_status fk_ypass(FluidKernel &k, bool inv, hipStream_t s, const ReduceArgs *r
 }
 
 awk_status fk_zsolve(FluidKernel &k, bool inverse_op, hipStream_t s, const Batch *b) {
+  k.used_on(s);
   const Batch bt = b ? *b : Batch();
   const bool eigen = (k.flags & AWK_FK_EIGEN) || k.lpow != 1.0f;
   if (eigen) {
@@ -644,6 +655,7 @@ awk_status fk_zsolve(FluidKernel &k, bool inverse_op, hipStream_t s, const Batch
 }
 
 awk_status fk_xinv(FluidKernel &k, const XInvArgs &a_in, hipStream_t s, int *nblocks, const Batch *b) {
+  k.used_on(s);
   const Batch bt = b ? *b : Batch();
   const unsigned grid = grid_for((long long)k.ny * k.nz, k.rt);
   XInvArgs a = a_in;

@@ -103,9 +103,9 @@ static void greedy_free(awk_greedy *g) {
     }
   g->ev.clear();
   g->ev_mask.clear();
-  fk_release(g->k);
-  void *const blocks[] = {g->idef, g->v, g->hbuf, g->partials, g->maxpart};
-  dev_free(blocks, 5);
+  void *blocks[kFkBlocks + 5] = {g->idef, g->v, g->hbuf, g->partials, g->maxpart};
+  fk_take_blocks(g->k, blocks + 5);
+  dev_free(blocks, kFkBlocks + 5, !g->k.other_stream);
 }
 
 extern "C" {
@@ -176,6 +176,7 @@ awk_status awk_greedy_update_step_next(awk_greedy_t g) {
 
 awk_status awk_greedy_set_step(awk_greedy_t g, float step, awk_stream_t stream) {
   if (!g) return fail(AWK_ERR_INVALID, "awk_greedy_set_step: null handle");
+  g->k.used_on(as_stream(stream));
   AWK_HIP(store_scalar_async(g->step, step, as_stream(stream)));
   g->update_step = false;
   return AWK_OK;
@@ -183,12 +184,14 @@ awk_status awk_greedy_set_step(awk_greedy_t g, float step, awk_stream_t stream) 
 
 awk_status awk_greedy_get_step(awk_greedy_t g, float *step, awk_stream_t stream) {
   if (!g || !step) return fail(AWK_ERR_INVALID, "awk_greedy_get_step: null argument");
+  g->k.used_on(as_stream(stream));
   AWK_HIP(load_scalar_sync(step, g->step, as_stream(stream)));
   return AWK_OK;
 }
 
 awk_status awk_greedy_get_flags(awk_greedy_t g, unsigned *flags, int clear, awk_stream_t stream) {
   if (!g) return fail(AWK_ERR_INVALID, "awk_greedy_get_flags: null handle");
+  g->k.used_on(as_stream(stream));
   return read_flags(&g->flags, 1, flags, clear, as_stream(stream), "awk_greedy_get_flags");
 }
 
@@ -210,6 +213,7 @@ static awk_status iterate_one(awk_greedy *g, const float *I0, const float *I1,
                               double *energy_dev, hipStream_t s, bool have_idef, bool fuse_apply,
                               bool *fused) {
   *fused = false;
+  g->k.used_on(s);
   const bool inv = hinv_in && hinv_out;
   const int nx = g->nx, ny = g->ny, nz = g->nz;
   const size_t N = (size_t)nx * ny * nz;

@@ -329,10 +329,12 @@ __global__ void k_orig_image_energy(const double *__restrict__ partials, int n, 
 using namespace awk;
 
 void awk::ldmm_release(awk_ldmm *l) {
-  fk_release(l->k);
-  void *const bufs[] = {l->h,      l->hs,     l->J,  l->diff,      l->acc,   l->partials, l->maxpart,
-                  l->step,   l->energy, l->jt, l->jd, l->sort_work, l->msplat, l->flags};
-  dev_free(bufs, (int)(sizeof(bufs) / sizeof(bufs[0])));
+  void *bufs[] = {l->h,      l->hs,     l->J,  l->diff,      l->acc,    l->partials, l->maxpart,
+                  l->step,   l->energy, l->jt, l->jd,        l->sort_work, l->msplat, l->flags,
+                  nullptr,   nullptr,   nullptr, nullptr};
+  constexpr int n = (int)(sizeof(bufs) / sizeof(bufs[0]));
+  fk_take_blocks(l->k, bufs + n - kFkBlocks);
+  dev_free(bufs, n);
 }
 
 awk_status awk::ldmm_init(awk_ldmm *l, int nx, int ny, int nz, const float sp[3], float alpha,

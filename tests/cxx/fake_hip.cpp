@@ -174,7 +174,10 @@ hipError_t hipMalloc(void **p, size_t n) {
   if (g_strict) return ret(hipErrorStreamCaptureUnsupported);
   return take(p, n, nullptr);
 }
-hipError_t hipFree(void *p) { return give(p); }
+hipError_t hipFree(void *p) {  // waits for the device
+  note("free");
+  return give(p);
+}
 hipError_t hipMallocAsync(void **p, size_t n, hipStream_t) { return take(p, n, nullptr); }
 hipError_t hipFreeAsync(void *p, hipStream_t) { return give(p); }
 hipError_t hipMemPoolCreate(hipMemPool_t *p, const hipMemPoolProps *) {

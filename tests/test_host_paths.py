@@ -216,3 +216,30 @@ for h in handles:
     assert rc == 0
 assert lib.awk_release_memory() == 0 and fake.fake_used() == 0
 """ % (_MAKERS[maker], _DESTROY[maker]))
+
+
+# calls after which work on the handle's buffers may be under way on stream s
+_USES = {
+    ("fluid", "apply"): "assert lib.awk_fluid_kernel_apply(h, p, p, p, 1, s) == 0",
+    ("greedy", "iterate"): "v = (P * 3)(1 << 16, 2 << 16, 3 << 16); assert lib.awk_greedy_iterate(h, p, q, v, v, None, None, None, s) == 0",
+    ("greedy", "set_step"): "assert lib.awk_greedy_set_step(h, 0.5, s) == 0",
+    ("greedy", "get_flags"): "assert lib.awk_greedy_get_flags(h, ctypes.byref(ctypes.c_uint()), 1, s) == 0",
+    ("ldmm", "iterate"): "v = (P * 6)(*[(i + 1) << 16 for i in range(6)]); assert lib.awk_ldmm_iterate(h, p, q, v, None, 0, s) == 0",
+}
+
+
+@pytest.mark.parametrize("maker,use", sorted(_USES))
+def test_blocks_are_put_away_after_their_streams(fake, maker, use):
+    """A block is put away once the work on it is done: behind a wait for the device (the free
+    of a small block) where its handle used a stream of its own, or for the null stream."""
+    fake_hip.run(fake, """
+p, q = P(0x4000), P(0x8000)
+for s, waits in ((P(0x77770), ("free",)), (None, ("free", "sync"))):
+    h = P()
+    %s
+    %s
+    fake.fake_clear()
+    assert lib.%s(h) == 0
+    kinds = [r[0] for r in log()]
+    assert kinds and kinds[0] in waits, kinds
+""" % (_MAKERS[maker], _USES[(maker, use)], _DESTROY[maker]))
